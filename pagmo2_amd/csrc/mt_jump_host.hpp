@@ -8,9 +8,10 @@
 // polynomial of T, T^J = p(T) for p = z^J mod phi, so that
 //   S_J = p(T) S_0,   word k of S_J = XOR over the set coefficients i of p of x[i+k].
 // T never reads the 31 low bits of x[j], so the identity holds on every bit
-// that a later word depends on.  phi has degree 19937; it is obtained here by
-// the Berlekamp-Massey algorithm from 2 x 19937 + 64 output bits of the
-// generator itself and checked to have that degree.
+// that a later word depends on.  phi has degree 19937 and the closed form that
+// Matsumoto and Nishimura give ("Mersenne Twister", ACM TOMACS 8, 1998,
+// appendix), so it costs nothing to set up (Berlekamp-Massey over 2 x 19937
+// output bits took 28 ms of a process's first jump).
 //
 // Polynomials over GF(2) are bit vectors (bit i = coefficient of z^i), 312
 // 64-bit words below degree 19937.  Products use carry-less multiplication
@@ -121,57 +122,6 @@ inline void mul_word_acc(const uint64_t *a, uint64_t n, uint64_t c, uint64_t *ac
     acc[n] ^= carry;
 }
 
-// ---- Berlekamp-Massey over GF(2) ------------------------------------------------
-// Connection polynomial C (c_0 = 1, degree L) of the shortest linear
-// recurrence s[n] = sum_{i=1..L} c_i s[n-i] of the bit sequence s.
-inline void berlekamp_massey(const std::vector<uint8_t> &s, poly &C, uint32_t &L)
-{
-    const uint64_t N = s.size();
-    const uint64_t words = (N + 64u) / 64u + 1u;
-    // rs: s reversed, so that the window s[n-1], s[n-2], ... is ascending
-    poly rs(words, 0u);
-    for (uint64_t k = 0; k < N; ++k) {
-        if (s[N - 1u - k]) rs[k >> 6] |= uint64_t(1) << (k & 63u);
-    }
-    C.assign(words, 0u);
-    poly B(words, 0u), Tm;
-    C[0] = B[0] = 1u;
-    L = 0u;
-    uint64_t m = 1u;
-    for (uint64_t n = 0; n < N; ++n) {
-        // d = s[n] + sum_{i=1..L} c_i s[n-i], with s[n-i] = rs[N-1-n+i]
-        uint64_t acc = 0u;
-        const uint64_t o = N - 1u - n;
-        for (uint64_t w = 0; w * 64u <= L; ++w) {
-            uint64_t c = C[w];
-            if (w == 0u) c &= ~uint64_t(1); // i >= 1
-            const uint64_t top = L - w * 64u; // keep i <= L
-            if (top < 63u) c &= (uint64_t(2) << top) - 1u;
-            if (c) acc ^= c & bits64(rs, o + w * 64u);
-        }
-        const unsigned d = (static_cast<unsigned>(__builtin_popcountll(acc)) & 1u) ^ s[n];
-        if (!d) {
-            ++m;
-            continue;
-        }
-        Tm = C;
-        // C ^= B z^m
-        const uint64_t ws = m >> 6, bs = m & 63u;
-        for (uint64_t w = 0; w + ws < words; ++w) {
-            uint64_t v = B[w] << bs;
-            if (bs && w > 0u) v |= B[w - 1u] >> (64u - bs);
-            C[w + ws] ^= v;
-        }
-        if (2u * L <= n) {
-            L = static_cast<uint32_t>(n + 1u - L);
-            B = Tm;
-            m = 1u;
-        } else {
-            ++m;
-        }
-    }
-}
-
 // ---- arithmetic modulo phi ------------------------------------------------------
 class field
 {
@@ -181,18 +131,26 @@ class field
 
     field()
     {
-        std::mt19937 e(5489u);
-        std::vector<uint8_t> s(2u * kDeg + 64u);
-        for (auto &b : s) b = static_cast<uint8_t>(e() & 1u);
-        poly C;
-        uint32_t L = 0;
-        berlekamp_massey(s, C, L);
-        if (L != kDeg) return;
-        // phi(z) = z^L C(1/z): coefficient i of phi is c_{L-i}
+        // phi = A (B^31 + a_0 B^30 + ... + a_30) + a_31 with A = z^624 + z^397,
+        // B = z^623 + z^396 and a_i bit i of 0x9908b0df, by Horner's rule
+        constexpr uint32_t a = 0x9908b0dfu;
         phi.assign(kWords + 1u, 0u);
-        for (uint32_t i = 0; i <= L; ++i) {
-            if (bit(C, L - i)) phi[i >> 6] |= uint64_t(1) << (i & 63u);
-        }
+        phi[0] = 1u;
+        const auto times = [&](uint32_t hi, uint32_t lo, uint32_t c) {
+            poly r(kWords + 1u, 0u);
+            for (uint32_t s : {hi, lo}) {
+                for (uint64_t w = 0; w <= kWords; ++w) {
+                    const uint64_t at = 64u * w + s, q = at >> 6, b = at & 63u;
+                    if (q <= kWords) r[q] ^= phi[w] << b;
+                    if (b && q < kWords) r[q + 1u] ^= phi[w] >> (64u - b);
+                }
+            }
+            r[0] ^= c;
+            phi = r;
+        };
+        for (uint32_t i = 0; i < 31u; ++i) times(623u, 396u, (a >> i) & 1u);
+        times(624u, 397u, (a >> 31) & 1u);
+        if (!bit(phi, kDeg) || bits64(phi, kDeg + 1u)) return;
         // tab[w - kWords] = z^(64 w) mod phi, w = kWords .. 2 kWords - 1
         poly t = shift_reduce_bits(unit_at(64u * kWords));
         tab.push_back(t);
@@ -361,29 +319,46 @@ inline void prefetch_jump_polys(const std::vector<uint64_t> &Js, unsigned thread
     for (size_t i = 0; i < todo.size(); ++i) c.map.emplace(todo[i], std::move(res[i]));
 }
 
-// z^(k S) mod phi for k = 1 .. count, memoised: one multiplication by z^S
-// each rather than one exponentiation each.
+// z^(k S) mod phi for k = 1 .. count, memoised: one multiplication each
+// rather than one exponentiation each.  With m of them known, the next
+// (up to m) are those times z^(m S), shared among the host's threads.
 inline void prefetch_multiples(uint64_t S, uint64_t count)
 {
     if (count == 0u || S == 0u) return;
-    {
-        // made by an earlier call (the multiples come in order, the last one
-        // is entered with the rest)
-        poly_cache &c = the_cache();
-        std::lock_guard<std::mutex> lk(c.mu);
-        if (count == 1u ? c.map.count(S) != 0u : c.map.count(count * S) != 0u) return;
-    }
-    const field &f = the_field();
-    const poly step = jump_poly(S);
-    poly cur = step;
-    std::vector<std::pair<uint64_t, poly>> res;
-    for (uint64_t k = 2; k <= count; ++k) {
-        cur = f.mul(cur, step);
-        res.emplace_back(k * S, cur);
-    }
     poly_cache &c = the_cache();
+    const auto known = [&](uint64_t k) {
+        std::lock_guard<std::mutex> lk(c.mu);
+        return c.map.count(k * S) != 0u;
+    };
+    // made by an earlier call (the multiples come in order, the last one is
+    // entered with the rest)
+    if (known(count)) return;
+    const field &f = the_field();
+    std::vector<poly> res(count + 1u); // res[k]: z^(k S)
+    res[1] = jump_poly(S);
+    const unsigned threads = std::min(8u, std::max(1u, std::thread::hardware_concurrency()));
+    for (uint64_t m = 1; m < count;) {
+        const uint64_t n = std::min(m, count - m);
+        std::atomic<uint64_t> next{1};
+        const auto work = [&] {
+            for (uint64_t k = next++; k <= n; k = next++) res[m + k] = f.mul(res[k], res[m]);
+        };
+        std::vector<std::thread> pool;
+        try {
+            if (n >= 8u) {
+                pool.reserve(threads);
+                for (unsigned t = 1; t < threads; ++t) pool.emplace_back(work);
+            }
+        } catch (...) {
+            // fewer helper threads: the work queue is shared, so this thread
+            // and those started finish it
+        }
+        work();
+        for (auto &th : pool) th.join();
+        m += n;
+    }
     std::lock_guard<std::mutex> lk(c.mu);
-    for (auto &kv : res) c.map.emplace(kv.first, std::move(kv.second));
+    for (uint64_t k = 2; k <= count; ++k) c.map.emplace(k * S, std::move(res[k]));
 }
 
 } // namespace mtj

@@ -81,20 +81,18 @@ pgh_status launch_mt19937(uint32_t seed, uint64_t skip, uint64_t n, uint32_t *ou
 pgh_status launch_batch_random_dv(const prob &p, uint64_t n, uint32_t seed, double *out, hipStream_t s);
 
 // ---- std::mt19937 jump-ahead (mt_jump.hip) ------------------------------------
-// Device table of the coefficient lists of z^d mod phi for each distance d
-// (layout: mt_dev.hpp, kMtIdxStride); made on first use per device and kept.
-// Synchronous the first time.
-pgh_status jump_table_device(const std::vector<uint64_t> &dists, const void **out);
-// The same table as bytes, for a caller that keeps its own device copy.
+// Bytes of one polynomial of a table (layout: mt_dev.hpp, mt_jump).
+constexpr size_t kJumpPolyBytes = 624u * 4u;
+// Device table of z^(k S) mod phi for k = 1 .. count; made on first use per
+// device, S and count, and kept.  Synchronous the first time; with make false
+// a table that does not exist yet gives a null pointer instead.
+pgh_status jump_table_device(uint64_t S, uint32_t count, bool make, const uint32_t **out);
+// The polynomials of the distances as bytes, for a caller that keeps its own
+// device copy.
 pgh_status jump_table_bytes(const std::vector<uint64_t> &dists, std::vector<uint8_t> &out);
 // Memoises z^(k S) mod phi for k = 1 .. count (host), so that a table of those
 // distances costs one multiplication per entry.
 pgh_status jump_polys_multiples(uint64_t S, uint64_t count);
-// Bytes of the table's header (one 32-bit length per distance, 16-byte padded).
-constexpr size_t jump_table_head(size_t n_dists)
-{
-    return (n_dists * 4u + 15u) / 16u * 16u;
-}
 
 // ---- migration between archipelago islands (migration.hip) ------------------
 struct migr_island {

@@ -11,8 +11,8 @@
 //               each row's best neighbour (pso_gen.cpp:593-622), move the
 //               rows (:302-361), evaluate them with the batch evaluator's
 //               device routines and update the memory (:443-449)
-//   k_rng,      on a second stream, during the current batch: the next
-//   k_rng_gen   batch's words, the island's generator split in segments that
+//   k_rng       on a second stream, during the current batch: the next
+//               batch's words, the island's generator split in segments that
 //               reach their own positions by jump-ahead (mt_dev.hpp,
 //               mt_jump): exactly the draws of the reference's sequential loop
 // plus k_gbest_update for islands of the gbest topology.  Batched mode
@@ -54,13 +54,17 @@ struct island_desc {
     // (kGenBatch, or all of a call's when fewer) is bwords = gps W words, and
     // segment s hands out its words s swords .. (s + 1) swords - 1 (the last
     // segment the rest); seg0 is the first segment's index; j_* index the
-    // archipelago's jump table: z^n0 (the velocity draws), z^(s swords) at
+    // archipelago's jump table: z^n0 (past the velocity draws), z^(s swords) at
     // j_pos + s - 1 (to segment s), z^(bwords - swords) and
     // z^((segs - 1) swords) (from the end of a full segment, and of the last
     // one, to the same segment of the next batch)
     uint64_t bwords, swords;
     uint32_t segs, seg0, gps;
     uint32_t j_n0, j_pos, j_main, j_last;
+    // the velocity draws (n0 words) split in vsegs shares of kVelShare words,
+    // share s reached by z^(s kVelShare) at j_vel + s - 1; 0: one share, made by
+    // segment 0 on its way to the first batch
+    uint32_t vsegs, j_vel;
     // pso_gen's variant (1..6) and topology (1 gbest, 2 lbest, 3 von Neumann),
     // the neighbours per particle (lbest 2 radius, von Neumann 4) and the von
     // Neumann lattice's columns; the random words of a generation (wgen) and
@@ -90,8 +94,12 @@ constexpr uint32_t kBlock = 256;
 // the batch's words are made by many workgroups at once
 constexpr uint32_t kGenBatch = 32;
 constexpr uint64_t kSegMin = uint64_t(1) << 16, kSegMax = uint64_t(1) << 22, kSoloWords = uint64_t(1) << 20;
-// k_rng_gen's workgroup: the generator steps 227 words at a time (mt_run)
-constexpr uint32_t kMtGenBlock = 256;
+// Words per share of the velocity draws: from two shares on, the draws of a
+// large island (4 M words at 4096 x 500, 1.4 ms in one workgroup) are made by
+// many workgroups before the call's first batch.
+constexpr uint64_t kVelShare = uint64_t(1) << 15;
+// seg_desc::s of the workgroup that copies an island's generator (k_rng_vel)
+constexpr uint32_t kSegCopy = 0xffffffffu;
 
 // "a <= b" in the sense of less_than_f(a, b) || equal_to_f(a, b)
 // (custom_comparisons.hpp:54-100): NaN is larger than everything but itself.
@@ -116,28 +124,6 @@ __device__ __forceinline__ uint32_t find_island(const island_desc *__restrict__ 
     return lo;
 }
 
-struct jump_tab {
-    const uint32_t *lens;
-    const uint16_t *lists; // kMtIdxStride values per distance
-};
-
-__device__ __forceinline__ void load_state(const mt_state *__restrict__ src, uint32_t *ring, uint64_t &K, uint64_t &C)
-{
-    for (uint32_t i = threadIdx.x; i < kMtRing; i += blockDim.x) ring[i] = src->ring[i];
-    K = src->K;
-    C = src->C;
-    __syncthreads();
-}
-
-__device__ __forceinline__ void store_state(mt_state *__restrict__ dst, const uint32_t *ring, uint64_t K, uint64_t C)
-{
-    for (uint32_t i = threadIdx.x; i < kMtRing; i += blockDim.x) dst->ring[i] = ring[i];
-    if (threadIdx.x == 0) {
-        dst->K = K;
-        dst->C = C;
-    }
-}
-
 // The island's std::mt19937 draws, by its segments (one workgroup each).
 // Every word of an evolve call has a position in the island's one sequential
 // stream: first the velocity draws (n0 = 2 words per element,
@@ -148,14 +134,16 @@ __device__ __forceinline__ void store_state(mt_state *__restrict__ dst, const ui
 // s swords .. (s + 1) swords - 1 (the last segment the rest) into their place
 // in the word buffer.
 //
-// k_rng phase 0, the start of an evolve call: every segment takes the
-// island's canonical generator (everything handed out so far); segment 0
-// hands out the velocity draws and every segment moves to its share of the
-// first batch, n0 + s swords (jumps z^n0 and z^(s swords)).  k_rng_gen, batch b: each segment hands out its share; the segment
+// k_rng_vel, the start of an evolve call: the velocities, each share of the
+// draws by a workgroup that jumps to it from the island's canonical generator
+// (everything handed out so far), and a copy of that generator for k_rng, whose
+// last segment replaces it.  k_rng, first batch: every segment takes the copy
+// and moves to its share, n0 + s swords (jumps z^n0 and z^(s swords); the one
+// segment of an island whose draws are one share makes the velocities on the
+// way); later batches: each segment with more to hand out jumps from the end
+// of its share of the batch before.  Then it hands out its share; the segment
 // that hands out the island's last word keeps the generator there as the
-// canonical one.  k_rng phase 2, after batch b when another follows: each
-// segment with more to hand out jumps from the end of its share to its share
-// of batch b + 1.  The words are those of one sequential generator, in order.
+// canonical one.  The words are those of one sequential generator, in order.
 __device__ __forceinline__ void seg_span(const island_desc &di, uint32_t s, uint32_t b, uint64_t n0, uint64_t &start,
                                          uint64_t &count, uint64_t &end)
 {
@@ -177,88 +165,131 @@ __device__ __forceinline__ uint64_t velocity_words(const island_desc &di, uint32
     return (di.memory && v_valid) ? 0u : 2ull * di.pop * di.nx;
 }
 
-__global__ __launch_bounds__(kMtJumpBlock) void k_rng(const island_desc *__restrict__ d,
-                                                      const seg_desc *__restrict__ sd, mt_state *__restrict__ st,
-                                                      mt_state *__restrict__ segst, jump_tab jt,
-                                                      uint32_t *__restrict__ words, uint32_t sg0, uint32_t phase,
-                                                      uint32_t b, uint32_t v_valid)
-{
-    __shared__ uint32_t ring[kMtRing];
-    __shared__ uint4 lds_idx[kMtIdxStride / 8u];
-    const seg_desc sg = sd[sg0 + blockIdx.x];
-    const island_desc di = d[sg.island];
-    const auto jump = [&](uint64_t &K, uint64_t &C, uint64_t J, uint32_t j) {
-        mt_jump(ring, K, C, J, jt.lists + static_cast<uint64_t>(j) * kMtIdxStride, jt.lens[j], lds_idx);
-    };
-    const uint64_t n0 = velocity_words(di, v_valid);
-    uint64_t K, C;
-    mt_state *mine = &segst[di.seg0 + sg.s];
-    if (phase == 0u) {
-        load_state(&st[sg.island], ring, K, C);
-        if (sg.s == 0u) {
-            if (n0) {
-                mt_run(ring, K, C, n0, words + di.woff);
-                C += n0;
-            }
-            if (di.gens == 0u) store_state(&st[sg.island], ring, K, C);
-        } else {
-            if (n0) jump(K, C, n0, di.j_n0);
-            jump(K, C, static_cast<uint64_t>(sg.s) * di.swords, di.j_pos + sg.s - 1u);
+// Words handed out become velocities, U(minv, maxv) (pso_gen.cpp:177-200).
+struct velocity_sink {
+    double *V;   // the island's
+    uint64_t m0; // element of the hand-out's first word
+    uint32_t nx;
+    int kind;
+    double max_vel, minv, w;
+    __device__ __forceinline__ void range(uint32_t j, double &lo, double &width) const
+    {
+        double lb, ub;
+        bounds_of(kind, j, lb, ub);
+        const double vwidth = (ub - lb) * max_vel;
+        lo = -1. * vwidth;
+        width = mt_width(lo, vwidth);
+    }
+    __device__ __forceinline__ velocity_sink(double *V_, uint64_t m0_, const island_desc &di)
+        : V(V_), m0(m0_), nx(di.nx), kind(di.kind), max_vel(di.max_vel)
+    {
+        range(0u, minv, w);
+    }
+    __device__ __forceinline__ void operator()(uint64_t at, const uint32_t *__restrict__ words, uint32_t n,
+                                               uint32_t tid, uint32_t nthr) const
+    {
+        const uint64_t m = m0 + at / 2u;
+        // only lennard_jones' bounds depend on the column
+        const bool cols = kind == LENNARD_JONES;
+        const uint32_t c0 = cols ? static_cast<uint32_t>(m % nx) : 0u;
+        for (uint32_t i = tid; i < n / 2u; i += nthr) {
+            const uint2 v = reinterpret_cast<const uint2 *>(words)[i];
+            double a = minv, wi = w;
+            if (cols) range((c0 + i) % nx, a, wi);
+            V[m + i] = mt_uniform(mt_temper(v.x), mt_temper(v.y), a, wi);
         }
-        store_state(mine, ring, K, C);
+    }
+};
+
+__global__ __launch_bounds__(kMtBlock) void k_rng_vel(const island_desc *__restrict__ d,
+                                                      const seg_desc *__restrict__ vsd,
+                                                      const mt_state *__restrict__ st, mt_state *__restrict__ stq,
+                                                      const uint32_t *__restrict__ polys, double *__restrict__ V,
+                                                      uint32_t vs0, uint32_t v_valid)
+{
+    __shared__ __align__(16) uint32_t buf[kMtBuf];
+    const seg_desc sg = vsd[vs0 + blockIdx.x];
+    const island_desc di = d[sg.island];
+    uint32_t pos;
+    if (sg.s == kSegCopy) {
+        mt_load(st[sg.island], buf, pos);
+        mt_store(stq[sg.island], buf, pos);
         return;
     }
-    // phase 2: after batch b, to batch b + 1 (a one-segment generator ends
-    // its share where the next begins)
-    if (di.segs == 1u) return;
-    uint64_t start, count, end;
-    seg_span(di, sg.s, b, n0, start, count, end);
-    if (count == 0u || start + count == end || start + di.bwords >= end) return;
-    load_state(mine, ring, K, C);
-    if (sg.s + 1u < di.segs) {
-        jump(K, C, di.bwords - di.swords, di.j_main);
-    } else {
-        jump(K, C, static_cast<uint64_t>(di.segs - 1u) * di.swords, di.j_last);
-    }
-    store_state(mine, ring, K, C);
+    const uint64_t n0 = velocity_words(di, v_valid), begin = sg.s * kVelShare;
+    if (begin >= n0) return;
+    mt_load(st[sg.island], buf, pos);
+    if (sg.s > 0u) mt_jump(buf, polys + static_cast<uint64_t>(di.j_vel + sg.s - 1u) * kMtN);
+    mt_hand_out(buf, pos, min(kVelShare, n0 - begin),
+                velocity_sink(V + di.xoff, begin / 2u, di));
 }
 
-// Batch b's words of one segment (see k_rng).
+// Batch b's words of one segment (see above) from the generator in buf, by a
+// workgroup of NT threads.
+template <uint32_t NT>
 __device__ __forceinline__ void rng_gen_segment(const island_desc &di, uint32_t s, uint32_t b, uint64_t n0,
                                                 mt_state *__restrict__ st, mt_state *__restrict__ mine,
-                                                uint32_t *__restrict__ batch_words, uint32_t *ring)
+                                                uint32_t *__restrict__ batch_words, uint32_t *__restrict__ buf,
+                                                uint32_t pos)
 {
     uint64_t start, count, end;
     seg_span(di, s, b, n0, start, count, end);
     if (count == 0u) return;
-    uint64_t K, C;
-    load_state(mine, ring, K, C);
-    mt_run(ring, K, C, count, batch_words + static_cast<uint64_t>(s) * di.swords);
-    C += count;
-    store_state(start + count == end ? st : mine, ring, K, C);
+    mt_hand_out<NT>(buf, pos, count, mt_word_sink{batch_words + static_cast<uint64_t>(s) * di.swords});
+    mt_store<NT>(start + count == end ? *st : *mine, buf, pos);
 }
 
-__global__ __launch_bounds__(kMtGenBlock) void k_rng_gen(const island_desc *__restrict__ d,
-                                                         const seg_desc *__restrict__ sd, mt_state *__restrict__ st,
-                                                         mt_state *__restrict__ segst, uint32_t *__restrict__ words,
-                                                         uint32_t sg0, uint32_t b, uint32_t v_valid)
+__global__ __launch_bounds__(kMtBlock) void k_rng(const island_desc *__restrict__ d, const seg_desc *__restrict__ sd,
+                                                  mt_state *__restrict__ st, const mt_state *__restrict__ stq,
+                                                  mt_state *__restrict__ segst, const uint32_t *__restrict__ polys,
+                                                  uint32_t *__restrict__ words, double *__restrict__ V, uint32_t sg0,
+                                                  uint32_t b, uint32_t v_valid)
 {
-    __shared__ uint32_t ring[kMtRing];
+    __shared__ __align__(16) uint32_t buf[kMtBuf];
     const seg_desc sg = sd[sg0 + blockIdx.x];
     const island_desc di = d[sg.island];
-    rng_gen_segment(di, sg.s, b, velocity_words(di, v_valid), &st[sg.island], &segst[di.seg0 + sg.s],
-                    words + di.woff + ((b & 1u) ? di.whalf : 0u), ring);
+    const uint64_t n0 = velocity_words(di, v_valid);
+    mt_state *mine = &segst[di.seg0 + sg.s];
+    // at most two jumps, at these entries of the table
+    constexpr uint32_t kNone = 0xffffffffu;
+    uint32_t j0 = kNone, j1 = kNone, pos;
+    if (b == 0u) {
+        if (di.gens == 0u && sg.s > 0u) return;
+        mt_load(stq[sg.island], buf, pos);
+        if (n0) {
+            if (di.vsegs == 0u && sg.s == 0u) {
+                mt_hand_out(buf, pos, n0, velocity_sink(V + di.xoff, 0u, di));
+            } else {
+                j0 = di.j_n0;
+            }
+        }
+        if (sg.s > 0u) j1 = di.j_pos + sg.s - 1u;
+    } else {
+        uint64_t start, count, end;
+        seg_span(di, sg.s, b, n0, start, count, end);
+        if (count == 0u) return;
+        mt_load(*mine, buf, pos);
+        // (a one-segment generator ends its share where the next begins)
+        if (di.segs > 1u) j0 = sg.s + 1u < di.segs ? di.j_main : di.j_last;
+    }
+    for (uint32_t r = 0; r < 2u; ++r) {
+        const uint32_t j = r ? j1 : j0;
+        if (j != kNone) mt_jump(buf, polys + static_cast<uint64_t>(j) * kMtN);
+    }
+    if (di.gens == 0u) {
+        mt_store(st[sg.island], buf, pos);
+        return;
+    }
+    rng_gen_segment<kMtBlock>(di, sg.s, b, n0, &st[sg.island], mine, words + di.woff + ((b & 1u) ? di.whalf : 0u), buf, pos);
 }
 
-// Start of an evolve call (pso_gen.cpp:183-200): V = U(minv, maxv) per
-// element, and X = lbX = the population.  The population is X/fit before the
+// Start of an evolve call (pso_gen.cpp:183-200): X = lbX = the population.  The population is X/fit before the
 // first call and lbX/lbfit after one (pop.set_xf(i, lbX, lbfit)).
 __global__ __launch_bounds__(kBlock) void k_vinit(const island_desc *__restrict__ d, uint32_t i0, uint32_t i1,
-                                                  uint64_t e0, uint64_t total, const uint32_t *__restrict__ words,
-                                                  double *__restrict__ X, double *__restrict__ V,
+                                                  uint64_t e0, uint64_t total, double *__restrict__ X,
                                                   double *__restrict__ lbX, double *__restrict__ fit,
                                                   double *__restrict__ lbfit, uint32_t *__restrict__ selA,
-                                                  uint32_t v_valid, uint32_t from_lb)
+                                                  uint32_t from_lb)
 {
     const uint64_t t = static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x;
     if (t >= total) return;
@@ -267,14 +298,6 @@ __global__ __launch_bounds__(kBlock) void k_vinit(const island_desc *__restrict_
     const island_desc di = d[k];
     const uint64_t m = e - di.eoff;
     const uint32_t j = static_cast<uint32_t>(m % di.nx);
-    if (!(di.memory && v_valid)) {
-        double lb, ub;
-        bounds_of(di.kind, j, lb, ub);
-        const double vwidth = (ub - lb) * di.max_vel; // pso_gen.cpp:177-181
-        const double minv = -1. * vwidth, maxv = vwidth;
-        const uint32_t *w = words + di.woff + 2u * m;
-        V[di.xoff + m] = mt_uniform(w[0], w[1], minv, maxv);
-    }
     const uint64_t p = m / di.nx;
     if (j == 0u) selA[di.foff + p] = 0u; // every row's memory starts in lbX0 (k_step)
     if (from_lb) {
@@ -1141,7 +1164,7 @@ __global__ __launch_bounds__(kBlock) void k_settle(const island_desc *__restrict
 //
 // With a second workgroup (gridDim.x == 2, an island whose generator is one
 // segment), that workgroup hands out the next batch's words (g1 ..) into
-// words_next, as k_rng's phase 1 would after this launch: the two workgroups
+// words_next, as k_rng would after this launch: the two workgroups
 // share no data, and the next launch reads those words.
 template <bool STAGE>
 __global__ __launch_bounds__(kBlock) void k_gens_one_tile(const island_desc *__restrict__ d,
@@ -1156,10 +1179,12 @@ __global__ __launch_bounds__(kBlock) void k_gens_one_tile(const island_desc *__r
     const island_desc di = d[island];
     const uint64_t elems = static_cast<uint64_t>(di.pop) * di.nx;
     if (blockIdx.x == 1u) {
-        // batch g1 / gps of a one-segment generator (k_rng_gen's work; the
+        // batch g1 / gps of a one-segment generator (k_rng's work; the
         // velocity draws shift the whole call's words alike)
-        __shared__ uint32_t ring[kMtRing];
-        rng_gen_segment(di, 0u, g1 / di.gps, 0u, &st[island], &segst[di.seg0], words_next + di.woff, ring);
+        __shared__ __align__(16) uint32_t buf[kMtBuf];
+        uint32_t pos;
+        mt_load<kBlock>(segst[di.seg0], buf, pos);
+        rng_gen_segment<kBlock>(di, 0u, g1 / di.gps, 0u, &st[island], &segst[di.seg0], words_next + di.woff, buf, pos);
         return;
     }
     const uint32_t end = min(g1, di.gens);
@@ -1249,6 +1274,10 @@ struct pgh_archi {
     // and go up in one copy
     dev_buf arena, trace_buf;
     arena_view desc, tiles, segs, jump_table, states, X, V, lbX, fit, lbfit, words, seg_states;
+    // the velocity draws' shares and generator copies (k_rng_vel), per island
+    // contiguous from vseg_begin[k], and those copies
+    arena_view vsegs, states_q;
+    std::vector<uint32_t> vseg_begin;
     // the gbest islands (their indices, in order) and their best positions
     arena_view gblist, gbest;
     std::vector<uint32_t> h_gb;
@@ -1269,7 +1298,6 @@ struct pgh_archi {
     pgh_archi_mapping map{PGH_ARCHI_STEP_ONE, 0u, 0u, 0u}; // the 64-island workload's fastest form
     uint32_t step_per_cu[4] = {1u, 1u, 1u, 1u}; // k_step workgroups per CU, per class
     uint32_t n_segs = 0;
-    jump_tab jt{nullptr, nullptr};
     hipStream_t own = nullptr;
     hipStream_t side = nullptr; // a batched evolve's random words for the next batch
     hipEvent_t ev_main = nullptr, ev_side = nullptr;
@@ -1497,13 +1525,18 @@ pgh_status launch_range(pgh_archi *a, uint32_t i0, uint32_t i1, bool v_valid, bo
     const uint32_t ng = (i1 < a->h_desc.size() ? a->h_desc[i1].seg0 : a->n_segs) - sg0;
     const auto *sd = static_cast<const seg_desc *>(a->segs.ptr);
     auto *segst = static_cast<mt_state *>(a->seg_states.ptr);
-    const jump_tab jt = a->jt;
+    auto *stq = static_cast<mt_state *>(a->states_q.ptr);
+    const auto *jt = static_cast<const uint32_t *>(a->jump_table.ptr);
     const uint32_t vv = v_valid ? 1u : 0u;
-    k_rng<<<ng, kMtJumpBlock, 0, s>>>(d, sd, st, segst, jt, w, sg0, 0u, 0u, vv);
+    const uint32_t vs0 = a->vseg_begin[i0];
+    k_rng_vel<<<a->vseg_begin[i1] - vs0, kMtBlock, 0, s>>>(d, static_cast<const seg_desc *>(a->vsegs.ptr), st, stq, jt,
+                                                           V, vs0, vv);
     PGH_HIP(hipGetLastError());
+    const auto make_words = [&](uint32_t b, hipStream_t on) {
+        k_rng<<<ng, kMtBlock, 0, on>>>(d, sd, st, stq, segst, jt, w, V, sg0, b, vv);
+    };
     auto *selA = static_cast<uint32_t *>(a->selA.ptr);
-    k_vinit<<<blocks_for(total), kBlock, 0, s>>>(d, i0, i1, e0, total, w, X, V, lbX, fit, lbfit, selA,
-                                                 v_valid ? 1u : 0u, from_lb ? 1u : 0u);
+    k_vinit<<<blocks_for(total), kBlock, 0, s>>>(d, i0, i1, e0, total, X, lbX, fit, lbfit, selA, from_lb ? 1u : 0u);
     PGH_HIP(hipGetLastError());
     // a single island of one tile, evolved by the one-shot entry point: a
     // batch of generations per launch (k_gens_one_tile)
@@ -1541,12 +1574,16 @@ pgh_status launch_range(pgh_archi *a, uint32_t i0, uint32_t i1, bool v_valid, bo
     // stream while the current batch's generations run (each island with more
     // than one batch alternates between the two halves of its word buffer)
     const bool side_rng = !fused && i1 > i0 + 1u;
+    if (gens == 0u) { // the generators still go past the velocity draws
+        make_words(0u, s);
+        PGH_HIP(hipGetLastError());
+    }
     for (uint32_t g = 0; g < gens; ++g) {
         if (g % kGenBatch == 0u) {
             const uint32_t b = g / kGenBatch;
             if (side_rng) {
                 if (b == 0u) {
-                    k_rng_gen<<<ng, kMtGenBlock, 0, s>>>(d, sd, st, segst, w, sg0, 0u, vv);
+                    make_words(0u, s);
                     PGH_HIP(hipGetLastError());
                 } else {
                     PGH_HIP(hipStreamWaitEvent(s, a->ev_side, 0)); // batch b's words
@@ -1556,14 +1593,12 @@ pgh_status launch_range(pgh_archi *a, uint32_t i0, uint32_t i1, bool v_valid, bo
                     // batch b + 1's words
                     PGH_HIP(hipEventRecord(a->ev_main, s));
                     PGH_HIP(hipStreamWaitEvent(a->side, a->ev_main, 0));
-                    k_rng<<<ng, kMtJumpBlock, 0, a->side>>>(d, sd, st, segst, jt, w, sg0, 2u, b, vv);
-                    k_rng_gen<<<ng, kMtGenBlock, 0, a->side>>>(d, sd, st, segst, w, sg0, b + 1u, vv);
+                    make_words(b + 1u, a->side);
                     PGH_HIP(hipGetLastError());
                     PGH_HIP(hipEventRecord(a->ev_side, a->side));
                 }
             } else if (!overlap || g == 0u) {
-                if (b > 0u) k_rng<<<ng, kMtJumpBlock, 0, s>>>(d, sd, st, segst, jt, w, sg0, 2u, b - 1u, vv);
-                k_rng_gen<<<ng, kMtGenBlock, 0, s>>>(d, sd, st, segst, w, sg0, b, vv);
+                make_words(b, s);
                 PGH_HIP(hipGetLastError());
             }
             if (fused) {
@@ -1693,11 +1728,16 @@ pgh_status archi_create(pgh_archi **out, const pgh_island_spec *islands, uint64_
     // islands' batches (a power of two in [kSegMin, kSegMax]), so that the
     // batch's words are made by workgroups spread over the device while the
     // jumps that position the segments (each costs about as much as making
-    // a few hundred thousand words) stay few.  The jumps z^(s seg_words) that
+    // 10^5 words) stay few.  The jumps z^(s seg_words) that
     // move segment s to its first share are the same for every island and
     // come first in the jump table (one multiplication each on the host);
     // other distances are entered once each.
-    uint64_t seg_words = kSegMin, max_segs = 1u;
+    uint64_t seg_words = kSegMin, max_segs = 1u, max_vsegs = 0u;
+    // shares of an island's velocity draws: up to four (44 us in one workgroup,
+    // about a jump) are left to segment 0
+    const auto vel_shares = [](uint64_t n0) {
+        return n0 > 4u * kVelShare ? static_cast<uint32_t>((n0 + kVelShare - 1u) / kVelShare) : 0u;
+    };
     {
         uint64_t total = 0;
         std::vector<uint64_t> bw(n_islands, 0u);
@@ -1710,6 +1750,7 @@ pgh_status archi_create(pgh_archi **out, const pgh_island_spec *islands, uint64_
             uint32_t wpu = 0u;
             bw[k] = gps * words_per_gen(q.variant, K, islands[k].pop, p.nx, wpu);
             total += bw[k];
+            max_vsegs = std::max<uint64_t>(max_vsegs, vel_shares(2u * islands[k].pop * p.nx));
         }
         const uint64_t want = total / (2u * a->n_cus);
         while (seg_words * 2u <= want && seg_words < kSegMax) seg_words *= 2u;
@@ -1722,6 +1763,10 @@ pgh_status archi_create(pgh_archi **out, const pgh_island_spec *islands, uint64_
     }
     for (uint64_t k = 1; k < max_segs; ++k) dists.push_back(k * seg_words);
     PGH_TRY(jump_polys_multiples(seg_words, max_segs - 1u));
+    const uint32_t j_vel = static_cast<uint32_t>(dists.size());
+    for (uint64_t k = 1; k < max_vsegs; ++k) dists.push_back(k * kVelShare);
+    if (max_vsegs > 1u) PGH_TRY(jump_polys_multiples(kVelShare, max_vsegs - 1u));
+    std::vector<seg_desc> vseg_list;
     const auto dist_index = [&dists](uint64_t J) {
         for (size_t i = 0; i < dists.size(); ++i) {
             if (dists[i] == J) return static_cast<uint32_t>(i);
@@ -1851,8 +1896,13 @@ pgh_status archi_create(pgh_archi **out, const pgh_island_spec *islands, uint64_
             di.swords = std::min(di.bwords, seg_words);
             di.segs = static_cast<uint32_t>((di.bwords + di.swords - 1u) / di.swords);
             di.j_n0 = di.j_pos = di.j_main = di.j_last = 0u;
+            di.vsegs = vel_shares(2u * elems);
+            di.j_vel = j_vel;
+            a->vseg_begin.push_back(static_cast<uint32_t>(vseg_list.size()));
+            for (uint32_t v = 0; v < di.vsegs; ++v) vseg_list.push_back(seg_desc{static_cast<uint32_t>(k), v});
+            vseg_list.push_back(seg_desc{static_cast<uint32_t>(k), kSegCopy});
+            if (di.segs > 1u || di.vsegs > 0u) di.j_n0 = dist_index(2u * elems);
             if (di.segs > 1u) {
-                di.j_n0 = dist_index(2u * elems);
                 di.j_pos = 0u; // the shared z^(s seg_words) block
                 di.j_main = dist_index(di.bwords - di.swords);
                 di.j_last = dist_index(static_cast<uint64_t>(di.segs - 1u) * di.swords);
@@ -1866,6 +1916,7 @@ pgh_status archi_create(pgh_archi **out, const pgh_island_spec *islands, uint64_
         a->tile_begin.push_back(static_cast<uint32_t>(a->h_tiles.size()));
         a->h_desc.push_back(di);
     }
+    a->vseg_begin.push_back(static_cast<uint32_t>(vseg_list.size()));
     a->total_elems = eoff;
     a->total_words = woff;
     a->total_trace = toff;
@@ -1889,6 +1940,7 @@ pgh_status archi_create(pgh_archi **out, const pgh_island_spec *islands, uint64_
     place(a->desc, a->h_desc.size() * sizeof(island_desc));
     place(a->tiles, a->h_tiles.size() * sizeof(tile));
     place(a->segs, seg_list.size() * sizeof(seg_desc));
+    place(a->vsegs, vseg_list.size() * sizeof(seg_desc));
     place(a->jump_table, std::max<size_t>(tab.size(), 16u));
     place(a->states, n_islands * sizeof(mt_state));
     place(a->gblist, a->h_gb.size() * sizeof(uint32_t));
@@ -1901,6 +1953,7 @@ pgh_status archi_create(pgh_archi **out, const pgh_island_spec *islands, uint64_
     place(a->gbest, gboff * 8u);
     place(a->words, std::max<uint64_t>(woff, 1u) * 4u);
     place(a->seg_states, seg_list.size() * sizeof(mt_state));
+    place(a->states_q, n_islands * sizeof(mt_state));
     place(a->lbX1, xoff * 8u);
     place(a->lbfitB, foff * 8u);
     place(a->selA, foff * 4u);
@@ -1911,7 +1964,7 @@ pgh_status archi_create(pgh_archi **out, const pgh_island_spec *islands, uint64_
     auto *base = static_cast<uint8_t *>(a->arena.ptr);
     for (arena_view *v : {&a->desc, &a->tiles, &a->segs, &a->jump_table, &a->states, &a->gblist, &a->X, &a->V,
                           &a->lbX, &a->fit, &a->lbfit, &a->gbest, &a->words, &a->seg_states, &a->lbX1, &a->lbfitB,
-                          &a->selA, &a->selB, &a->queues}) {
+                          &a->selA, &a->selB, &a->queues, &a->vsegs, &a->states_q}) {
         v->ptr = base + v->off;
     }
     PGH_TRY(build_items(a.get()));
@@ -1923,14 +1976,12 @@ pgh_status archi_create(pgh_archi **out, const pgh_island_spec *islands, uint64_
         put(a->desc, a->h_desc.data(), a->h_desc.size() * sizeof(island_desc));
         put(a->tiles, a->h_tiles.data(), a->h_tiles.size() * sizeof(tile));
         put(a->segs, seg_list.data(), seg_list.size() * sizeof(seg_desc));
+        put(a->vsegs, vseg_list.data(), vseg_list.size() * sizeof(seg_desc));
         put(a->jump_table, tab.data(), tab.size());
         put(a->states, states.data(), n_islands * sizeof(mt_state));
         put(a->gblist, a->h_gb.data(), a->h_gb.size() * sizeof(uint32_t));
         PGH_HIP(hipMemcpy(base, head.data(), head_bytes, hipMemcpyHostToDevice));
     }
-    a->jt.lens = static_cast<const uint32_t *>(a->jump_table.ptr);
-    a->jt.lists = reinterpret_cast<const uint16_t *>(static_cast<const char *>(a->jump_table.ptr) +
-                                                     jump_table_head(dists.size()));
     for (uint64_t k = 0; k < n_islands; ++k) {
         const island_desc &di = a->h_desc[k];
         double *Xk = static_cast<double *>(a->X.ptr) + di.xoff;

@@ -13,95 +13,124 @@ using namespace dev;
 namespace
 {
 
-constexpr uint32_t kMtBlock = 256;
-
-// One workgroup: seed, discard `skip` words, hand out n words.
-__global__ __launch_bounds__(kMtBlock) void k_mt19937(uint32_t seed, uint64_t skip, uint64_t n,
-                                                      uint32_t *__restrict__ out)
-{
-    __shared__ uint32_t ring[kMtRing];
-    mt_seed_lds(seed, ring);
-    uint64_t K = 0;
-    if (skip) mt_run(ring, K, 0, skip, nullptr);
-    mt_run(ring, K, skip, n, out);
-}
+// Words handed out become U(lb_j, ub_j), two per element (generic.hpp:376-380),
+// element e of the row-major matrix at column e mod nx.  Every run starts at an
+// even word and has an even length.  COLS: the bounds depend on the column
+// (lennard_jones); otherwise they are column 0's.
+template <bool COLS>
+struct uniform_sink {
+    double *out;
+    uint64_t e0; // element of the hand-out's first word
+    uint32_t nx;
+    int kind;
+    double lb, w;
+    __device__ __forceinline__ uniform_sink(double *out_, uint64_t e0_, uint32_t nx_, int kind_)
+        : out(out_), e0(e0_), nx(nx_), kind(kind_)
+    {
+        double ub;
+        bounds_of(kind, 0u, lb, ub);
+        w = mt_width(lb, ub);
+    }
+    __device__ __forceinline__ void operator()(uint64_t at, const uint32_t *__restrict__ words, uint32_t n,
+                                               uint32_t tid, uint32_t nthr) const
+    {
+        const uint64_t e = e0 + at / 2u;
+        double *o = out + e;
+        const uint32_t c0 = COLS ? static_cast<uint32_t>(e % nx) : 0u;
+        for (uint32_t i = tid; i < n / 2u; i += nthr) {
+            const uint2 v = reinterpret_cast<const uint2 *>(words)[i];
+            double a = lb, wi = w;
+            if constexpr (COLS) {
+                double ub;
+                bounds_of(kind, (c0 + i) % nx, a, ub);
+                wi = mt_width(a, ub);
+            }
+            o[i] = mt_uniform(mt_temper(v.x), mt_temper(v.y), a, wi);
+        }
+    }
+};
 
 // Segment blockIdx.x = s of a stream split in segments of B words: words
-// [s B, min((s + 1) B, n)) of std::mt19937(seed), written to out at their
-// stream positions.  The segment's generator reaches s B by one jump,
-// z^(s B) (entry s - 1 of the jump table).
-__global__ __launch_bounds__(kMtJumpBlock) void k_mt19937_seg(uint32_t seed, uint64_t n, uint64_t B, uint32_t nd,
-                                                               const void *__restrict__ table,
-                                                               uint32_t *__restrict__ out)
+// [s B, min((s + 1) B, n)) of the generator that `st` holds, after `skip`
+// words (one segment only), handed to out (kElems, kElemsCols: as the elements
+// of a matrix of nx columns; else as words).  The segment's generator reaches s B
+// by one jump, z^(s B) (entry s - 1 of the table).
+// The mapping to doubles in the same pass saves writing the words and reading
+// them back.  65536 x 1000 on 500 segments: 1.13 ms -> 0.22 ms, about 0.1 ms of
+// it the jumps; the 524 MB of stores alone take 0.1 ms.
+enum : int { kWordsOut, kElems, kElemsCols };
+
+template <int OUT>
+__global__ __launch_bounds__(kMtBlock) void k_mt19937(mt_state st, uint64_t skip, uint64_t n, uint64_t B,
+                                                      const uint32_t *__restrict__ table, void *__restrict__ out,
+                                                      uint32_t nx, int kind)
 {
-    __shared__ uint32_t ring[kMtRing];
-    __shared__ uint4 lds_idx[kMtIdxStride / 8u];
-    mt_seed_lds(seed, ring);
-    uint64_t K = 0, C = 0;
-    const uint32_t s = blockIdx.x;
-    const uint32_t *lens = static_cast<const uint32_t *>(table);
-    const uint16_t *lists = reinterpret_cast<const uint16_t *>(static_cast<const char *>(table) + jump_table_head(nd));
-    if (s > 0u) {
-        mt_jump(ring, K, C, static_cast<uint64_t>(s) * B, lists + static_cast<uint64_t>(s - 1u) * kMtIdxStride,
-                lens[s - 1u], lds_idx);
+    __shared__ __align__(16) uint32_t buf[kMtBuf];
+    uint32_t pos;
+    mt_load(st, buf, pos);
+    const uint64_t s = blockIdx.x, begin = s * B;
+    if (s > 0u) mt_jump(buf, table + (s - 1u) * kMtN);
+    if (skip) mt_hand_out(buf, pos, skip, mt_no_sink{});
+    const uint64_t count = min(B, n - begin);
+    if constexpr (OUT != kWordsOut) {
+        mt_hand_out(buf, pos, count,
+                    uniform_sink<OUT == kElemsCols>(static_cast<double *>(out), begin / 2u, nx, kind));
+    } else {
+        mt_hand_out(buf, pos, count, mt_word_sink{static_cast<uint32_t *>(out) + begin});
     }
-    const uint64_t begin = static_cast<uint64_t>(s) * B;
-    mt_run(ring, K, C, min(B, n - begin), out + begin);
 }
 
-// In place: slot m holds the words 2m, 2m+1 and becomes U(lb_j, ub_j).
-__global__ __launch_bounds__(256) void k_uniform_inplace(double *__restrict__ io, uint64_t count, uint32_t nx,
-                                                         int kind)
+// The first n words after `skip` of std::mt19937(seed): one workgroup up to
+// kMtSplitMin words, else segments of B words, a power of two that makes at
+// most kMtMaxSegs of them and is at least kMtSegMin.  The jump polynomials
+// z^(s B) depend on B alone: the host makes them once per process, as
+// consecutive multiples, and the device keeps a table per B and power-of-two
+// count of them (2.5 KB each).  At most two segments per CU: 2^27 words take
+// 263 us in 512 segments, 291 us in 256 and 329 us in 1024 (a jump costs a CU as
+// much as making 1.5 10^5 words).  Split from 2^17 words on: one workgroup makes
+// 2^17 words in 52 us, a split call of 2^18 takes 77 us.
+constexpr uint64_t kMtSplitMin = uint64_t(1) << 17, kMtSegMin = uint64_t(1) << 14;
+constexpr uint32_t kMtMaxSegs = 512;
+// While the caller's stream is being captured no table is made for calls of up
+// to kMtCaptureSolo words: they run as one segment unless the table exists.
+constexpr uint64_t kMtCaptureSolo = uint64_t(1) << 21;
+
+template <int OUT>
+pgh_status launch_mt(uint32_t seed, uint64_t skip, uint64_t n, void *out, uint32_t nx, int kind, hipStream_t s)
 {
-    const uint64_t m = static_cast<uint64_t>(blockIdx.x) * 256u + threadIdx.x;
-    if (m >= count) return;
-    const uint2 w = reinterpret_cast<const uint2 *>(io)[m];
-    double lb, ub;
-    bounds_of(kind, static_cast<uint32_t>(m % nx), lb, ub);
-    io[m] = mt_uniform(w.x, w.y, lb, ub);
+    mt_state st;
+    mt_seed_host(seed, st);
+    uint64_t B = n;
+    const uint32_t *table = nullptr;
+    if (skip == 0u && n > kMtSplitMin) {
+        B = kMtSegMin;
+        while (B * kMtMaxSegs < n) B <<= 1;
+        const uint32_t segs = static_cast<uint32_t>((n + B - 1u) / B);
+        uint32_t count = 32u;
+        while (count < segs) count <<= 1;
+        PGH_TRY(jump_table_device(B, count - 1u, false, &table));
+        if (!table) {
+            hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+            if (n <= kMtCaptureSolo && hipStreamIsCapturing(s, &cs) != hipSuccess) (void)hipGetLastError();
+            if (cs == hipStreamCaptureStatusNone) {
+                PGH_TRY(jump_table_device(B, count - 1u, true, &table));
+            } else {
+                B = n;
+            }
+        }
+    }
+    const uint32_t segs = static_cast<uint32_t>((n + B - 1u) / B);
+    k_mt19937<OUT><<<dim3(segs), dim3(kMtBlock), 0, s>>>(st, skip, n, B, table, out, nx, kind);
+    PGH_HIP(hipGetLastError());
+    return PGH_OK;
 }
 
 } // namespace
 
-// The first n words of std::mt19937(seed) into out: one workgroup up to
-// kMtSplitMin words, else up to kMtMaxSegs workgroups, each starting its
-// segment by one jump.  The jump polynomials z^(s B) depend on B alone: the
-// host makes them once per process, as consecutive multiples
-// (jump_polys_multiples), and one device table per B holds all kMtMaxSegs - 1
-// of them (kept for the process: at most one per power of two B, 12 MB each),
-// whatever the number of segments of a call.
-constexpr uint64_t kMtSplitMin = uint64_t(1) << 21;
-constexpr uint32_t kMtMaxSegs = 256;
-
-pgh_status launch_mt_words(uint32_t seed, uint64_t n, uint32_t *out, hipStream_t s)
-{
-    if (n <= kMtSplitMin) {
-        k_mt19937<<<dim3(1), dim3(kMtBlock), 0, s>>>(seed, 0, n, out);
-        PGH_HIP(hipGetLastError());
-        return PGH_OK;
-    }
-    // B: the power of two that splits n into at most kMtMaxSegs segments
-    uint64_t B = 1;
-    while (B * kMtMaxSegs < n) B <<= 1;
-    const uint32_t segs = static_cast<uint32_t>((n + B - 1u) / B);
-    std::vector<uint64_t> dists;
-    for (uint32_t k = 1; k < kMtMaxSegs; ++k) dists.push_back(static_cast<uint64_t>(k) * B);
-    PGH_TRY(jump_polys_multiples(B, kMtMaxSegs - 1u));
-    const void *table = nullptr;
-    PGH_TRY(jump_table_device(dists, &table));
-    k_mt19937_seg<<<dim3(segs), dim3(kMtJumpBlock), 0, s>>>(seed, n, B, static_cast<uint32_t>(dists.size()), table,
-                                                             out);
-    PGH_HIP(hipGetLastError());
-    return PGH_OK;
-}
-
 pgh_status launch_mt19937(uint32_t seed, uint64_t skip, uint64_t n, uint32_t *out, hipStream_t s)
 {
     if (n == 0u) return PGH_OK;
-    if (skip == 0u) return launch_mt_words(seed, n, out, s);
-    k_mt19937<<<dim3(1), dim3(kMtBlock), 0, s>>>(seed, skip, n, out);
-    PGH_HIP(hipGetLastError());
-    return PGH_OK;
+    return launch_mt<kWordsOut>(seed, skip, n, out, 1u, 0, s);
 }
 
 pgh_status launch_batch_random_dv(const prob &p, uint64_t n, uint32_t seed, double *out, hipStream_t s)
@@ -111,11 +140,8 @@ pgh_status launch_batch_random_dv(const prob &p, uint64_t n, uint32_t seed, doub
     if (count == 0u) return PGH_OK;
     // every bound pair of the supported problems has lb < ub, so each element
     // consumes exactly two words (generic.hpp:376-380)
-    PGH_TRY(launch_mt_words(seed, 2u * count, reinterpret_cast<uint32_t *>(out), s));
-    k_uniform_inplace<<<dim3(static_cast<uint32_t>((count + 255u) / 256u)), dim3(256), 0, s>>>(out, count, p.nx,
-                                                                                                p.kind);
-    PGH_HIP(hipGetLastError());
-    return PGH_OK;
+    if (p.kind == LENNARD_JONES) return launch_mt<kElemsCols>(seed, 0u, 2u * count, out, p.nx, p.kind, s);
+    return launch_mt<kElems>(seed, 0u, 2u * count, out, p.nx, p.kind, s);
 }
 
 } // namespace pgh
