@@ -7,15 +7,18 @@
 //               after +inf and equals every NaN, and -0 equals +0
 //               (detail::less_than_f/greater_than_f/equal_to_f,
 //               include/pagmo/detail/custom_comparisons.hpp:54-100)
-//   k_pairs     one lane per row i against a chunk of columns j: builds the
-//               row-major dominance bit matrix D (bit j of row i set iff i
-//               dominates j, multi_objective.cpp:97-113), the number of rows
-//               dominating i (dom_count) and |dom_list[i]| (popcount of row i)
-//   k_scan      exclusive prefix of |dom_list[i]| -> dom_offsets
+//   k_pairs     (fnds_chain.hip) the number of rows dominating each row
+//               (dom_count) and, for the lists, the row-major dominance bit
+//               matrix D (bit j of row i set iff i dominates j,
+//               multi_objective.cpp:97-113) and |dom_list[i]|
+//   k_offsets,  exclusive prefix of |dom_list[i]| -> dom_offsets (the second
+//   k_scan      for n beyond one workgroup's LDS)
 //   k_emit      dom_list[i] = set bits of row i in increasing j: exactly the
 //               reference's push_back order (multi_objective.cpp:215-227 appends
 //               j < i while scanning row i, then larger indices in scan order)
-//   k_front0 +  the front peel (multi_objective.cpp:228-254), n <= 32768:
+// and the fronts (multi_objective.cpp:228-254):
+//   fnds_chain.hip   up to kChainMaxN points of one to kChainMaxM objectives
+//   k_front0 +  the peel, otherwise and n <= 32768:
 //   k_peel_cols F0 ascending; then per level, each workgroup decrements the
 //               counters of its own columns (in LDS) for the rows of the
 //               current front and records for each element the position of
@@ -44,68 +47,26 @@ constexpr uint32_t kBlock = 256;
 constexpr uint32_t kPeelBlock = 1024;
 
 
-__global__ __launch_bounds__(kBlock) void k_keys(const double *__restrict__ objs, uint64_t count,
-                                                 int64_t *__restrict__ keys)
+// Keys of the `count` objectives, and the counters of the n points cleared.
+__global__ __launch_bounds__(kBlock) void k_keys(const double *__restrict__ objs, uint64_t count, uint32_t n,
+                                                 int64_t *__restrict__ keys, uint32_t *__restrict__ cnt,
+                                                 uint32_t *__restrict__ ndom, uint32_t *__restrict__ last,
+                                                 uint64_t *__restrict__ scalars)
 {
     const uint64_t t = static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x;
     if (t < count) keys[t] = order_key(objs[t]);
+    if (t < n) {
+        cnt[t] = 0u;
+        ndom[t] = 0u;
+        last[t] = 0u;
+    }
+    if (t < 2u) scalars[2u + t] = 0u; // a peel's time-out; a front too large for one workgroup's sort
 }
 
 __global__ __launch_bounds__(kBlock) void k_fill_u32(uint32_t *__restrict__ p, uint64_t count, uint32_t v)
 {
     const uint64_t t = static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x;
     if (t < count) p[t] = v;
-}
-
-// Row i (one lane) against columns [j0, j0 + JC).  MT > 0: the row's keys are
-// held in registers; MT == 0: any m, keys re-read from memory.
-template <int MT>
-__global__ __launch_bounds__(kBlock) void k_pairs(const int64_t *__restrict__ keys, uint32_t n, uint32_t m,
-                                                  uint32_t jc, uint64_t *__restrict__ D, uint32_t words,
-                                                  uint32_t *__restrict__ dom_count, uint32_t *__restrict__ ndom)
-{
-    extern __shared__ int64_t kj[]; // jc x m
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    const uint32_t j0 = blockIdx.y * jc;
-    const uint32_t jn = min(jc, n - j0);
-    for (uint32_t t = threadIdx.x; t < jn * m; t += kBlock) kj[t] = keys[static_cast<uint64_t>(j0) * m + t];
-    __syncthreads();
-    if (i >= n) return;
-    int64_t ki[MT > 0 ? MT : 1];
-    if constexpr (MT > 0) {
-#pragma unroll
-        for (int q = 0; q < MT; ++q) ki[q] = keys[static_cast<uint64_t>(i) * MT + q];
-    }
-    uint32_t dominated_by = 0, dominates = 0;
-    for (uint32_t jb = 0; jb < jn; jb += 64u) {
-        uint64_t word = 0;
-        const uint32_t je = min(jb + 64u, jn);
-        for (uint32_t j = jb; j < je; ++j) {
-            bool lt = false, gt = false;
-            if constexpr (MT > 0) {
-#pragma unroll
-                for (int q = 0; q < MT; ++q) {
-                    const int64_t a = ki[q], b = kj[j * MT + q];
-                    lt |= a < b;
-                    gt |= a > b;
-                }
-            } else {
-                for (uint32_t q = 0; q < m; ++q) {
-                    const int64_t a = keys[static_cast<uint64_t>(i) * m + q], b = kj[j * m + q];
-                    lt |= a < b;
-                    gt |= a > b;
-                }
-            }
-            // pareto_dominance(i, j): no worse anywhere, better somewhere
-            const bool idomj = lt && !gt;
-            dominated_by += (gt && !lt) ? 1u : 0u;
-            word |= idomj ? (uint64_t(1) << (j - jb)) : uint64_t(0);
-        }
-        D[static_cast<uint64_t>(i) * words + (j0 + jb) / 64u] = word;
-        dominates += static_cast<uint32_t>(__popcll(word));
-    }
-    if (dominated_by) atomicAdd(&dom_count[i], dominated_by);
-    if (dominates) atomicAdd(&ndom[i], dominates);
 }
 
 __device__ __forceinline__ uint64_t shfl_up_u64(uint64_t v, uint32_t d)
@@ -167,35 +128,31 @@ __global__ __launch_bounds__(kPeelBlock) void k_scan(const uint32_t *__restrict_
     }
 }
 
-// dom_items: one wavefront per row; lane l takes words l, l+64, ... of the row
-// (coalesced), and a wavefront scan of the popcounts places every set bit,
-// so each row's items come out in increasing column order.
+// dom_items: one wavefront per row.  The row's words, 64 at a time, are taken
+// one after another (uniform): lane l stores column 64 w + l if its bit is set,
+// at the number of set bits below it, so a word's items are one contiguous
+// store and come out in increasing column order.  Bound by the stores (8192 x 2:
+// 135 MB; a lane per word, each storing its own run of items, took 100 us).
 __global__ __launch_bounds__(kBlock) void k_emit(const uint64_t *__restrict__ D, uint32_t n, uint32_t words,
                                                  const uint64_t *__restrict__ offsets, uint64_t *__restrict__ items)
 {
     const uint32_t row = blockIdx.x * (kBlock / 64u) + threadIdx.x / 64u;
     const uint32_t lane = threadIdx.x & 63u;
     if (row >= n) return; // whole wavefronts retire together
-    uint64_t o = offsets[row];
+    uint64_t *o = items + offsets[row];
     const uint64_t *r = D + static_cast<uint64_t>(row) * words;
     for (uint32_t w0 = 0; w0 < words; w0 += 64u) {
-        const uint32_t w = w0 + lane;
-        uint64_t word = w < words ? r[w] : 0u;
-        const uint32_t c = static_cast<uint32_t>(__popcll(word));
-        uint32_t x = c;
-#pragma unroll
-        for (uint32_t d = 1; d < 64u; d <<= 1) {
-            const uint32_t y = __shfl_up(x, d);
-            if (lane >= d) x += y;
+        const uint64_t mine = w0 + lane < words ? r[w0 + lane] : 0u;
+        uint64_t some = __ballot(mine != 0u);
+        while (some) {
+            const uint32_t k = static_cast<uint32_t>(__builtin_ctzll(some));
+            some &= some - 1u;
+            const uint32_t lo = __builtin_amdgcn_readlane(static_cast<uint32_t>(mine), k);
+            const uint32_t hi = __builtin_amdgcn_readlane(static_cast<uint32_t>(mine >> 32), k);
+            const uint32_t below = __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0u));
+            if (((lane < 32u ? lo : hi) >> (lane & 31u)) & 1u) o[below] = 64u * (w0 + k) + lane;
+            o += __builtin_popcount(lo) + __builtin_popcount(hi);
         }
-        const uint32_t total = __shfl(x, 63);
-        uint64_t pos = o + (x - c);
-        while (word) {
-            items[pos++] = static_cast<uint64_t>(w) * 64u +
-                           static_cast<uint32_t>(__ffsll(static_cast<unsigned long long>(word)) - 1);
-            word &= word - 1u;
-        }
-        o += total;
     }
 }
 
@@ -691,6 +648,102 @@ pgh_status thread_fnds_ws(pgh_fnds_ws **ws)
     return PGH_OK;
 }
 
+// The domination lists' offsets from the counts.
+static pgh_status scan_lists(pgh_fnds_ws *ws, hipStream_t s, uint32_t n)
+{
+    if (n <= kChainMaxN) return launch_offsets(ws, s, n);
+    k_scan<<<1, kPeelBlock, 0, s>>>(
+        static_cast<const uint32_t *>(ws->ndom32.ptr), static_cast<const uint32_t *>(ws->cnt32.ptr), n,
+        static_cast<uint64_t *>(ws->dom_offsets.ptr), static_cast<uint64_t *>(ws->dom_count.ptr),
+        static_cast<uint64_t *>(ws->scalars.ptr));
+    PGH_HIP(hipGetLastError());
+    return PGH_OK;
+}
+
+static pgh_status reserve_lists(pgh_fnds_ws *ws, uint64_t n)
+{
+    PGH_TRY(ws_carve(ws->lists_mem,
+                     {{&ws->D, n * ws->words * 8u}, {&ws->dom_count, n * 8u}, {&ws->dom_offsets, (n + 1u) * 8u}}));
+    return PGH_OK;
+}
+
+// The lists of a result that was made without them, from its keys.
+static pgh_status make_lists(pgh_fnds_ws *ws)
+{
+    const uint32_t n = static_cast<uint32_t>(ws->n);
+    PGH_TRY(reserve_lists(ws, ws->n));
+    k_fill_u32<<<grid_for(n), kBlock, 0, ws->stream>>>(static_cast<uint32_t *>(ws->cnt32.ptr), n, 0u);
+    k_fill_u32<<<grid_for(n), kBlock, 0, ws->stream>>>(static_cast<uint32_t *>(ws->ndom32.ptr), n, 0u);
+    PGH_HIP(hipGetLastError());
+    PGH_TRY(launch_pairs(ws, ws->stream, n, static_cast<uint32_t>(ws->m), true));
+    PGH_TRY(scan_lists(ws, ws->stream, n));
+    ws->lists = true;
+    return PGH_OK;
+}
+
+pgh_status fnds_all_items(pgh_fnds_ws *ws)
+{
+    if (ws->items) return PGH_OK;
+    PGH_TRY(launch_chain_items(ws, ws->stream, static_cast<uint32_t>(ws->n), static_cast<uint32_t>(ws->n)));
+    ws->items = true;
+    return PGH_OK;
+}
+
+pgh_status fnds_run(pgh_fnds_ws *ws, const double *objs, uint64_t n, uint64_t m, hipStream_t s, bool lists,
+                    uint64_t upto)
+{
+    if (!ws) return fail(PGH_INVALID_ARGUMENT, "null workspace");
+    ws->sized = false;
+    if (n < 2u) {
+        return fail(PGH_INVALID_ARGUMENT, "At least two points are needed for fast_non_dominated_sorting: "
+                                              + std::to_string(n) + " detected.");
+    }
+    if (n >= (uint64_t(1) << 31)) return fail(PGH_OVERFLOW, "too many points for fast_non_dominated_sorting");
+    if (m && !objs) return fail(PGH_INVALID_ARGUMENT, "null objective matrix");
+    if (m > 512u) return fail(PGH_UNSUPPORTED, "at most 512 objectives are supported");
+    const bool chain = n <= kChainMaxN && m >= 1u && m <= kChainMaxM && ws->peel_blocks == 0u;
+    ws->stream = s;
+    ws->n = 0u; // (no result while the buffers may be replaced)
+    ws->m = m;
+    ws->words = (n + 63u) / 64u;
+    ws->lists = lists || !chain; // a peel reads D
+    ws->items = upto >= n || !chain;
+    std::vector<ws_part> parts = {
+        {&ws->keys, n * m * 8u},         {&ws->cnt32, n * 4u},
+        {&ws->ndom32, n * 4u},           {&ws->key32, n * 4u},
+        {&ws->rank, n * 8u},             {&ws->front_items, n * 8u},
+        {&ws->front_offsets, (n + 1u) * 8u}, {&ws->scalars, 32u},
+    };
+    if (chain) chain_parts(ws, static_cast<uint32_t>(n), static_cast<uint32_t>(m), parts);
+    PGH_TRY(ws_carve(ws->main, parts));
+    if (ws->lists) PGH_TRY(reserve_lists(ws, n));
+    ws->n = n;
+    auto *cnt = static_cast<uint32_t *>(ws->cnt32.ptr);
+    auto *key = static_cast<uint32_t *>(ws->key32.ptr);
+    auto *scalars = static_cast<uint64_t *>(ws->scalars.ptr);
+    const uint32_t n32 = static_cast<uint32_t>(n), m32 = static_cast<uint32_t>(m);
+    const uint32_t w32 = static_cast<uint32_t>(ws->words);
+    k_keys<<<grid_for(std::max<uint64_t>(n * m, n)), kBlock, 0, s>>>(objs, n * m, n32,
+                                                                     static_cast<int64_t *>(ws->keys.ptr), cnt,
+                                                                     static_cast<uint32_t *>(ws->ndom32.ptr), key,
+                                                                     scalars);
+    PGH_HIP(hipGetLastError());
+    PGH_TRY(launch_pairs(ws, s, n32, m32, ws->lists));
+    if (ws->lists) PGH_TRY(scan_lists(ws, s, n32));
+    if (chain) return launch_chain_fronts(ws, s, n32, m32, static_cast<uint32_t>(std::min(upto, n)));
+    if (n <= kGridMaxN) {
+        PGH_TRY(ws->comp.reserve(n * 8u));
+        PGH_TRY(ws->ctl.reserve(2u * kColMaxG * 4u));
+        return launch_grid_peel(ws, s, n32, w32);
+    }
+    k_peel<<<1, kPeelBlock, 0, s>>>(static_cast<const uint64_t *>(ws->D.ptr), n32, w32, cnt, key,
+                                    static_cast<uint64_t *>(ws->front_items.ptr),
+                                    static_cast<uint64_t *>(ws->front_offsets.ptr),
+                                    static_cast<uint64_t *>(ws->rank.ptr), scalars);
+    PGH_HIP(hipGetLastError());
+    return PGH_OK;
+}
+
 } // namespace pgh
 
 using namespace pgh;
@@ -748,85 +801,7 @@ try {
 
 pgh_status pgh_fnds_run(pgh_fnds_ws *ws, const double *objs, uint64_t n, uint64_t m, void *stream)
 try {
-    if (!ws) return fail(PGH_INVALID_ARGUMENT, "null workspace");
-    ws->sized = false;
-    if (n < 2u) {
-        return fail(PGH_INVALID_ARGUMENT, "At least two points are needed for fast_non_dominated_sorting: "
-                                              + std::to_string(n) + " detected.");
-    }
-    if (n >= (uint64_t(1) << 31)) return fail(PGH_OVERFLOW, "too many points for fast_non_dominated_sorting");
-    if (m && !objs) return fail(PGH_INVALID_ARGUMENT, "null objective matrix");
-    if (m > 512u) return fail(PGH_UNSUPPORTED, "at most 512 objectives are supported");
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    ws->stream = s;
-    ws->n = n;
-    ws->m = m;
-    const uint64_t words = (n + 63u) / 64u;
-    ws->words = words;
-    PGH_TRY(ws->keys.reserve(std::max<uint64_t>(n * m, 1u) * 8u));
-    PGH_TRY(ws->D.reserve(n * words * 8u));
-    PGH_TRY(ws->cnt32.reserve(n * 4u));
-    PGH_TRY(ws->ndom32.reserve(n * 4u));
-    PGH_TRY(ws->key32.reserve(n * 4u));
-    PGH_TRY(ws->dom_count.reserve(n * 8u));
-    PGH_TRY(ws->rank.reserve(n * 8u));
-    PGH_TRY(ws->front_items.reserve(n * 8u));
-    PGH_TRY(ws->front_offsets.reserve((n + 1u) * 8u));
-    PGH_TRY(ws->dom_offsets.reserve((n + 1u) * 8u));
-    PGH_TRY(ws->scalars.reserve(32u));
-    auto *keys = static_cast<int64_t *>(ws->keys.ptr);
-    auto *D = static_cast<uint64_t *>(ws->D.ptr);
-    auto *cnt = static_cast<uint32_t *>(ws->cnt32.ptr);
-    auto *ndom = static_cast<uint32_t *>(ws->ndom32.ptr);
-    auto *key = static_cast<uint32_t *>(ws->key32.ptr);
-    const uint32_t n32 = static_cast<uint32_t>(n), m32 = static_cast<uint32_t>(m);
-    if (m) {
-        k_keys<<<grid_for(n * m), kBlock, 0, s>>>(objs, n * m, keys);
-        PGH_HIP(hipGetLastError());
-    }
-    k_fill_u32<<<grid_for(n), kBlock, 0, s>>>(cnt, n, 0u);
-    k_fill_u32<<<grid_for(n), kBlock, 0, s>>>(ndom, n, 0u);
-    k_fill_u32<<<grid_for(n), kBlock, 0, s>>>(key, n, 0u);
-    k_fill_u32<<<1, kBlock, 0, s>>>(static_cast<uint32_t *>(ws->scalars.ptr) + 4, 2u, 0u); // timeout flag
-    PGH_HIP(hipGetLastError());
-    // columns per workgroup: a multiple of 64 whose keys fit 32 KiB of LDS
-    uint32_t jc = 1024u;
-    while (jc > 64u && static_cast<uint64_t>(jc) * std::max<uint64_t>(m, 1u) * 8u > 32768u) jc >>= 1;
-    const size_t lds = static_cast<size_t>(jc) * std::max<uint64_t>(m, 1u) * 8u;
-    const dim3 grid(grid_for(n), static_cast<uint32_t>((n + jc - 1u) / jc));
-    const uint32_t w32 = static_cast<uint32_t>(words);
-    switch (m) {
-        case 1:
-            k_pairs<1><<<grid, kBlock, lds, s>>>(keys, n32, m32, jc, D, w32, cnt, ndom);
-            break;
-        case 2:
-            k_pairs<2><<<grid, kBlock, lds, s>>>(keys, n32, m32, jc, D, w32, cnt, ndom);
-            break;
-        case 3:
-            k_pairs<3><<<grid, kBlock, lds, s>>>(keys, n32, m32, jc, D, w32, cnt, ndom);
-            break;
-        case 4:
-            k_pairs<4><<<grid, kBlock, lds, s>>>(keys, n32, m32, jc, D, w32, cnt, ndom);
-            break;
-        default:
-            k_pairs<0><<<grid, kBlock, lds, s>>>(keys, n32, m32, jc, D, w32, cnt, ndom);
-    }
-    PGH_HIP(hipGetLastError());
-    auto *dom_offsets = static_cast<uint64_t *>(ws->dom_offsets.ptr);
-    auto *scalars = static_cast<uint64_t *>(ws->scalars.ptr);
-    k_scan<<<1, kPeelBlock, 0, s>>>(ndom, cnt, n32, dom_offsets, static_cast<uint64_t *>(ws->dom_count.ptr), scalars);
-    PGH_HIP(hipGetLastError());
-    if (n <= kGridMaxN) {
-        PGH_TRY(ws->comp.reserve(n * 8u));
-        PGH_TRY(ws->ctl.reserve(2u * kColMaxG * 4u));
-        PGH_TRY(launch_grid_peel(ws, s, n32, w32));
-    } else {
-        k_peel<<<1, kPeelBlock, 0, s>>>(D, n32, w32, cnt, key, static_cast<uint64_t *>(ws->front_items.ptr),
-                                        static_cast<uint64_t *>(ws->front_offsets.ptr),
-                                        static_cast<uint64_t *>(ws->rank.ptr), scalars);
-    }
-    PGH_HIP(hipGetLastError());
-    return PGH_OK;
+    return fnds_run(ws, objs, n, m, static_cast<hipStream_t>(stream), true, n);
 } catch (...) {
     return api_exception();
 }
@@ -858,7 +833,10 @@ try {
     const uint32_t w32 = (n32 + 63u) / 64u;
     uint32_t gmin = 0, gmax = 0;
     peel_range(w32, device_cus(), gmin, gmax);
+    // the peel's counts, and 0: the way taken without one (fnds_chain.hip up to
+    // kChainMaxN points)
     std::vector<uint32_t> cands;
+    if (n <= kChainMaxN && m >= 1u && m <= kChainMaxM) cands.push_back(0u);
     for (uint32_t per : {64u, 128u, 256u, 512u, 1024u}) {
         const uint32_t b = std::min(gmax, std::max(gmin, (n32 + per - 1u) / per));
         if (std::find(cands.begin(), cands.end(), b) == cands.end()) cands.push_back(b);
@@ -871,7 +849,7 @@ try {
         return hip_fail(ce, "hipEventCreate");
     }
     hipStream_t s = static_cast<hipStream_t>(stream);
-    float best = 0.f;
+    float best = 0.f, chain = 0.f;
     uint32_t best_b = 0u;
     pgh_status st = PGH_OK;
     for (uint32_t b : cands) {
@@ -894,7 +872,9 @@ try {
         }
         float ms = 0.f;
         if ((st = hip_status(hipEventElapsedTime(&ms, e0, e1), "hipEventElapsedTime")) != PGH_OK) break;
-        if (best_b == 0u || ms < best) {
+        if (b == 0u) {
+            chain = ms;
+        } else if (best_b == 0u || ms < best) {
             best = ms;
             best_b = b;
         }
@@ -905,7 +885,7 @@ try {
         ws->peel_blocks = 0u;
         return st;
     }
-    ws->peel_blocks = best_b;
+    ws->peel_blocks = chain > 0.f && chain <= best ? 0u : best_b;
     if (chosen) *chosen = best_b;
     // leave the workspace holding a result computed with the chosen grid
     return pgh_fnds_run(ws, objs, n, m, stream);
@@ -917,6 +897,8 @@ pgh_status pgh_fnds_sizes(pgh_fnds_ws *ws, uint64_t *n_fronts, uint64_t *n_dom_i
 try {
     if (!ws || !ws->n) return fail(PGH_INVALID_ARGUMENT, "fnds workspace has no result");
     if (!ws->sized) {
+        if (!ws->lists) PGH_TRY(make_lists(ws));
+        PGH_TRY(fnds_all_items(ws));
         PGH_HIP(hipMemcpyAsync(ws->h_sizes, ws->scalars.ptr, 24u, hipMemcpyDeviceToHost, ws->stream));
         PGH_HIP(hipStreamSynchronize(ws->stream));
         if (ws->h_sizes[2]) return fail(PGH_DEVICE_ERROR, "fast_non_dominated_sorting: a grid barrier timed out");

@@ -4,7 +4,9 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
+#include <vector>
 
 #include "pgh_internal.hpp"
 
@@ -20,6 +22,46 @@ __device__ __forceinline__ int64_t order_key(double x)
     const int64_t b = __double_as_longlong(x);
     return b >= 0 ? b : (b ^ INT64_MAX);
 }
+
+// Orders a wavefront's LDS writes before its following reads (its LDS accesses
+// execute in order; the compiler must keep them so).
+__device__ __forceinline__ void wave_lds_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// fnds_chain.hip takes up to kChainMaxN points (its sort keys, positions and bit
+// planes fit one workgroup's LDS) of one to kChainMaxM objectives.  With more
+// objectives the fronts are few and large, and the grid-wide peel, whose cost is
+// an exchange per front, is faster: 16384 x 3 (54 fronts) 0.70 against 0.90 ms
+// for the peel, 16384 x 5 (15 fronts) 1.30 against 0.67 ms; with two objectives
+// (8192: 176-213 fronts) 0.40 against 1.2-1.4 ms.
+constexpr uint32_t kChainMaxN = 16384, kChainMaxM = 3;
+
+// A buffer inside one of the workspace's allocations.
+struct ws_view {
+    void *ptr = nullptr;
+};
+struct ws_part {
+    ws_view *view;
+    uint64_t bytes;
+};
+// Lays the parts out in `mem`, grown if needed, each on a 256-byte boundary.
+inline pgh_status ws_carve(dev_buf &mem, const std::vector<ws_part> &parts)
+{
+    const auto padded = [](uint64_t b) { return (std::max<uint64_t>(b, 8u) + 255u) & ~uint64_t(255); };
+    uint64_t total = 0;
+    for (const ws_part &p : parts) total += padded(p.bytes);
+    PGH_TRY(mem.reserve(total));
+    auto *at = static_cast<char *>(mem.ptr);
+    for (const ws_part &p : parts) {
+        p.view->ptr = at;
+        at += padded(p.bytes);
+    }
+    return PGH_OK;
+}
 } // namespace pgh
 
 struct pgh_fnds_ws {
@@ -27,11 +69,22 @@ struct pgh_fnds_ws {
     hipStream_t own = nullptr; // created by the host-buffer entry points
     pgh::dev_buf staged;
     uint64_t n = 0, m = 0, words = 0;
-    pgh::dev_buf keys, D, cnt32, ndom32, key32, dom_count, rank, front_items, front_offsets, dom_offsets, dom_items,
-        scalars;
+    // every call's buffers, and those of the domination lists, in one device
+    // allocation each (a new workspace's first call took 26, 1.7 ms)
+    pgh::dev_buf main, lists_mem;
+    pgh::ws_view keys, cnt32, ndom32, key32, rank, front_items, front_offsets, scalars;
+    pgh::ws_view D, dom_count, dom_offsets;
+    pgh::dev_buf dom_items;
     pgh::dev_buf comp, ctl; // the grid peel's sort-key lists and flags (two halves each)
+    // fnds_chain.hip: the order by dominator count with the keys, counts and
+    // ranks in it, the dominance bits, what far blocks give a rank, the ranks'
+    // bit planes; ranks by index, front offsets, offsets of the fronts' words
+    // of `masks`, the members in any order and by index, and their positions
+    pgh::ws_view perm, skeys, scnt, srank, tiles, base, planes, rank32, fo32, wbase, any, members, masks, pos32;
     uint64_t h_sizes[3] = {0, 0, 0}; // n_fronts, n_dom_items, peel barrier timeout
     bool sized = false;
+    bool lists = false; // D, dom_offsets and dom_count hold this result's
+    bool items = false; // front_items holds every front's
     // workgroups of the grid-wide front peel: 0 = the default rule, else the
     // value set or found by pgh_fnds_tune (any count gives the same result)
     uint32_t peel_blocks = 0;
@@ -42,3 +95,27 @@ struct pgh_fnds_ws {
     // with its thread, never by pgh_fnds_destroy
     bool thread_owned = false;
 };
+
+namespace pgh
+{
+// The buffers of fnds_chain.hip for n points.
+void chain_parts(pgh_fnds_ws *ws, uint32_t n, uint32_t m, std::vector<ws_part> &parts);
+// Front offsets, items, ranks and the number of fronts of the n <= kChainMaxN
+// points whose keys and dominator counts the workspace holds (fnds_chain.hip);
+// the items of the fronts that start at or before `upto` only (n: all).
+pgh_status launch_chain_fronts(pgh_fnds_ws *ws, hipStream_t s, uint32_t n, uint32_t m, uint32_t upto);
+// The items again, for another `upto`.
+pgh_status launch_chain_items(pgh_fnds_ws *ws, hipStream_t s, uint32_t n, uint32_t upto);
+// Dominator counts (cnt32, zeroed before) from the keys and, with `lists`, D
+// and its rows' bit counts (ndom32, zeroed before).
+pgh_status launch_pairs(pgh_fnds_ws *ws, hipStream_t s, uint32_t n, uint32_t m, bool lists);
+// dom_offsets, dom_count and scalars[1] from those counts, n <= kChainMaxN.
+pgh_status launch_offsets(pgh_fnds_ws *ws, hipStream_t s, uint32_t n);
+// pgh_fnds_run, where they cost extra without the domination lists (D,
+// dom_offsets, dom_count) and the items of fronts that start after `upto`;
+// pgh_fnds_sizes makes what is missing when asked.
+pgh_status fnds_run(pgh_fnds_ws *ws, const double *objs, uint64_t n, uint64_t m, hipStream_t s, bool lists,
+                    uint64_t upto);
+// Makes the items that a run with a smaller `upto` left out.
+pgh_status fnds_all_items(pgh_fnds_ws *ws);
+} // namespace pgh

@@ -1,0 +1,93 @@
+"""The ranks and orders of fast_non_dominated_sorting without a peel, at the
+sizes where its parts change hands: blocks of 64 points, spans of 32 blocks,
+fronts of 64, 128 and 1024 members, bins of 64; and the orderings of fronts
+within and beyond one workgroup's sort.  Bit for bit with the oracle."""
+import numpy as np
+import pytest
+
+import oracle as O
+import pagmo2_amd as P
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+KEYS = ("dom_count", "rank", "front_offsets", "front_items", "dom_offsets", "dom_items")
+
+
+def dev(a):
+    return torch.from_numpy(np.ascontiguousarray(a, np.float64)).to("cuda:0")
+
+
+def check(objs):
+    ws = P.Fnds()
+    ws.run(dev(objs))
+    got = ws.to_host(len(objs))
+    ws.close()
+    ref = O.fnds(objs)
+    for k in KEYS:
+        assert np.array_equal(got[k], ref[k]), k
+
+
+def layers(sizes, seed, delta):
+    """Fronts of the given sizes for small deltas: points on anti-diagonals
+    x + y = L, L growing by delta; larger deltas leave fewer dominators."""
+    rng = np.random.default_rng(seed)
+    out = []
+    for L, c in enumerate(sizes):
+        x = np.sort(rng.uniform(0, 1, c))
+        out.append(np.stack([x + L * delta, 1 - x + L * delta], axis=1))
+    objs = np.concatenate(out)
+    return objs[rng.permutation(len(objs))]
+
+
+@pytest.mark.parametrize("n", [2, 3, 63, 64, 65, 127, 128, 129, 191, 193, 2047, 2048, 2049, 4097])
+@pytest.mark.parametrize("m", [1, 2, 3])
+def test_sizes(n, m):
+    check(np.random.default_rng(n + m).uniform(0, 1, (n, m)))
+
+
+@pytest.mark.parametrize("sizes", [(64, 64, 64), (65, 64, 65), (1, 128, 1, 128), (129, 128, 129), (64, 65, 128, 129),
+                                   (3, 1024, 1024, 2), (1025, 1024, 1025), (2, 3000, 2500), (1023, 700, 40, 90)])
+@pytest.mark.parametrize("delta", [2.0, 0.01, 0.0005])
+def test_front_sizes(sizes, delta):
+    check(layers(sizes, sum(sizes), delta))
+
+
+@pytest.mark.parametrize("kind", ["chain", "one front", "equal", "few values", "special", "one over all"])
+@pytest.mark.parametrize("n", [100, 2300])
+def test_shapes(kind, n):
+    rng = np.random.default_rng(n)
+    if kind == "chain":
+        objs = np.repeat(rng.permutation(n)[:, None], 3, axis=1).astype(float)
+    elif kind == "one front":
+        x = rng.uniform(0, 1, n)
+        objs = np.stack([x, -x], axis=1)
+    elif kind == "equal":
+        objs = np.full((n, 2), 0.5)
+    elif kind == "few values":
+        objs = rng.integers(0, 6, (n, 3)).astype(float)
+    elif kind == "special":
+        objs = rng.choice([np.nan, np.inf, -np.inf, -0.0, 0.0, 1.0, 5e-324, -1.0], (n, 3))
+    else:  # every member of front 1 has the same last dominator
+        x = rng.uniform(0, 1, n)
+        objs = np.stack([x, -x], axis=1)
+        objs[n // 3] = (-2.0, -2.0)
+    check(objs)
+
+
+@pytest.mark.parametrize("n,m", [(16384, 1), (16384, 2), (16385, 2)])
+def test_largest(n, m):
+    check(np.random.default_rng(m).uniform(0, 1, (n, m)))
+
+
+def test_equal_to_the_peel():
+    objs = dev(np.random.default_rng(4).uniform(0, 1, (12000, 3)))
+    ws = P.Fnds()
+    ws.run(objs)
+    a = ws.to_host(12000)
+    ws.set_peel_blocks(20)
+    ws.run(objs)
+    b = ws.to_host(12000)
+    ws.close()
+    for k in KEYS:
+        assert np.array_equal(a[k], b[k]), k
