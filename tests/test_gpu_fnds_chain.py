@@ -91,3 +91,53 @@ def test_equal_to_the_peel():
     ws.close()
     for k in KEYS:
         assert np.array_equal(a[k], b[k]), k
+
+
+@pytest.mark.parametrize("n,m,N", [(300, 2, 1), (300, 3, 150), (5000, 2, 2500), (5000, 3, 4999)])
+def test_results_after_a_selection(n, m, N):
+    """select_best_N_mo orders only the fronts it needs; the workspace still
+    gives every output of the sort afterwards."""
+    objs = np.random.default_rng(N).uniform(0, 1, (n, m))
+    objs[: n // 10] = objs[n // 2: n // 2 + n // 10]
+    ws = P.Fnds()
+    out = torch.empty(N, dtype=torch.int64, device="cuda:0")
+    assert ws.select_best_N_mo(dev(objs), N, out) == N
+    assert np.array_equal(out.cpu().numpy().astype(np.uint64), O.select_best_N_mo(objs, N, stable=True))
+    got = ws.to_host(n)
+    ws.close()
+    ref = O.fnds(objs)
+    for k in KEYS:
+        assert np.array_equal(got[k], ref[k]), k
+
+
+@pytest.mark.parametrize("sizes", [(4096, 10), (4097, 10), (5, 4500, 300), (700, 700, 700), (1, 1, 2, 1)])
+def test_orderings(sizes):
+    """Fronts of 4096 members and less are ordered by one workgroup each, larger
+    ones by radix sorts."""
+    objs = layers(sizes, 3, 0.02)
+    objs = np.concatenate([objs, objs[: len(objs) // 8]])  # duplicates
+    n = len(objs)
+    d = dev(objs)
+    ws = P.Fnds()
+    out = torch.empty(n, dtype=torch.int64, device="cuda:0")
+    ws.sort_population_mo(d, out)
+    assert np.array_equal(out.cpu().numpy().astype(np.uint64), O.sort_population_mo(objs, stable=True))
+    for N in (1, n // 3, n - 1):
+        got = torch.empty(N, dtype=torch.int64, device="cuda:0")
+        if ws.select_best_N_mo(d, N, got) == 0:
+            continue
+        assert np.array_equal(got.cpu().numpy().astype(np.uint64), O.select_best_N_mo(objs, N, stable=True)), N
+    ws.close()
+
+
+@pytest.mark.parametrize("n", [2, 3, 4095, 4096, 4097])
+@pytest.mark.parametrize("m", [2, 4])
+def test_crowding(n, m):
+    pts = np.random.default_rng(n).integers(0, max(2, n // 2), (n, m)).astype(float)
+    ws = P.Fnds()
+    out = torch.empty(n, dtype=torch.float64, device="cuda:0")
+    ws.crowding_distance(dev(pts), out)
+    ws.close()
+    ref = O.crowding_distance(pts, stable=True)
+    assert np.array_equal(out.cpu().numpy(), ref, equal_nan=True)
+    assert np.array_equal(P.crowding_distance_host(pts), ref, equal_nan=True)
