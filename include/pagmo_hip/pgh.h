@@ -315,8 +315,8 @@ pgh_status pgh_archi_get_trace(pgh_archi *a, uint64_t k, double *trace_F);
 
 /* Launch mapping of a generation (no counterpart in the reference; no
  * result depends on it): a generation moves, evaluates and updates the memory
- * of every island's individuals in items of rows, handed out by a queue to a
- * persistent grid.
+ * of every island's individuals in items of rows, a workgroup each, the
+ * costliest first.
  *   form:          PGH_ARCHI_STEP_ONE (the default), one launch per
  *                  generation over every item; PGH_ARCHI_STEP_SPLIT, one
  *                  launch per problem class (rosenbrock, separable,
@@ -324,9 +324,9 @@ pgh_status pgh_archi_get_trace(pgh_archi *a, uint64_t k, double *trace_F);
  *                  footprint (batched mode only)
  *   lj_lds:        LDS bytes for a Lennard-Jones item's staged individuals
  *                  (as many individuals per item as fit, at least one; 0 =
- *                  64 KiB, at most 64 KiB)
- *   blocks_per_cu: persistent workgroups per CU and launch (0 = as many as
- *                  can be resident)
+ *                  48 KiB, at most 64 KiB)
+ *   blocks_per_cu: resident workgroups per CU, at most (0 = as many as can
+ *                  be)
  * pgh_archi_tune times candidate mappings (form x lj_lds in {64, 32, 16}
  * KiB x blocks_per_cu in {0, 2}) with one batched evolve call each, `reps`
  * times, from the archipelago's current state, which it restores afterwards;

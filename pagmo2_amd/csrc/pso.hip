@@ -6,11 +6,11 @@
 // std::mt19937 state and a word buffer for a batch of kGenBatch generations
 // (in draw order: r1 and r2 of pso_gen.cpp:300-301 for variants 1 and 5, the
 // other variants' words as they draw them).  A generation is:
-//   k_step      one persistent launch (or one per problem class): workgroups
-//               take (island, rows) items from a queue and, per item, find
-//               each row's best neighbour (pso_gen.cpp:593-622), move the
-//               rows (:302-361), evaluate them with the batch evaluator's
-//               device routines and update the memory (:443-449)
+//   k_step      one launch (or one per problem class) with a workgroup per
+//               (island, rows) item: it finds each row's best neighbour
+//               (pso_gen.cpp:593-622), moves the rows (:302-361), evaluates
+//               them with the batch evaluator's device routines and updates
+//               the memory (:443-449)
 //   k_rng       on a second stream, during the current batch: the next
 //               batch's words, the island's generator split in segments that
 //               reach their own positions by jump-ahead (mt_dev.hpp,
@@ -623,9 +623,9 @@ __device__ __forceinline__ void eval_tile(const island_desc &di, const tile &tl,
 
 // ---- one generation of every island in one launch (k_step) ------------------
 // A generation's work is split in items: rows [first, first + count) of one
-// island.  A workgroup takes an item, moves its rows (best neighbour, velocity,
+// island.  A workgroup moves its item's rows (best neighbour, velocity,
 // position), evaluates them and updates their memory; a generation is one
-// launch of workgroups that take items from a queue until it is empty.
+// launch of a workgroup per item.
 //
 // Items of different islands, and of the same island, run concurrently.  A
 // particle's move reads the memory (lbX, lbfit) of its neighbours, which
@@ -657,16 +657,24 @@ __host__ __device__ constexpr uint32_t step_class(int kind)
     return kind == ROSENBROCK ? kStepRosen : (kind == LENNARD_JONES ? kStepLj : kStepSep);
 }
 
-// LDS of a rosenbrock item: each wavefront's term tile (rosenbrock_wave_rows)
+// LDS of a rosenbrock item: each wavefront's term tile (rosenbrock_wave_rows),
+// then the item's rows, if they are no more than kStepRosenElems elements
 constexpr uint32_t kStepRosenRows = (kBlock / 64u) * kRosenWaveRows;
-constexpr size_t kStepRosenLds = (kBlock / 64u) * kRosenWaveRows * kRosenWaveStride * sizeof(double);
+constexpr uint32_t kStepRosenTerms = (kBlock / 64u) * kRosenWaveRows * kRosenWaveStride, kStepRosenElems = 4096;
+constexpr size_t kStepRosenLds = (kStepRosenTerms + kStepRosenElems) * sizeof(double);
+// Default LDS for the individuals of a Lennard-Jones item: with it (and a
+// rosenbrock item's) three workgroups fit a CU (two: 101 against 88 us a
+// generation of the 32-island workload, 133 against 114 us of the 64-island one;
+// four, with 36 KiB: 90 and 111; 16 KiB cuts the items of 12 islands too small,
+// 56 against 51 us).
+constexpr uint32_t kStepLjLds = 49152;
+constexpr size_t kCuLds = 163840; // LDS of a CU
 
 struct step_args {
     const island_desc *d;
     const tile *items;
     const uint32_t *order; // item indices in the order they are handed out; null: base + i
     uint32_t base, n_items;
-    uint32_t *queue; // this launch's counter, zero before the launch
     const uint32_t *words;
     double *X, *V, *lbX0, *lbX1, *fit, *trace;
     const double *lbf_cur;
@@ -677,13 +685,23 @@ struct step_args {
     uint32_t gen;
 };
 
-// Per row of an item (at most kBlock rows): its best neighbour and the
-// memory rows of the particle and of that neighbour, found once per row
-// rather than once per element.
+// Per row of an item (at most kBlock rows): its best neighbour, the memory rows
+// of the particle and of that neighbour, and the particle's memory fitness, found
+// once per row rather than once per element (the fitness: before the evaluation
+// that is compared with it, which then waits for no load).
 struct step_rows {
+    double lbf[kBlock];
     uint32_t bn[kBlock];
     uint32_t sel[kBlock]; // bit 0: the particle's memory is in lbX1, bit 1: the neighbour's
 };
+
+__device__ __forceinline__ void step_row(step_rows &rw, uint32_t t, uint32_t bn, uint32_t p, const double *lbf,
+                                         const uint32_t *sel)
+{
+    rw.bn[t] = bn;
+    rw.sel[t] = (sel[p] ? 1u : 0u) | (sel[bn] ? 2u : 0u);
+    rw.lbf[t] = lbf[p];
+}
 
 // step_move for every variant and topology but variant 5 with lbest
 // (pso_gen.cpp:232-327): the best neighbour of the island's topology, or the
@@ -697,9 +715,7 @@ __device__ __noinline__ void step_move_general(const island_desc &di, const tile
     const bool fips = di.variant == 6u, gbest = di.topo == 1u;
     for (uint32_t t = threadIdx.x; t < tl.count; t += kBlock) {
         const uint32_t p = tl.first + t;
-        const uint32_t bn = (fips || gbest) ? p : best_neighbour_any(di, p, lbf);
-        rw.bn[t] = bn;
-        rw.sel[t] = (sel[p] ? 1u : 0u) | (sel[bn] ? 2u : 0u);
+        step_row(rw, t, (fips || gbest) ? p : best_neighbour_any(di, p, lbf), p, lbf, sel);
     }
     __syncthreads();
     const uint64_t e0 = static_cast<uint64_t>(tl.first) * di.nx;
@@ -740,61 +756,103 @@ __device__ __noinline__ void step_move_general(const island_desc &di, const tile
 }
 
 // Moves the rows of item tl (update_elem's arithmetic, the memory read through
-// the selectors).  All threads of the workgroup; a __syncthreads() must
-// follow.
+// the selectors); put(t, dd, x) gets row t's new element dd.  All threads of the
+// workgroup; a __syncthreads() must follow.
+// Bound by the latency of its loads: a thread moves U elements, kBlock apart, per
+// round with their five loads each issued together, and its row and column
+// advance by additions.  With U = 4 a generation of 4.1M elements moves alone in
+// 47 us (198 MB, 4.2 TB/s).  U = 8 spills (142 us a generation with everything
+// against 88), and loading the next round's words, positions and velocities
+// before a round's arithmetic takes registers and gives nothing (94 us).
 // GEN: the kernel serves an archipelago with islands of other variants or
 // topologies (a separate instantiation, so that the call of the out-of-line
-// path does not weigh on the register allocation of the default kernel).
-template <bool GEN>
-__device__ __forceinline__ void step_move(const island_desc &di, const tile &tl, const step_args &a, step_rows &rw)
+// path does not weigh on the register allocation of the default kernel); false
+// if it took that path, which does not call put.
+template <bool GEN, uint32_t U, class Put>
+__device__ __forceinline__ bool step_move(const island_desc &di, const tile &tl, const step_args &a, step_rows &rw,
+                                          Put put)
 {
     if constexpr (GEN) {
         if (di.variant != 5u || di.topo != 2u) { // island-uniform
             step_move_general(di, tl, a, rw);
-            return;
+            return false;
         }
     }
     const double *lbf = a.lbf_cur + di.foff;
     const uint32_t *sel = a.sel_cur + di.foff;
     for (uint32_t t = threadIdx.x; t < tl.count; t += kBlock) {
         const uint32_t p = tl.first + t;
-        const uint32_t bn = best_neighbour(p, di.pop, di.radius, lbf);
-        rw.bn[t] = bn;
-        rw.sel[t] = (sel[p] ? 1u : 0u) | (sel[bn] ? 2u : 0u);
+        step_row(rw, t, best_neighbour(p, di.pop, di.radius, lbf), p, lbf, sel);
     }
     __syncthreads();
     // item-local element e (count * nx < 2^32, build_items): row t, column dd
     const uint64_t e0 = static_cast<uint64_t>(tl.first) * di.nx;
-    const uint32_t span = tl.count * di.nx;
-    for (uint32_t e = threadIdx.x; e < span; e += kBlock) {
-        const uint32_t t = e / di.nx, dd = e - t * di.nx;
-        const uint64_t m = e0 + e;
-        const uint32_t bn = rw.bn[t], sb = rw.sel[t];
-        const uint4 w = *gen_words4(di, a.words, a.gen, m);
-        const double r1 = mt_canonical(w.x, w.y);
-        const double r2 = mt_canonical(w.z, w.w);
-        const uint64_t xi = di.xoff + m;
-        const double best = ((sb & 2u) ? a.lbX1 : a.lbX0)[di.xoff + static_cast<uint64_t>(bn) * di.nx + dd];
-        const double lbx = ((sb & 1u) ? a.lbX1 : a.lbX0)[xi];
-        double v;
-        a.X[xi] = pso_move(di, dd, a.X[xi], a.V[xi], lbx, best, r1, r2, v);
-        a.V[xi] = v;
+    const uint32_t span = tl.count * di.nx, nx = di.nx;
+    const uint4 *words = gen_words4(di, a.words, a.gen, e0);
+    double *X = a.X + di.xoff + e0, *V = a.V + di.xoff + e0;
+    const double *L0 = a.lbX0 + di.xoff, *L1 = a.lbX1 + di.xoff;
+    const uint32_t dq = kBlock / nx, dr = kBlock - dq * nx;
+    uint32_t t = threadIdx.x / nx, dd = threadIdx.x - t * nx;
+    for (uint32_t e = threadIdx.x; e < span;) {
+        const uint32_t left = span - e; // elements from e on
+        uint32_t tu[U], du[U], eu[U];
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+            // past the item's end: the round's first element again, not stored
+            const bool in = u * kBlock < left;
+            eu[u] = in ? e + u * kBlock : e;
+            tu[u] = in ? t : tu[0];
+            du[u] = in ? dd : du[0];
+            t += dq;
+            dd += dr;
+            if (dd >= nx) {
+                dd -= nx;
+                ++t;
+            }
+        }
+        uint4 w[U];
+        double x[U], v[U], lbx[U], best[U];
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+            const uint32_t sb = rw.sel[tu[u]];
+            const uint64_t own = e0 + eu[u], other = static_cast<uint64_t>(rw.bn[tu[u]]) * nx + du[u];
+            w[u] = words[eu[u]];
+            x[u] = X[eu[u]];
+            v[u] = V[eu[u]];
+            lbx[u] = ((sb & 1u) ? L1 : L0)[own];
+            best[u] = ((sb & 2u) ? L1 : L0)[other];
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+            const double r1 = mt_canonical(w[u].x, w[u].y), r2 = mt_canonical(w[u].z, w[u].w);
+            double vn;
+            const double xn = pso_move(di, du[u], x[u], v[u], lbx[u], best[u], r1, r2, vn);
+            if (u * kBlock < left) {
+                X[eu[u]] = xn;
+                V[eu[u]] = vn;
+                put(tu[u], du[u], xn);
+            }
+        }
+        if (left <= U * kBlock) break;
+        e += U * kBlock;
     }
+    return true;
 }
 
-// Memory update of particle p with fitness f (pso_gen.cpp:443-449) by the L
-// lanes of its group (lane r copies elements r, r + L, ...), and its fitness
-// and trace.
-__device__ __forceinline__ void step_remember(const island_desc &di, const step_args &a, uint32_t p, double f,
-                                              uint32_t r, uint32_t L)
+// Memory update of row t of the item with fitness f (pso_gen.cpp:443-449) by the
+// L lanes of its group (lane r copies elements r, r + L, ..., element i of the row
+// from x(i)), and its fitness and trace.
+template <class Elem>
+__device__ __forceinline__ void step_remember(const island_desc &di, const tile &tl, const step_args &a,
+                                              const step_rows &rw, uint32_t t, double f, uint32_t r, uint32_t L, Elem x)
 {
+    const uint32_t p = tl.first + t;
     const uint64_t fi = di.foff + p;
-    const double lbf = a.lbf_cur[fi];
-    const uint32_t s = a.sel_cur[fi];
+    const double lbf = rw.lbf[t];
+    const uint32_t s = rw.sel[t] & 1u;
     if (le_f(f, lbf)) {
-        const uint64_t row = di.xoff + static_cast<uint64_t>(p) * di.nx;
-        double *dst = (s ? a.lbX0 : a.lbX1) + row;
-        for (uint32_t i = r; i < di.nx; i += L) dst[i] = a.X[row + i];
+        double *dst = (s ? a.lbX0 : a.lbX1) + di.xoff + static_cast<uint64_t>(p) * di.nx;
+        for (uint32_t i = r; i < di.nx; i += L) dst[i] = x(i);
         if (r == 0u) {
             a.lbf_nxt[fi] = f;
             a.sel_nxt[fi] = s ^ 1u;
@@ -810,18 +868,21 @@ __device__ __forceinline__ void step_remember(const island_desc &di, const step_
 }
 
 // Rosenbrock: 8 rows per wavefront (rosenbrock_wave_rows), then the memory
-// update by the wavefront's 64 lanes, row by row.
+// update by the wavefront's 64 lanes, row by row.  X: the item's rows, in LDS or
+// in memory.
 __device__ __forceinline__ void step_eval_rosen(const island_desc &di, const tile &tl, const step_args &a,
-                                                double *lds)
+                                                const step_rows &rw, const double *X, double *terms)
 {
     const uint32_t wave = threadIdx.x / 64u, lane = threadIdx.x % 64u;
     const uint32_t r0 = wave * kRosenWaveRows;
     if (r0 >= tl.count) return; // wavefront-uniform
-    const uint32_t rows = min(kRosenWaveRows, tl.count - r0);
-    const uint32_t p0 = tl.first + r0;
-    const double f = rosenbrock_wave_rows(a.X + di.xoff + static_cast<uint64_t>(p0) * di.nx, rows, di.nx,
-                                          lds + wave * kRosenWaveRows * kRosenWaveStride, lane);
-    for (uint32_t r = 0; r < rows; ++r) step_remember(di, a, p0 + r, __shfl(f, static_cast<int>(r), 64), lane, 64u);
+    const uint32_t rows = min(kRosenWaveRows, tl.count - r0), nx = di.nx;
+    const double *first = X + static_cast<uint64_t>(r0) * nx;
+    const double f = rosenbrock_wave_rows(first, rows, nx, terms + wave * kRosenWaveRows * kRosenWaveStride, lane);
+    for (uint32_t r = 0; r < rows; ++r) {
+        step_remember(di, tl, a, rw, r0 + r, __shfl(f, static_cast<int>(r), 64), lane, 64u,
+                      [&](uint32_t i) { return first[static_cast<uint64_t>(r) * nx + i]; });
+    }
 }
 
 // An individual with an element beyond the streaming cosine's range, again
@@ -835,7 +896,8 @@ __device__ __noinline__ double step_sep_cold(const double *__restrict__ x, uint3
 }
 
 template <int KIND, int L>
-__device__ __forceinline__ void step_eval_sep_l(const island_desc &di, const tile &tl, const step_args &a)
+__device__ __forceinline__ void step_eval_sep_l(const island_desc &di, const tile &tl, const step_args &a,
+                                                const step_rows &rw)
 {
     const uint32_t g = threadIdx.x / L, r = threadIdx.x % L;
     const uint32_t gg = g < tl.count ? g : tl.count - 1u;
@@ -848,54 +910,56 @@ __device__ __forceinline__ void step_eval_sep_l(const island_desc &di, const til
         if (r == 0u) e = step_sep_cold<KIND>(x, di.nx);
         f = __shfl(e, 0, L);
     }
-    if (g < tl.count) step_remember(di, a, p, f, r, L);
+    if (g < tl.count) step_remember(di, tl, a, rw, gg, f, r, L, [x](uint32_t i) { return x[i]; });
 }
 
 template <int KIND>
-__device__ __forceinline__ void step_eval_sep(const island_desc &di, const tile &tl, const step_args &a)
+__device__ __forceinline__ void step_eval_sep(const island_desc &di, const tile &tl, const step_args &a,
+                                              const step_rows &rw)
 {
     switch (di.lanes) {
         case 64:
-            step_eval_sep_l<KIND, 64>(di, tl, a);
+            step_eval_sep_l<KIND, 64>(di, tl, a, rw);
             return;
         case 32:
-            step_eval_sep_l<KIND, 32>(di, tl, a);
+            step_eval_sep_l<KIND, 32>(di, tl, a, rw);
             return;
         case 16:
-            step_eval_sep_l<KIND, 16>(di, tl, a);
+            step_eval_sep_l<KIND, 16>(di, tl, a, rw);
             return;
         default:
-            step_eval_sep_l<KIND, 4>(di, tl, a);
+            step_eval_sep_l<KIND, 4>(di, tl, a, rw);
     }
 }
 
 template <int L, uint32_t APL>
-__device__ __forceinline__ void step_eval_lj_a(const island_desc &di, const tile &tl, const step_args &a, double *lds)
+__device__ __forceinline__ void step_eval_lj_a(const island_desc &di, const tile &tl, const step_args &a,
+                                               const step_rows &rw, const double *lds)
 {
     const uint32_t atoms = di.dim;
-    lj_stage(a.X + di.xoff + static_cast<uint64_t>(tl.first) * di.nx, tl.count, atoms, false, lds);
-    __syncthreads();
     const uint32_t g = threadIdx.x / L, r = threadIdx.x % L;
     if (g * L >= kBlock || g >= tl.count) return; // the item's groups
-    const double f = lj_energy<L, APL, false>(lds + g * lj_stride(atoms, false), atoms, static_cast<int>(r));
-    step_remember(di, a, tl.first + g, f, r, L);
+    const double *P = lds + g * lj_stride(atoms, false);
+    const double f = lj_energy<L, APL, false>(P, atoms, static_cast<int>(r));
+    step_remember(di, tl, a, rw, g, f, r, L, [P](uint32_t i) { return P[i ? i + 6u : 5u]; }); // lj_stage's places
 }
 
 template <int L>
-__device__ __forceinline__ void step_eval_lj_l(const island_desc &di, const tile &tl, const step_args &a, double *lds)
+__device__ __forceinline__ void step_eval_lj_l(const island_desc &di, const tile &tl, const step_args &a,
+                                               const step_rows &rw, const double *lds)
 {
     switch (lj_apl(di.dim, L)) {
         case 1:
-            step_eval_lj_a<L, 1>(di, tl, a, lds);
+            step_eval_lj_a<L, 1>(di, tl, a, rw, lds);
             return;
         case 2:
-            step_eval_lj_a<L, 2>(di, tl, a, lds);
+            step_eval_lj_a<L, 2>(di, tl, a, rw, lds);
             return;
         case 3:
-            step_eval_lj_a<L, 3>(di, tl, a, lds);
+            step_eval_lj_a<L, 3>(di, tl, a, rw, lds);
             return;
         case 4:
-            step_eval_lj_a<L, 4>(di, tl, a, lds);
+            step_eval_lj_a<L, 4>(di, tl, a, rw, lds);
             return;
         default:
             break;
@@ -903,47 +967,48 @@ __device__ __forceinline__ void step_eval_lj_l(const island_desc &di, const tile
     if constexpr (L >= 32) {
         switch (lj_apl(di.dim, L)) {
             case 5:
-                step_eval_lj_a<L, 5>(di, tl, a, lds);
+                step_eval_lj_a<L, 5>(di, tl, a, rw, lds);
                 return;
             case 6:
-                step_eval_lj_a<L, 6>(di, tl, a, lds);
+                step_eval_lj_a<L, 6>(di, tl, a, rw, lds);
                 return;
             case 7:
-                step_eval_lj_a<L, 7>(di, tl, a, lds);
+                step_eval_lj_a<L, 7>(di, tl, a, rw, lds);
                 return;
             case 8:
-                step_eval_lj_a<L, 8>(di, tl, a, lds);
+                step_eval_lj_a<L, 8>(di, tl, a, rw, lds);
                 return;
             default:
                 break;
         }
     }
-    step_eval_lj_a<L, 0>(di, tl, a, lds);
+    step_eval_lj_a<L, 0>(di, tl, a, rw, lds);
 }
 
-__device__ __forceinline__ void step_eval_lj(const island_desc &di, const tile &tl, const step_args &a, double *lds)
+__device__ __forceinline__ void step_eval_lj(const island_desc &di, const tile &tl, const step_args &a,
+                                             const step_rows &rw, const double *lds)
 {
     switch (di.lanes) {
         case 64:
-            step_eval_lj_l<64>(di, tl, a, lds);
+            step_eval_lj_l<64>(di, tl, a, rw, lds);
             return;
         case 32:
-            step_eval_lj_l<32>(di, tl, a, lds);
+            step_eval_lj_l<32>(di, tl, a, rw, lds);
             return;
         case 16:
-            step_eval_lj_l<16>(di, tl, a, lds);
+            step_eval_lj_l<16>(di, tl, a, rw, lds);
             return;
         case 8:
-            step_eval_lj_l<8>(di, tl, a, lds);
+            step_eval_lj_l<8>(di, tl, a, rw, lds);
             return;
         case 4:
-            step_eval_lj_l<4>(di, tl, a, lds);
+            step_eval_lj_l<4>(di, tl, a, rw, lds);
             return;
         case 2:
-            step_eval_lj_l<2>(di, tl, a, lds);
+            step_eval_lj_l<2>(di, tl, a, rw, lds);
             return;
         default:
-            step_eval_lj_l<1>(di, tl, a, lds);
+            step_eval_lj_l<1>(di, tl, a, rw, lds);
             return;
     }
 }
@@ -952,64 +1017,102 @@ template <uint32_t CLASS, bool GEN>
 __device__ __forceinline__ void step_item(const island_desc &di, const tile &tl, const step_args &a, double *lds,
                                           step_rows &rw)
 {
-    step_move<GEN>(di, tl, a, rw);
-    __syncthreads(); // the item's new rows are visible to the whole workgroup
+    // elements in flight per thread of the move: as many as the class's register
+    // budget takes
+    constexpr uint32_t U = CLASS == kStepAll || CLASS == kStepLj ? 4u : 2u;
     const uint32_t cls = CLASS == kStepAll ? step_class(di.kind) : CLASS;
+    // a rosenbrock item that fits and a Lennard-Jones item are staged in LDS as
+    // they are moved, so that the evaluation does not read them back from memory
     if (cls == kStepRosen) {
-        if constexpr (CLASS == kStepRosen || CLASS == kStepAll) step_eval_rosen(di, tl, a, lds);
+        if constexpr (CLASS == kStepRosen || CLASS == kStepAll) {
+            double *terms = lds, *rows = lds + kStepRosenTerms;
+            const uint32_t nx = di.nx;
+            const double *X = a.X + di.xoff + static_cast<uint64_t>(tl.first) * nx;
+            if (tl.count * nx <= kStepRosenElems) {
+                if (step_move<GEN, U>(di, tl, a, rw, [=](uint32_t t, uint32_t dd, double x) { rows[t * nx + dd] = x; })) {
+                    __syncthreads(); // the item's new rows are visible to the whole workgroup
+                    step_eval_rosen(di, tl, a, rw, rows, terms);
+                    return;
+                }
+            } else {
+                step_move<GEN, U>(di, tl, a, rw, [](uint32_t, uint32_t, double) {});
+            }
+            __syncthreads();
+            step_eval_rosen(di, tl, a, rw, X, terms);
+        }
     } else if (cls == kStepLj) {
-        if constexpr (CLASS == kStepLj || CLASS == kStepAll) step_eval_lj(di, tl, a, lds);
+        if constexpr (CLASS == kStepLj || CLASS == kStepAll) {
+            // lj_stage's places: element el of a row at el + 6, x[0] at 5, the
+            // fixed coordinates zero, and the first atoms again after the last
+            const uint32_t atoms = di.dim, stride = lj_stride(atoms, false), copy = 3u * atoms;
+            const uint32_t copied = 3u * lj_copy_atoms(atoms, false);
+            for (uint32_t z = threadIdx.x; z < 6u * tl.count; z += kBlock) {
+                const uint32_t g = z / 6u, zz = z - 6u * g, f = zz < 5u ? zz : 6u;
+                lds[g * stride + f] = 0.0;
+                if (f < copied) lds[g * stride + copy + f] = 0.0;
+            }
+            if (!step_move<GEN, U>(di, tl, a, rw, [=](uint32_t t, uint32_t dd, double x) {
+                    const uint32_t f = dd == 0u ? 5u : dd + 6u;
+                    double *ind = lds + t * stride;
+                    ind[f] = x;
+                    if (f < copied) ind[copy + f] = x;
+                })) {
+                __syncthreads();
+                lj_stage(a.X + di.xoff + static_cast<uint64_t>(tl.first) * di.nx, tl.count, atoms, false, lds);
+            }
+            __syncthreads();
+            step_eval_lj(di, tl, a, rw, lds);
+        }
     } else {
         if constexpr (CLASS == kStepSep || CLASS == kStepAll) {
+            step_move<GEN, U>(di, tl, a, rw, [](uint32_t, uint32_t, double) {});
+            __syncthreads(); // the item's new rows are visible to the whole workgroup
             switch (di.kind) {
                 case RASTRIGIN:
-                    step_eval_sep<RASTRIGIN>(di, tl, a);
+                    step_eval_sep<RASTRIGIN>(di, tl, a, rw);
                     break;
                 case ACKLEY:
-                    step_eval_sep<ACKLEY>(di, tl, a);
+                    step_eval_sep<ACKLEY>(di, tl, a, rw);
                     break;
                 case SCHWEFEL:
-                    step_eval_sep<SCHWEFEL>(di, tl, a);
+                    step_eval_sep<SCHWEFEL>(di, tl, a, rw);
                     break;
                 default:
-                    step_eval_sep<GRIEWANK>(di, tl, a);
+                    step_eval_sep<GRIEWANK>(di, tl, a, rw);
                     break;
             }
         }
     }
 }
 
-// One generation of the items order[0 .. n_items) (or base + i): a persistent
-// grid whose workgroups take items from the queue until it is empty (every
-// wavefront reads the same index, so all leave the loop together).
-// Wavefronts per SIMD each class's kernel is built for (its register budget):
-// the move phase streams from HBM and wants occupancy; the Lennard-Jones
-// evaluation wants registers for its atom slots.
+// One generation of item order[blockIdx.x] (or base + blockIdx.x): a workgroup
+// per item, so that nothing is kept over items.  (A persistent grid that took
+// items from a queue kept the constants of every class's evaluation over that
+// loop, more than the registers hold: each wavefront first stored 110 of them to
+// scratch, 150 of a generation's 320 MB at 4.1M elements, and read them back in
+// the evaluations.)  32 uneven islands, 4.1M elements: 70 us a generation against
+// 122; alone, the move takes 47 (memory) and the evaluation with the stores 50
+// (vector units, 29 us of issue).
+// Wavefronts per SIMD each class's kernel is built for (its register budget, so
+// that none spills in its loops): rosenbrock's move streams from memory and wants
+// occupancy, the separable and Lennard-Jones evaluations want registers.
 #ifndef PGH_STEP_BOUNDED
 #define PGH_STEP_BOUNDED 1
 #endif
 constexpr int step_min_waves(uint32_t cls)
 {
-    return !PGH_STEP_BOUNDED ? 1 : (cls == kStepRosen || cls == kStepSep ? 8 : (cls == kStepLj ? 4 : 3));
+    return !PGH_STEP_BOUNDED ? 1 : (cls == kStepRosen ? 8 : 4);
 }
 
 template <uint32_t CLASS, bool GEN>
 __global__ __launch_bounds__(kBlock, step_min_waves(CLASS)) void k_step(step_args a)
 {
     extern __shared__ double lds[];
-    __shared__ uint32_t s_next;
     __shared__ step_rows rw;
-    for (;;) {
-        if (threadIdx.x == 0) s_next = atomicAdd(a.queue, 1u);
-        __syncthreads();
-        const uint32_t i = s_next;
-        if (i >= a.n_items) return;
-        const uint32_t it = a.order ? a.order[i] : a.base + i;
-        const tile tl = a.items[it];
-        const island_desc di = a.d[tl.island];
-        if (a.gen < di.gens) step_item<CLASS, GEN>(di, tl, a, lds, rw);
-        __syncthreads(); // LDS and s_next are reused by the next item
-    }
+    const uint32_t it = a.order ? a.order[blockIdx.x] : a.base + blockIdx.x;
+    const tile tl = a.items[it];
+    const island_desc di = a.d[tl.island];
+    if (a.gen < di.gens) step_item<CLASS, GEN>(di, tl, a, lds, rw);
 }
 
 // gbest (pso_gen.cpp:644-662): the swarm's best position at the start of an
@@ -1282,11 +1385,10 @@ struct pgh_archi {
     arena_view gblist, gbest;
     std::vector<uint32_t> h_gb;
     bool general = false; // an island other than variant 5 with lbest: the step kernels with that path
-    // k_step: the second memory buffers, the selectors and one queue counter
-    // per launch (in the arena); its items (per island, contiguous) and their
-    // dispatch orders in a table of their own, rebuilt with the mapping
-    arena_view lbX1, lbfitB, selA, selB, queues;
-    uint64_t queue_stride = 0; // counters per generation: one per island, then one per step class
+    // k_step: the second memory buffers and the selectors (in the arena); its
+    // items (per island, contiguous) and their dispatch orders in a table of
+    // their own, rebuilt with the mapping
+    arena_view lbX1, lbfitB, selA, selB;
     dev_buf step_tab;
     const tile *d_items = nullptr;
     const uint32_t *d_order_all = nullptr, *d_order_cls = nullptr;
@@ -1296,7 +1398,7 @@ struct pgh_archi {
     size_t lj_lds = 0;                      // LDS of the Lennard-Jones items
     uint32_t n_cus = 0;
     pgh_archi_mapping map{PGH_ARCHI_STEP_ONE, 0u, 0u, 0u}; // the 64-island workload's fastest form
-    uint32_t step_per_cu[4] = {1u, 1u, 1u, 1u}; // k_step workgroups per CU, per class
+    size_t step_bytes[4] = {0, 0, 0, 0}; // k_step's dynamic LDS, per class
     uint32_t n_segs = 0;
     hipStream_t own = nullptr;
     hipStream_t side = nullptr; // a batched evolve's random words for the next batch
@@ -1355,7 +1457,7 @@ void step_occupancy(pgh_archi *a);
 
 pgh_status build_items(pgh_archi *a)
 {
-    const uint64_t budget = a->map.lj_lds ? a->map.lj_lds : 65536u;
+    const uint64_t budget = a->map.lj_lds ? a->map.lj_lds : kStepLjLds;
     a->h_items.clear();
     a->item_begin.assign(1u, 0u);
     a->lj_lds = 0u;
@@ -1419,33 +1521,6 @@ pgh_status build_items(pgh_archi *a)
     return PGH_OK;
 }
 
-size_t step_lds(const pgh_archi *a, uint32_t cls);
-
-// k_step workgroups per CU for each class at the current items' LDS: as many
-// as can be resident, or the mapping's count.
-void step_occupancy(pgh_archi *a)
-{
-    const void *fn[4] = {a->general ? reinterpret_cast<const void *>(&k_step<kStepRosen, true>)
-                                    : reinterpret_cast<const void *>(&k_step<kStepRosen, false>),
-                         a->general ? reinterpret_cast<const void *>(&k_step<kStepSep, true>)
-                                    : reinterpret_cast<const void *>(&k_step<kStepSep, false>),
-                         a->general ? reinterpret_cast<const void *>(&k_step<kStepLj, true>)
-                                    : reinterpret_cast<const void *>(&k_step<kStepLj, false>),
-                         a->general ? reinterpret_cast<const void *>(&k_step<kStepAll, true>)
-                                    : reinterpret_cast<const void *>(&k_step<kStepAll, false>)};
-    for (uint32_t c = 0; c < 4u; ++c) {
-        int per_cu = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn[c], static_cast<int>(kBlock), step_lds(a, c)) !=
-                hipSuccess ||
-            per_cu < 1) {
-            (void)hipGetLastError();
-            per_cu = 1;
-        }
-        if (a->map.blocks_per_cu) per_cu = std::min<int>(per_cu, static_cast<int>(a->map.blocks_per_cu));
-        a->step_per_cu[c] = static_cast<uint32_t>(per_cu);
-    }
-}
-
 size_t step_lds(const pgh_archi *a, uint32_t cls)
 {
     switch (cls) {
@@ -1460,13 +1535,24 @@ size_t step_lds(const pgh_archi *a, uint32_t cls)
     }
 }
 
-// Launches k_step<cls> over n_items items as a persistent grid: as many
-// workgroups as can be resident (or the mapping's count per CU), at most one
-// per item.
+// k_step's LDS for each class: what its items need, or as much as leaves room
+// for no more workgroups on a CU than the mapping's count.
+void step_occupancy(pgh_archi *a)
+{
+    for (uint32_t c = 0; c < 4u; ++c) {
+        a->step_bytes[c] = step_lds(a, c);
+        if (a->map.blocks_per_cu) {
+            const size_t share = kCuLds / a->map.blocks_per_cu, taken = sizeof(step_rows) + 1024u;
+            if (share > taken) a->step_bytes[c] = std::max(a->step_bytes[c], share - taken);
+        }
+    }
+}
+
+// Launches k_step<cls> over n_items items.
 pgh_status launch_step(const pgh_archi *a, uint32_t cls, const step_args &args, hipStream_t s)
 {
-    const size_t lds = step_lds(a, cls);
-    const uint32_t grid = std::min<uint32_t>(args.n_items, a->step_per_cu[cls] * a->n_cus);
+    const size_t lds = a->step_bytes[cls];
+    const uint32_t grid = args.n_items;
     if (grid == 0u) return PGH_OK;
     if (a->general) {
         switch (cls) {
@@ -1565,8 +1651,6 @@ pgh_status launch_range(pgh_archi *a, uint32_t i0, uint32_t i1, bool v_valid, bo
     auto *lbX1 = static_cast<double *>(a->lbX1.ptr);
     auto *lbfitB = static_cast<double *>(a->lbfitB.ptr);
     auto *selB = static_cast<uint32_t *>(a->selB.ptr);
-    auto *queues = static_cast<uint32_t *>(a->queues.ptr);
-    const uint32_t n_isl = static_cast<uint32_t>(a->h_desc.size());
     // ... and the next batch's words handed out beside it, into the other
     // half of the word buffer, when the generator is one segment
     const bool overlap = fused && a->words_half != 0u && a->h_desc[i0].segs == 1u;
@@ -1616,12 +1700,6 @@ pgh_status launch_range(pgh_archi *a, uint32_t i0, uint32_t i1, bool v_valid, bo
             }
         }
         if (fused) continue;
-        if (g == 0u) {
-            // this call's queue counters
-            const uint64_t nq = static_cast<uint64_t>(a->max_gens) * a->queue_stride;
-            k_zero_u32<<<blocks_for(nq), kBlock, 0, s>>>(queues, nq);
-            PGH_HIP(hipGetLastError());
-        }
         step_args args{};
         args.d = d;
         args.items = a->d_items;
@@ -1639,23 +1717,19 @@ pgh_status launch_range(pgh_archi *a, uint32_t i0, uint32_t i1, bool v_valid, bo
         args.sel_nxt = (g % 2u) ? selA : selB;
         args.gbest = gbest;
         args.gen = g;
-        uint32_t *qg = queues + static_cast<uint64_t>(g) * a->queue_stride;
         if (i1 == i0 + 1u) {
             // one island: its own items, in order
             args.base = a->item_begin[i0];
             args.n_items = a->item_begin[i1] - a->item_begin[i0];
-            args.queue = qg + i0;
             PGH_TRY(launch_step(a, step_class(a->h_desc[i0].kind), args, s));
         } else if (a->map.form == PGH_ARCHI_STEP_ONE) {
             args.order = a->d_order_all + a->item_begin[i0];
             args.n_items = a->item_begin[i1] - a->item_begin[i0];
-            args.queue = qg + n_isl + kStepAll;
             PGH_TRY(launch_step(a, kStepAll, args, s));
         } else {
             for (uint32_t c = 0; c < 3u; ++c) {
                 args.order = a->d_order_cls + a->class_begin[c];
                 args.n_items = a->class_begin[c + 1u] - a->class_begin[c];
-                args.queue = qg + n_isl + c;
                 PGH_TRY(launch_step(a, c, args, s));
             }
         }
@@ -1958,13 +2032,11 @@ pgh_status archi_create(pgh_archi **out, const pgh_island_spec *islands, uint64_
     place(a->lbfitB, foff * 8u);
     place(a->selA, foff * 4u);
     place(a->selB, foff * 4u);
-    a->queue_stride = n_islands + 4u;
-    place(a->queues, std::max<uint64_t>(a->max_gens, 1u) * a->queue_stride * 4u);
     PGH_TRY(a->arena.reserve(arena_bytes));
     auto *base = static_cast<uint8_t *>(a->arena.ptr);
     for (arena_view *v : {&a->desc, &a->tiles, &a->segs, &a->jump_table, &a->states, &a->gblist, &a->X, &a->V,
                           &a->lbX, &a->fit, &a->lbfit, &a->gbest, &a->words, &a->seg_states, &a->lbX1, &a->lbfitB,
-                          &a->selA, &a->selB, &a->queues, &a->vsegs, &a->states_q}) {
+                          &a->selA, &a->selB, &a->vsegs, &a->states_q}) {
         v->ptr = base + v->off;
     }
     PGH_TRY(build_items(a.get()));

@@ -1,0 +1,66 @@
+"""One generation of an archipelago (k_step) at the edges of its items: rows that
+fill a round of the move, miss one element of it or take several; rosenbrock items
+staged in LDS and too long for it; Lennard-Jones individuals from 3 atoms on; each
+with the default update rule and with the others.
+"""
+import numpy as np
+import pytest
+
+import oracle as O
+import pagmo2_amd as P
+from parity_bars import assert_fitness
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+
+def island(kind, dim, pop, gens, variant=5, topo=2):
+    X0, F0 = O.population_init(kind, dim, pop, 7)
+    return dict(kind=kind, dim=dim, X0=X0, F0=F0,
+                algo=P.pso_params(gen=gens, seed=13, variant=variant, neighb_type=topo))
+
+
+def evolve(islands, mode, mapping=None):
+    a = P.Archipelago(islands, trace=True)
+    if mapping:
+        a.set_mapping(*mapping)
+    a.evolve(mode)
+    out = [(a.get(k), a.trace(k)) for k in range(len(islands))]
+    a.close()
+    return out
+
+
+@pytest.mark.parametrize("variant,topo", [(5, 2), (1, 2), (6, 3)])
+@pytest.mark.parametrize("dim,pop", [
+    (2, 33), (32, 32),        # less than a round; exactly one
+    (128, 33), (129, 17),     # 32 rows of 4096 elements; 16 rows of 2064
+    (255, 9), (256, 17), (257, 16),
+    (512, 9), (513, 8),       # 8 rows: 4096 elements are staged, 4104 are not
+    (4100, 3),
+])
+def test_rosenbrock_items_against_oracle(dim, pop, variant, topo):
+    """Rosenbrock trajectories are the oracle's bit for bit."""
+    X0, F0 = O.population_init(P.ROSENBROCK, dim, pop, 7)
+    kw = dict(variant=variant, neighb_type=topo)
+    Xo, Fo = O.pso_gen_evolve(P.ROSENBROCK, dim, X0, F0, 4, 13, **kw)
+    for mode in (0, 1):
+        (X, F), _ = evolve([island(P.ROSENBROCK, dim, pop, 4, variant, topo)], mode)[0]
+        assert np.array_equal(X, Xo) and np.array_equal(F, Fo)
+
+
+@pytest.mark.parametrize("mapping", [None, (0, 0, 1), (1, 0, 0), (1, 4096, 3)])
+@pytest.mark.parametrize("variant,topo", [(5, 2), (2, 1)])
+def test_fitness_of_the_final_positions(variant, topo, mapping):
+    """Every item evaluates the rows that it moved: a row's final fitness is its
+    best over the generations and the batch evaluator's (at the kind's bar) at its
+    final position; every mapping and the island-by-island launches give one result."""
+    cases = [(P.LENNARD_JONES, 3, 300), (P.LENNARD_JONES, 4, 37), (P.LENNARD_JONES, 75, 20), (P.RASTRIGIN, 1, 300),
+             (P.ACKLEY, 31, 65), (P.SCHWEFEL, 257, 9), (P.GRIEWANK, 1025, 5), (P.ROSENBROCK, 513, 9)]
+    islands = [island(k, d, p, 5, variant, topo) for k, d, p in cases]
+    got = evolve(islands, 0, mapping)
+    for (kind, dim, _), isl, ((X, F), trace), ((Xp, Fp), tp) in zip(cases, islands, got, evolve(islands, 1)):
+        assert np.array_equal(X, Xp) and np.array_equal(F, Fp) and np.array_equal(trace, tp)
+        best = np.minimum(np.ravel(isl["F0"]), np.asarray(trace).reshape(5, -1).min(axis=0))
+        assert np.array_equal(np.ravel(F), best)
+        assert_fitness(kind, X, F, P.bfe_eval_host(kind, dim, X), (kind, dim))
