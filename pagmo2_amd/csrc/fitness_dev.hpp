@@ -425,8 +425,24 @@ __device__ __forceinline__ double rosenbrock_eval(const double *__restrict__ x, 
 {
     double retval = 0.;
     double xi = x[0];
-    for (uint32_t i = 0u; i + 1u < m_dim; ++i) {
-        const double xn = x[i + 1u];
+    uint32_t i = 1u;
+    // eight terms' loads and arithmetic together, then their sum in order: one
+    // term at a time waits for each load
+    for (; i + 8u <= m_dim; i += 8u) {
+        double xn[8], term[8];
+#pragma unroll
+        for (uint32_t u = 0; u < 8u; ++u) xn[u] = x[i + u];
+#pragma unroll
+        for (uint32_t u = 0; u < 8u; ++u) {
+            const double a = u ? xn[u - 1u] : xi, t = a * a - xn[u];
+            term[u] = 100. * t * t + (a - 1) * (a - 1);
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < 8u; ++u) retval += term[u];
+        xi = xn[7];
+    }
+    for (; i < m_dim; ++i) {
+        const double xn = x[i];
         const double t = xi * xi - xn;
         retval += 100. * t * t + (xi - 1) * (xi - 1);
         xi = xn;

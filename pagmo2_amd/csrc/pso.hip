@@ -105,10 +105,7 @@ constexpr uint32_t kSegCopy = 0xffffffffu;
 // (custom_comparisons.hpp:54-100): NaN is larger than everything but itself.
 __device__ __forceinline__ bool le_f(double a, double b)
 {
-    const bool an = a != a, bn = b != b;
-    if (an) return bn;
-    if (bn) return true;
-    return a <= b;
+    return (b != b) | (a <= b); // (a NaN: only with b NaN; b NaN: always)
 }
 
 __device__ __forceinline__ uint32_t find_island(const island_desc *__restrict__ d, uint32_t i0, uint32_t i1,
@@ -342,24 +339,43 @@ __device__ __forceinline__ uint32_t neighbour(const island_desc &di, uint32_t p,
 __device__ __noinline__ uint32_t best_neighbour_any(const island_desc &di, uint32_t p, const double *__restrict__ lbf)
 {
     uint32_t bn = neighbour(di, p, 0u);
+    double f = lbf[bn];
     for (uint32_t n = 1u; n < di.nbk; ++n) {
         const uint32_t q = neighbour(di, p, n);
-        if (le_f(lbf[q], lbf[bn])) bn = q;
+        const double fq = lbf[q];
+        if (le_f(fq, f)) {
+            bn = q;
+            f = fq;
+        }
     }
     return bn;
 }
 
+// The best's fitness is kept beside its index, so that no comparison waits for a
+// load that depends on the one before; the default's four neighbours are read
+// together.
 __device__ __forceinline__ uint32_t best_neighbour(uint32_t p, uint32_t S, uint32_t R, const double *__restrict__ lbf)
 {
-    uint32_t bn = p < R ? p - R + S : p - R;
-    for (uint32_t j = R - 1u; j >= 1u; --j) {
-        const uint32_t q = p < j ? p - j + S : p - j;
-        if (le_f(lbf[q], lbf[bn])) bn = q;
+    const auto before = [=](uint32_t j) { return p < j ? p - j + S : p - j; };
+    const auto after = [=](uint32_t j) { return p + j >= S ? p + j - S : p + j; };
+    uint32_t bn = before(R);
+    double f = lbf[bn];
+    const auto take = [&](uint32_t q, double fq) {
+        if (le_f(fq, f)) {
+            bn = q;
+            f = fq;
+        }
+    };
+    if (R == 2u) {
+        const uint32_t q1 = before(1u), q2 = after(1u), q3 = after(2u);
+        const double f1 = lbf[q1], f2 = lbf[q2], f3 = lbf[q3];
+        take(q1, f1);
+        take(q2, f2);
+        take(q3, f3);
+        return bn;
     }
-    for (uint32_t j = 1u; j <= R; ++j) {
-        const uint32_t q = p + j >= S ? p + j - S : p + j;
-        if (le_f(lbf[q], lbf[bn])) bn = q;
-    }
+    for (uint32_t j = R - 1u; j >= 1u; --j) take(before(j), lbf[before(j)]);
+    for (uint32_t j = 1u; j <= R; ++j) take(after(j), lbf[after(j)]);
     return bn;
 }
 
@@ -459,6 +475,9 @@ struct eval_ctx {
     uint32_t gen;
 };
 
+// The problem classes of the kernels that evolve.
+enum : uint32_t { kStepRosen = 0u, kStepSep = 1u, kStepLj = 2u, kStepAll = 3u };
+
 // Memory update of individual p by the L lanes of its group (lane r copies
 // elements r, r+L, ...).
 __device__ __forceinline__ void remember(const island_desc &di, const eval_ctx &c, uint32_t p, double f, uint32_t r,
@@ -475,8 +494,8 @@ __device__ __forceinline__ void remember(const island_desc &di, const eval_ctx &
     }
 }
 
-template <int KIND, int L>
-__device__ __forceinline__ void eval_separable(const island_desc &di, const tile &tl, const eval_ctx &c)
+template <int KIND, int L, class Rem>
+__device__ __forceinline__ void eval_separable(const island_desc &di, const tile &tl, const eval_ctx &c, Rem rem)
 {
     const uint32_t g = threadIdx.x / L, r = threadIdx.x % L;
     if (g * L >= kBlock) return;
@@ -496,29 +515,29 @@ __device__ __forceinline__ void eval_separable(const island_desc &di, const tile
         }
         f = __shfl(e, 0, L);
     }
-    if (g < tl.count) remember(di, c, p, f, r, L);
+    if (g < tl.count) rem(p, f, r, L);
 }
 
-template <int KIND>
-__device__ __forceinline__ void eval_sep_dispatch(const island_desc &di, const tile &tl, const eval_ctx &c)
+template <int KIND, class Rem>
+__device__ __forceinline__ void eval_sep_dispatch(const island_desc &di, const tile &tl, const eval_ctx &c, Rem rem)
 {
     switch (di.lanes) {
         case 64:
-            eval_separable<KIND, 64>(di, tl, c);
+            eval_separable<KIND, 64>(di, tl, c, rem);
             return;
         case 32:
-            eval_separable<KIND, 32>(di, tl, c);
+            eval_separable<KIND, 32>(di, tl, c, rem);
             return;
         case 16:
-            eval_separable<KIND, 16>(di, tl, c);
+            eval_separable<KIND, 16>(di, tl, c, rem);
             return;
         default:
-            eval_separable<KIND, 4>(di, tl, c);
+            eval_separable<KIND, 4>(di, tl, c, rem);
     }
 }
 
-template <int L, uint32_t APL>
-__device__ __forceinline__ void eval_lj_a(const island_desc &di, const tile &tl, const eval_ctx &c, double *lds)
+template <int L, uint32_t APL, class Rem>
+__device__ __forceinline__ void eval_lj_a(const island_desc &di, const tile &tl, const eval_ctx &c, double *lds, Rem rem)
 {
     const uint32_t atoms = di.dim;
     lj_stage(c.X + di.xoff + static_cast<uint64_t>(tl.first) * di.nx, tl.count, atoms, false, lds);
@@ -527,24 +546,24 @@ __device__ __forceinline__ void eval_lj_a(const island_desc &di, const tile &tl,
     if (g >= lj_group_count(atoms, false)) return;
     const uint32_t gg = g < tl.count ? g : tl.count - 1u;
     const double f = lj_energy<L, APL, false>(lds + gg * lj_stride(atoms, false), atoms, static_cast<int>(r));
-    if (g < tl.count) remember(di, c, tl.first + gg, f, r, L);
+    if (g < tl.count) rem(tl.first + gg, f, r, L);
 }
 
-template <int L>
-__device__ __forceinline__ void eval_lj(const island_desc &di, const tile &tl, const eval_ctx &c, double *lds)
+template <int L, class Rem>
+__device__ __forceinline__ void eval_lj(const island_desc &di, const tile &tl, const eval_ctx &c, double *lds, Rem rem)
 {
     switch (lj_apl(di.dim, L)) {
         case 1:
-            eval_lj_a<L, 1>(di, tl, c, lds);
+            eval_lj_a<L, 1>(di, tl, c, lds, rem);
             return;
         case 2:
-            eval_lj_a<L, 2>(di, tl, c, lds);
+            eval_lj_a<L, 2>(di, tl, c, lds, rem);
             return;
         case 3:
-            eval_lj_a<L, 3>(di, tl, c, lds);
+            eval_lj_a<L, 3>(di, tl, c, lds, rem);
             return;
         case 4:
-            eval_lj_a<L, 4>(di, tl, c, lds);
+            eval_lj_a<L, 4>(di, tl, c, lds, rem);
             return;
         default:
             break;
@@ -552,72 +571,73 @@ __device__ __forceinline__ void eval_lj(const island_desc &di, const tile &tl, c
     if constexpr (L >= 32) {
         switch (lj_apl(di.dim, L)) {
             case 5:
-                eval_lj_a<L, 5>(di, tl, c, lds);
+                eval_lj_a<L, 5>(di, tl, c, lds, rem);
                 return;
             case 6:
-                eval_lj_a<L, 6>(di, tl, c, lds);
+                eval_lj_a<L, 6>(di, tl, c, lds, rem);
                 return;
             case 7:
-                eval_lj_a<L, 7>(di, tl, c, lds);
+                eval_lj_a<L, 7>(di, tl, c, lds, rem);
                 return;
             case 8:
-                eval_lj_a<L, 8>(di, tl, c, lds);
+                eval_lj_a<L, 8>(di, tl, c, lds, rem);
                 return;
             default:
                 break;
         }
     }
-    eval_lj_a<L, 0>(di, tl, c, lds);
+    eval_lj_a<L, 0>(di, tl, c, lds, rem);
 }
 
-// Fitness and memory update of the individuals of tile tl (all threads of
-// the workgroup call it).
-__device__ __forceinline__ void eval_tile(const island_desc &di, const tile &tl, const eval_ctx &c, double *lds)
+// Fitness of the individuals of tile tl, each given to rem(p, f, r, L) by the L
+// lanes r of its group (all threads of the workgroup call it, at least kBlock).
+template <uint32_t CLASS, class Rem>
+__device__ __forceinline__ void eval_tile(const island_desc &di, const tile &tl, const eval_ctx &c, double *lds, Rem rem)
 {
-    switch (di.kind) {
-        case ROSENBROCK:
-            if (threadIdx.x < tl.count) {
-                const uint32_t p = tl.first + threadIdx.x;
-                const double f = rosenbrock_eval(c.X + di.xoff + static_cast<uint64_t>(p) * di.nx, di.nx);
-                remember(di, c, p, f, 0u, 1u);
-            }
-            return;
-        case RASTRIGIN:
-            eval_sep_dispatch<RASTRIGIN>(di, tl, c);
-            return;
-        case ACKLEY:
-            eval_sep_dispatch<ACKLEY>(di, tl, c);
-            return;
-        case SCHWEFEL:
-            eval_sep_dispatch<SCHWEFEL>(di, tl, c);
-            return;
-        case GRIEWANK:
-            eval_sep_dispatch<GRIEWANK>(di, tl, c);
-            return;
-        case LENNARD_JONES:
-            switch (di.lanes) {
-                case 64:
-                    eval_lj<64>(di, tl, c, lds);
-                    return;
-                case 32:
-                    eval_lj<32>(di, tl, c, lds);
-                    return;
-                case 16:
-                    eval_lj<16>(di, tl, c, lds);
-                    return;
-                case 8:
-                    eval_lj<8>(di, tl, c, lds);
-                    return;
-                case 4:
-                    eval_lj<4>(di, tl, c, lds);
-                    return;
-                case 2:
-                    eval_lj<2>(di, tl, c, lds);
-                    return;
-                default:
-                    eval_lj<1>(di, tl, c, lds);
-                    return;
-            }
+    if constexpr (CLASS == kStepRosen) {
+        if (threadIdx.x < tl.count) {
+            const uint32_t p = tl.first + threadIdx.x;
+            rem(p, rosenbrock_eval(c.X + di.xoff + static_cast<uint64_t>(p) * di.nx, di.nx), 0u, 1u);
+        }
+    } else if constexpr (CLASS == kStepSep) {
+        switch (di.kind) {
+            case RASTRIGIN:
+                eval_sep_dispatch<RASTRIGIN>(di, tl, c, rem);
+                return;
+            case ACKLEY:
+                eval_sep_dispatch<ACKLEY>(di, tl, c, rem);
+                return;
+            case SCHWEFEL:
+                eval_sep_dispatch<SCHWEFEL>(di, tl, c, rem);
+                return;
+            default:
+                eval_sep_dispatch<GRIEWANK>(di, tl, c, rem);
+                return;
+        }
+    } else {
+        switch (di.lanes) {
+            case 64:
+                eval_lj<64>(di, tl, c, lds, rem);
+                return;
+            case 32:
+                eval_lj<32>(di, tl, c, lds, rem);
+                return;
+            case 16:
+                eval_lj<16>(di, tl, c, lds, rem);
+                return;
+            case 8:
+                eval_lj<8>(di, tl, c, lds, rem);
+                return;
+            case 4:
+                eval_lj<4>(di, tl, c, lds, rem);
+                return;
+            case 2:
+                eval_lj<2>(di, tl, c, lds, rem);
+                return;
+            default:
+                eval_lj<1>(di, tl, c, lds, rem);
+                return;
+        }
     }
 }
 
@@ -639,8 +659,6 @@ __device__ __forceinline__ void eval_tile(const island_desc &di, const tile &tl,
 // So no generation writes anything that the same generation reads from
 // another item, and the arithmetic per element is that of the launch-per-phase
 // evolve (update_elem, eval_tile), bit for bit.
-
-enum : uint32_t { kStepRosen = 0u, kStepSep = 1u, kStepLj = 2u, kStepAll = 3u };
 
 // Lanes per Lennard-Jones individual in an archipelago: the batch evaluator's
 // for its cyclic schedule (lj_lanes_cyclic), or a whole wavefront from 80
@@ -1257,96 +1275,193 @@ __global__ __launch_bounds__(kBlock) void k_settle(const island_desc *__restrict
 }
 
 // Generations g0 .. g1 - 1 (within one batch of random words) of one island
-// that is a single evaluation tile, in one workgroup: k_update's and k_eval's
-// work in turn, with workgroup barriers where their launches would end.
-// Only this workgroup touches the island's X, V, lbX, fit and lbfit, so the
-// barriers order every write before the reads of the next phase.  STAGE: the
-// island is held in LDS for the batch, at byte offset stage_off of the
-// dynamic LDS (after the evaluation's own staging area), read at the start
-// and written back at the end; the arithmetic is the same.
+// that is a single evaluation tile, in one workgroup of kMtBlock threads: the
+// moves and the evaluation in turn, with workgroup barriers where their launches
+// would end.  Only this workgroup touches the island's X, V, lbX, fit and lbfit,
+// so the barriers order every write before the reads of the next phase.
+//
+// STAGE: the island is held in LDS for the batch, at byte offset stage_off of the
+// dynamic LDS (after the evaluation's own staging area), read at the start and
+// written back at the end; the arithmetic is the same.  A generation is then a
+// chain of LDS reads, arithmetic and two barriers, and what bounds it is that
+// chain's length.  So the positions are held twice and a row that improved is
+// only marked by its evaluation: in the next move its memory is its position
+// before that move, which the row's own elements enter in lbX meanwhile and
+// every other reader takes from there.  (A row's lane copying its elements after
+// its evaluation is a chain of its own.)  Row and column of a thread's elements
+// advance by additions, and a generation's first words are loaded a generation
+// ahead (loaded where they are needed: 2.0 us a generation).  A kernel per problem
+// class: one for all keeps every evaluation's constants over the generations and
+// spills (2.5 us).  Rosenbrock 64 x 10: 1.5 us a generation against 3.6, of them 1.0
+// the move, 0.4 the evaluation.
 //
 // With a second workgroup (gridDim.x == 2, an island whose generator is one
 // segment), that workgroup hands out the next batch's words (g1 ..) into
 // words_next, as k_rng would after this launch: the two workgroups
 // share no data, and the next launch reads those words.
-template <bool STAGE>
-__global__ __launch_bounds__(kBlock) void k_gens_one_tile(const island_desc *__restrict__ d,
-                                                          const tile *__restrict__ tiles, uint32_t island,
-                                                          uint32_t tl_index, const uint32_t *__restrict__ words,
-                                                          double *V, eval_ctx c, uint32_t g0, uint32_t g1,
-                                                          uint32_t stage_off, uint32_t *__restrict__ words_next,
-                                                          mt_state *__restrict__ st, mt_state *__restrict__ segst)
+template <uint32_t CLASS, bool STAGE>
+__global__ __launch_bounds__(kMtBlock) void k_gens_one_tile(const island_desc *__restrict__ d,
+                                                            const tile *__restrict__ tiles, uint32_t island,
+                                                            uint32_t tl_index, const uint32_t *__restrict__ words,
+                                                            double *V, eval_ctx c, uint32_t g0, uint32_t g1,
+                                                            uint32_t stage_off, uint32_t *__restrict__ words_next,
+                                                            mt_state *__restrict__ st, mt_state *__restrict__ segst)
 {
     extern __shared__ double lds[];
     const tile tl = tiles[tl_index];
     const island_desc di = d[island];
-    const uint64_t elems = static_cast<uint64_t>(di.pop) * di.nx;
     if (blockIdx.x == 1u) {
         // batch g1 / gps of a one-segment generator (k_rng's work; the
         // velocity draws shift the whole call's words alike)
         __shared__ __align__(16) uint32_t buf[kMtBuf];
         uint32_t pos;
-        mt_load<kBlock>(segst[di.seg0], buf, pos);
-        rng_gen_segment<kBlock>(di, 0u, g1 / di.gps, 0u, &st[island], &segst[di.seg0], words_next + di.woff, buf, pos);
+        mt_load(segst[di.seg0], buf, pos);
+        rng_gen_segment<kMtBlock>(di, 0u, g1 / di.gps, 0u, &st[island], &segst[di.seg0], words_next + di.woff, buf, pos);
         return;
     }
     const uint32_t end = min(g1, di.gens);
     if (g0 >= end) return;
-    island_desc dl = di;
-    eval_ctx cl = c;
-    double *Vl = V;
-    double *sX = nullptr, *sV = nullptr, *sL = nullptr, *sF = nullptr, *sLf = nullptr;
-    if constexpr (STAGE) {
-        sX = lds + stage_off / 8u;
-        sV = sX + elems;
-        sL = sV + elems;
-        sF = sL + elems;
-        sLf = sF + di.pop;
-        for (uint64_t m = threadIdx.x; m < elems; m += kBlock) {
-            sX[m] = c.X[di.xoff + m];
+    if constexpr (!STAGE) {
+        const uint64_t elems = static_cast<uint64_t>(di.pop) * di.nx;
+        for (uint32_t g = g0; g < end; ++g) {
+            for (uint64_t m = threadIdx.x; m < elems; m += kMtBlock) {
+                update_elem(di, m, words, c.X, V, c.lbX, c.lbfit, g);
+            }
+            __syncthreads();
+            eval_ctx cg = c;
+            cg.gen = g;
+            eval_tile<CLASS>(di, tl, cg, lds,
+                      [&](uint32_t p, double f, uint32_t r, uint32_t L) { remember(di, cg, p, f, r, L); });
+            __syncthreads();
+        }
+    } else {
+        const uint32_t nx = di.nx, elems = di.pop * nx; // staged: far below 2^32 (one_tile_bytes)
+        double *X0 = lds + stage_off / 8u, *X1 = X0 + elems, *sV = X1 + elems, *sL = sV + elems, *sF = sL + elems;
+        double *sLf = sF + di.pop;
+        uint32_t *better = reinterpret_cast<uint32_t *>(sLf + di.pop);
+        for (uint32_t m = threadIdx.x; m < elems; m += kMtBlock) {
+            X0[m] = c.X[di.xoff + m];
             sV[m] = V[di.xoff + m];
             sL[m] = c.lbX[di.xoff + m];
         }
-        for (uint32_t p = threadIdx.x; p < di.pop; p += kBlock) {
+        for (uint32_t p = threadIdx.x; p < di.pop; p += kMtBlock) {
             sF[p] = c.fit[di.foff + p];
             sLf[p] = c.lbfit[di.foff + p];
+            better[p] = 0u;
         }
         __syncthreads();
-        dl.xoff = 0u;
-        dl.foff = 0u;
-        dl.toff = 0u;
-        cl.X = sX;
-        cl.lbX = sL;
-        cl.fit = sF;
-        cl.lbfit = sLf;
-        cl.trace = c.trace ? c.trace + di.toff : nullptr;
-        Vl = sV;
-    }
-    for (uint32_t g = g0; g < end; ++g) {
-        for (uint64_t m = threadIdx.x; m < elems; m += kBlock) update_elem(dl, m, words, cl.X, Vl, cl.lbX, cl.lbfit, g);
-        __syncthreads();
-        eval_ctx cg = cl;
-        cg.gen = g;
-        eval_tile(dl, tl, cg, lds);
-        __syncthreads();
-    }
-    if constexpr (STAGE) {
-        for (uint64_t m = threadIdx.x; m < elems; m += kBlock) {
-            c.X[di.xoff + m] = sX[m];
+        const uint32_t dq = kMtBlock / nx, dr = kMtBlock - dq * nx;
+        const uint32_t t0 = threadIdx.x / nx, dd0 = threadIdx.x - t0 * nx;
+        double *X = X0, *Xn = X1;
+        // one round of the move: a thread's elements e, e + kMtBlock, ... (U of them,
+        // the first in row t, column dd) with the words w; past the island's end
+        // the first one again, not stored
+        constexpr uint32_t U = 2u;
+        const auto load = [&](uint4(&w)[U], const uint4 *from, uint32_t e) {
+#pragma unroll
+            for (uint32_t u = 0; u < U; ++u) w[u] = from[min(e + u * kMtBlock, elems - 1u)];
+        };
+        const auto move = [&](uint32_t e, uint32_t &t, uint32_t &dd, const uint4(&w)[U], const double *X, double *Xn) {
+            uint32_t eu[U], du[U], mine[U];
+            double x[U], v[U], lbx[U], best[U];
+#pragma unroll
+            for (uint32_t u = 0; u < U; ++u) {
+                const bool in = u * kMtBlock < elems - e;
+                eu[u] = in ? e + u * kMtBlock : e;
+                du[u] = in ? dd : du[0];
+                const uint32_t row = in ? t : 0u;
+                const uint32_t bn = best_neighbour(row, di.pop, di.radius, sLf);
+                x[u] = X[eu[u]];
+                v[u] = sV[eu[u]];
+                mine[u] = better[row];
+                lbx[u] = mine[u] ? x[u] : sL[eu[u]];
+                best[u] = (better[bn] ? X : sL)[bn * nx + du[u]];
+                t += dq;
+                dd += dr;
+                if (dd >= nx) {
+                    dd -= nx;
+                    ++t;
+                }
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < U; ++u) {
+                const double r1 = mt_canonical(w[u].x, w[u].y), r2 = mt_canonical(w[u].z, w[u].w);
+                double vn;
+                const double xn = pso_move(di, du[u], x[u], v[u], lbx[u], best[u], r1, r2, vn);
+                if (u * kMtBlock < elems - e) {
+                    Xn[eu[u]] = xn;
+                    sV[eu[u]] = vn;
+                    if (mine[u]) sL[eu[u]] = x[u];
+                }
+            }
+        };
+        // (the words of a generation's first round are loaded a generation ahead)
+        const uint4 *wg = gen_words4(di, words, g0, 0u);
+        uint4 w[U], wn[U];
+        load(w, wg, threadIdx.x);
+        for (uint32_t g = g0; g < end; ++g) {
+            const uint4 *next = gen_words4(di, words, min(g + 1u, end - 1u), 0u);
+            uint32_t t = t0, dd = dd0;
+            load(wn, next, threadIdx.x);
+            if (threadIdx.x < elems) move(threadIdx.x, t, dd, w, X, Xn);
+            for (uint32_t e = threadIdx.x; elems > U * kMtBlock + e;) {
+                e += U * kMtBlock;
+                uint4 wr[U];
+                load(wr, wg, e);
+                move(e, t, dd, wr, X, Xn);
+            }
+            wg = next;
+            __syncthreads();
+            island_desc dl = di;
+            dl.xoff = 0u;
+            eval_ctx cg{};
+            cg.X = Xn;
+            double *trace = c.trace ? c.trace + di.toff + static_cast<uint64_t>(g) * di.pop : nullptr;
+            eval_tile<CLASS>(dl, tl, cg, lds, [=](uint32_t p, double f, uint32_t r, uint32_t) {
+                if (r != 0u) return;
+                const bool b = le_f(f, sLf[p]);
+                if (b) sLf[p] = f;
+                better[p] = b ? 1u : 0u;
+                sF[p] = f;
+                if (trace) trace[p] = f;
+            });
+            __syncthreads();
+            double *const last = X;
+            X = Xn;
+            Xn = last;
+#pragma unroll
+            for (uint32_t u = 0; u < U; ++u) w[u] = wn[u];
+        }
+        uint32_t t = t0, dd = dd0;
+        for (uint32_t m = threadIdx.x; m < elems; m += kMtBlock) {
+            const double x = X[m];
+            c.X[di.xoff + m] = x;
             V[di.xoff + m] = sV[m];
-            c.lbX[di.xoff + m] = sL[m];
+            c.lbX[di.xoff + m] = better[t] ? x : sL[m];
+            t += dq;
+            dd += dr;
+            if (dd >= nx) {
+                dd -= nx;
+                ++t;
+            }
         }
-        for (uint32_t p = threadIdx.x; p < di.pop; p += kBlock) {
+        for (uint32_t p = threadIdx.x; p < di.pop; p += kMtBlock) {
             c.fit[di.foff + p] = sF[p];
             c.lbfit[di.foff + p] = sLf[p];
         }
     }
 }
 
-
 uint64_t align_up(uint64_t v, uint64_t a)
 {
     return (v + a - 1u) / a * a;
+}
+
+// LDS of an island that k_gens_one_tile holds, after the evaluation's area: two X,
+// V, lbX (pop x nx), fit, lbfit and the marks (pop).
+uint64_t one_tile_bytes(uint64_t pop, uint64_t nx)
+{
+    return (4u * pop * nx + 2u * pop) * 8u + align_up(pop * 4u, 8u);
 }
 
 // A buffer inside an archipelago's arena: its byte offset while the layout
@@ -1589,6 +1704,24 @@ pgh_status launch_step(const pgh_archi *a, uint32_t cls, const step_args &args, 
     return PGH_OK;
 }
 
+// k_gens_one_tile over the batch from generation g on of island i0 (tile t0).
+template <uint32_t CLASS>
+void launch_one_tile(pgh_archi *a, uint32_t grid, uint64_t stage_off, uint64_t stage_bytes, hipStream_t s, uint32_t i0,
+                     uint32_t t0, const uint32_t *w, uint32_t g, uint32_t *w_next)
+{
+    const auto *d = static_cast<const island_desc *>(a->desc.ptr);
+    const auto *tl = static_cast<const tile *>(a->tiles.ptr);
+    auto *V = static_cast<double *>(a->V.ptr);
+    auto *st = static_cast<mt_state *>(a->states.ptr), *segst = static_cast<mt_state *>(a->seg_states.ptr);
+    if (stage_bytes) {
+        k_gens_one_tile<CLASS, true><<<grid, kMtBlock, stage_off + stage_bytes, s>>>(
+            d, tl, i0, t0, w, V, make_ctx(a, g), g, g + kGenBatch, static_cast<uint32_t>(stage_off), w_next, st, segst);
+    } else {
+        k_gens_one_tile<CLASS, false><<<grid, kMtBlock, a->lds_bytes, s>>>(d, tl, i0, t0, w, V, make_ctx(a, g), g,
+                                                                           g + kGenBatch, 0u, w_next, st, segst);
+    }
+}
+
 // Launches the evolve call for islands [i0, i1) on stream s.  v_valid: the
 // islands have velocities from an earlier call (kept by those with memory).
 pgh_status launch_range(pgh_archi *a, uint32_t i0, uint32_t i1, bool v_valid, bool from_lb, hipStream_t s)
@@ -1638,16 +1771,15 @@ pgh_status launch_range(pgh_archi *a, uint32_t i0, uint32_t i1, bool v_valid, bo
         k_gbest_init<<<n_gb, kBlock, 0, s>>>(d, gbl, X, fit, gbest);
         PGH_HIP(hipGetLastError());
     }
-    // the island in LDS when it fits beside the evaluation's staging area
-    // within 64 KiB: X, V, lbX (pop x nx) and fit, lbfit (pop)
+    // the island in LDS when it fits beside the evaluation's staging area and the
+    // generator's buffer
     const uint64_t stage_off = align_up(a->lds_bytes, 256u);
     uint64_t stage_bytes = 0u;
     if (fused) {
         const island_desc &di = a->h_desc[i0];
-        const uint64_t need = (3u * static_cast<uint64_t>(di.pop) * di.nx + 2u * di.pop) * 8u;
-        if (stage_off + need <= 65536u) stage_bytes = need;
+        const uint64_t need = one_tile_bytes(di.pop, di.nx);
+        if (stage_off + need + kMtBuf * 4u + 1024u <= kCuLds) stage_bytes = need;
     }
-    const auto *tl = static_cast<const tile *>(a->tiles.ptr);
     auto *lbX1 = static_cast<double *>(a->lbX1.ptr);
     auto *lbfitB = static_cast<double *>(a->lbfitB.ptr);
     auto *selB = static_cast<uint32_t *>(a->selB.ptr);
@@ -1689,12 +1821,16 @@ pgh_status launch_range(pgh_archi *a, uint32_t i0, uint32_t i1, bool v_valid, bo
                 const uint32_t *wc = w + (overlap ? (b % 2u) * a->words_half : 0u);
                 uint32_t *wn = w + (overlap ? ((b + 1u) % 2u) * a->words_half : 0u);
                 const uint32_t grid = overlap && g + kGenBatch < gens ? 2u : 1u;
-                if (stage_bytes) {
-                    k_gens_one_tile<true><<<grid, kBlock, stage_off + stage_bytes, s>>>(
-                        d, tl, i0, t0, wc, V, make_ctx(a, g), g, g + kGenBatch, stage_off, wn, st, segst);
-                } else {
-                    k_gens_one_tile<false><<<grid, kBlock, a->lds_bytes, s>>>(d, tl, i0, t0, wc, V, make_ctx(a, g), g,
-                                                                              g + kGenBatch, 0u, wn, st, segst);
+                switch (step_class(a->h_desc[i0].kind)) {
+                    case kStepRosen:
+                        launch_one_tile<kStepRosen>(a, grid, stage_off, stage_bytes, s, i0, t0, wc, g, wn);
+                        break;
+                    case kStepSep:
+                        launch_one_tile<kStepSep>(a, grid, stage_off, stage_bytes, s, i0, t0, wc, g, wn);
+                        break;
+                    default:
+                        launch_one_tile<kStepLj>(a, grid, stage_off, stage_bytes, s, i0, t0, wc, g, wn);
+                        break;
                 }
                 PGH_HIP(hipGetLastError());
             }

@@ -64,3 +64,28 @@ def test_fitness_of_the_final_positions(variant, topo, mapping):
         best = np.minimum(np.ravel(isl["F0"]), np.asarray(trace).reshape(5, -1).min(axis=0))
         assert np.array_equal(np.ravel(F), best)
         assert_fitness(kind, X, F, P.bfe_eval_host(kind, dim, X), (kind, dim))
+
+
+@pytest.mark.parametrize("kind,dim,pop,param", [
+    (P.ROSENBROCK, 2, 5, 4),      # fewer elements than threads
+    (P.ROSENBROCK, 8, 64, 4),     # 512 elements: one each
+    (P.ROSENBROCK, 27, 19, 4),    # 513
+    (P.ROSENBROCK, 16, 64, 2),    # 1024: one round, two neighbours
+    (P.ROSENBROCK, 25, 41, 6),    # 1025: a second round, six neighbours
+    (P.ROSENBROCK, 600, 3, 2),    # rows longer than the workgroup
+    (P.ROSENBROCK, 16, 256, 4),   # the largest tile held in LDS
+    (P.ROSENBROCK, 17, 256, 4),   # not held
+    (P.RASTRIGIN, 1, 16, 2), (P.GRIEWANK, 65, 4, 2), (P.SCHWEFEL, 33, 16, 4), (P.ACKLEY, 300, 5, 4),
+    (P.LENNARD_JONES, 3, 9, 4), (P.LENNARD_JONES, 75, 4, 2),
+])
+def test_one_shot_tiles(kind, dim, pop, param):
+    """pgh_pso_gen_evolve_host of a single tile equals the archipelago's launches bit
+    for bit (and the oracle's, for rosenbrock) over two batches of words."""
+    X0, F0 = O.population_init(kind, dim, pop, 3)
+    prm = dict(gen=35, seed=21, neighb_param=param)
+    Xh, Fh = P.pso_gen_evolve_host(kind, dim, X0, F0, P.pso_params(**prm))
+    (Xa, Fa), _ = evolve([dict(kind=kind, dim=dim, X0=X0, F0=F0, algo=P.pso_params(**prm))], 1)[0]
+    assert np.array_equal(Xh, Xa) and np.array_equal(np.ravel(Fh), np.ravel(Fa))
+    if kind == P.ROSENBROCK:
+        Xo, Fo = O.pso_gen_evolve(kind, dim, X0, F0, 35, 21, neighb_param=param)
+        assert np.array_equal(Xh, Xo) and np.array_equal(Fh, Fo)
