@@ -132,7 +132,9 @@ __global__ __launch_bounds__(kPeelBlock) void k_scan(const uint32_t *__restrict_
 // one after another (uniform): lane l stores column 64 w + l if its bit is set,
 // at the number of set bits below it, so a word's items are one contiguous
 // store and come out in increasing column order.  Bound by the stores (8192 x 2:
-// 135 MB; a lane per word, each storing its own run of items, took 100 us).
+// 135 MB in 41 us; a lane per word, each storing its own run of items, took 100),
+// so it writes the caller's memory where it can: the copy from a buffer of its
+// own took 48 us more.
 __global__ __launch_bounds__(kBlock) void k_emit(const uint64_t *__restrict__ D, uint32_t n, uint32_t words,
                                                  const uint64_t *__restrict__ offsets, uint64_t *__restrict__ items)
 {
@@ -154,6 +156,24 @@ __global__ __launch_bounds__(kBlock) void k_emit(const uint64_t *__restrict__ D,
             o += __builtin_popcount(lo) + __builtin_popcount(hi);
         }
     }
+}
+
+// Up to five ranges of words copied by one launch (blockIdx.y: the range), each of
+// at most gridDim.x * kBlock words: a copy per range took 4 us and a gap each.
+struct out_range {
+    uint64_t *dst;
+    const uint64_t *src;
+    uint64_t count;
+};
+struct out_ranges {
+    out_range r[5];
+    uint32_t used;
+};
+__global__ __launch_bounds__(kBlock) void k_copy_out(out_ranges o)
+{
+    const out_range r = o.r[blockIdx.y];
+    const uint64_t i = static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x;
+    if (i < r.count) r.dst[i] = r.src[i];
 }
 
 __device__ __forceinline__ uint32_t ld_relaxed(const uint32_t *p)
@@ -681,6 +701,30 @@ static pgh_status make_lists(pgh_fnds_ws *ws)
     return PGH_OK;
 }
 
+// dom_items of the result into `to` (this device's memory, its size known).
+static pgh_status emit_items(pgh_fnds_ws *ws, uint64_t *to)
+{
+    k_emit<<<static_cast<uint32_t>((ws->n + 3u) / 4u), kBlock, 0, ws->stream>>>(
+        static_cast<const uint64_t *>(ws->D.ptr), static_cast<uint32_t>(ws->n), static_cast<uint32_t>(ws->words),
+        static_cast<const uint64_t *>(ws->dom_offsets.ptr), to);
+    PGH_HIP(hipGetLastError());
+    return PGH_OK;
+}
+
+// A kernel beside `here` (device memory) can write words to p: null, or aligned
+// memory of the same device.  (A copy also takes peers' and host memory.)
+static bool writable_here(const void *p, const void *here)
+{
+    if (!p) return true;
+    if (reinterpret_cast<uintptr_t>(p) & 7u) return false;
+    hipPointerAttribute_t a{}, b{};
+    if (hipPointerGetAttributes(&a, p) != hipSuccess || hipPointerGetAttributes(&b, here) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return a.type == hipMemoryTypeDevice && b.type == hipMemoryTypeDevice && a.device == b.device;
+}
+
 pgh_status fnds_all_items(pgh_fnds_ws *ws)
 {
     if (ws->items) return PGH_OK;
@@ -902,14 +946,8 @@ try {
         PGH_HIP(hipMemcpyAsync(ws->h_sizes, ws->scalars.ptr, 24u, hipMemcpyDeviceToHost, ws->stream));
         PGH_HIP(hipStreamSynchronize(ws->stream));
         if (ws->h_sizes[2]) return fail(PGH_DEVICE_ERROR, "fast_non_dominated_sorting: a grid barrier timed out");
-        // dom_items is written once its size is known
-        const uint64_t total = ws->h_sizes[1];
-        PGH_TRY(ws->dom_items.reserve(std::max<uint64_t>(total, 1u) * 8u));
-        k_emit<<<static_cast<uint32_t>((ws->n + 3u) / 4u), kBlock, 0, ws->stream>>>(
-            static_cast<const uint64_t *>(ws->D.ptr), static_cast<uint32_t>(ws->n), static_cast<uint32_t>(ws->words),
-            static_cast<const uint64_t *>(ws->dom_offsets.ptr), static_cast<uint64_t *>(ws->dom_items.ptr));
-        PGH_HIP(hipGetLastError());
         ws->sized = true;
+        ws->emitted = false;
     }
     if (n_fronts) *n_fronts = ws->h_sizes[0];
     if (n_dom_items) *n_dom_items = ws->h_sizes[1];
@@ -923,21 +961,42 @@ pgh_status pgh_fnds_copy(pgh_fnds_ws *ws, uint64_t *dom_count, uint64_t *rank, u
 try {
     uint64_t nfr = 0, ndi = 0;
     PGH_TRY(pgh_fnds_sizes(ws, &nfr, &ndi));
-    const hipMemcpyKind kind = to_host ? hipMemcpyDeviceToHost : hipMemcpyDeviceToDevice;
     const uint64_t n = ws->n;
-    struct item {
-        void *dst;
-        const void *src;
-        uint64_t count;
-    } items[] = {
-        {dom_count, ws->dom_count.ptr, n},       {rank, ws->rank.ptr, n},
-        {front_offsets, ws->front_offsets.ptr, nfr + 1u}, {front_items, ws->front_items.ptr, n},
-        {dom_offsets, ws->dom_offsets.ptr, n + 1u},       {dom_items, ws->dom_items.ptr, ndi},
+    const auto words = [](const pgh::ws_view &v) { return static_cast<const uint64_t *>(v.ptr); };
+    const out_range small[] = {
+        {dom_count, words(ws->dom_count), n},
+        {rank, words(ws->rank), n},
+        {front_offsets, words(ws->front_offsets), nfr + 1u},
+        {front_items, words(ws->front_items), n},
+        {dom_offsets, words(ws->dom_offsets), n + 1u},
     };
-    for (const auto &it : items) {
-        if (it.dst && it.count) {
-            PGH_HIP(hipMemcpyAsync(it.dst, it.src, it.count * 8u, kind, ws->stream));
+    bool direct = !to_host && writable_here(dom_items, ws->D.ptr);
+    for (const out_range &r : small) direct = direct && writable_here(r.dst, ws->D.ptr);
+    if (direct) {
+        // the caller's memory is this device's: the lists are emitted where they
+        // go and one launch copies the rest
+        out_ranges out{};
+        for (const out_range &r : small) {
+            if (r.dst) out.r[out.used++] = r;
         }
+        if (out.used) {
+            k_copy_out<<<dim3(grid_for(n + 1u), out.used), kBlock, 0, ws->stream>>>(out);
+            PGH_HIP(hipGetLastError());
+        }
+        if (dom_items && ndi) PGH_TRY(emit_items(ws, dom_items));
+        return PGH_OK;
+    }
+    const hipMemcpyKind kind = to_host ? hipMemcpyDeviceToHost : hipMemcpyDeviceToDevice;
+    for (const out_range &r : small) {
+        if (r.dst) PGH_HIP(hipMemcpyAsync(r.dst, r.src, r.count * 8u, kind, ws->stream));
+    }
+    if (dom_items && ndi) {
+        if (!ws->emitted) {
+            PGH_TRY(ws->dom_items.reserve(ndi * 8u));
+            PGH_TRY(emit_items(ws, static_cast<uint64_t *>(ws->dom_items.ptr)));
+            ws->emitted = true;
+        }
+        PGH_HIP(hipMemcpyAsync(dom_items, ws->dom_items.ptr, ndi * 8u, kind, ws->stream));
     }
     if (to_host) PGH_HIP(hipStreamSynchronize(ws->stream));
     return PGH_OK;

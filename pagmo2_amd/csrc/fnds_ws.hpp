@@ -83,6 +83,7 @@ struct pgh_fnds_ws {
     pgh::ws_view perm, skeys, scnt, srank, tiles, base, planes, rank32, fo32, wbase, any, members, masks, pos32;
     uint64_t h_sizes[3] = {0, 0, 0}; // n_fronts, n_dom_items, peel barrier timeout
     bool sized = false;
+    bool emitted = false; // dom_items holds the result's lists
     bool lists = false; // D, dom_offsets and dom_count hold this result's
     bool items = false; // front_items holds every front's
     // workgroups of the grid-wide front peel: 0 = the default rule, else the

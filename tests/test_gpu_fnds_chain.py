@@ -141,3 +141,30 @@ def test_crowding(n, m):
     ref = O.crowding_distance(pts, stable=True)
     assert np.array_equal(out.cpu().numpy(), ref, equal_nan=True)
     assert np.array_equal(P.crowding_distance_host(pts), ref, equal_nan=True)
+
+
+@pytest.mark.parametrize("n,m", [(2, 2), (65, 1), (700, 3), (16385, 2)])
+@pytest.mark.parametrize("shift", [0, 4])
+@pytest.mark.parametrize("only", [KEYS, ("dom_items",), ("rank", "front_offsets")])
+def test_copies_to_device(n, m, shift, only):
+    """pgh_fnds_copy into device memory (words in place, and an address that only a
+    copy can take), any subset of the outputs, twice, and to the host afterwards."""
+    objs = np.random.default_rng(n).uniform(0, 1, (n, m))
+    ws = P.Fnds()
+    ws.run(dev(objs))
+    n_fronts, n_dom = ws.sizes()
+    count = dict(dom_count=n, rank=n, front_offsets=n_fronts + 1, front_items=n, dom_offsets=n + 1, dom_items=n_dom)
+    for _ in range(2):
+        out = {k: torch.full((8 * count[k] + 16,), 255, dtype=torch.uint8, device="cuda:0") for k in only}
+        P.check(P.lib().pgh_fnds_copy(ws.h, *(out[k].data_ptr() + shift if k in out else None for k in KEYS), 0))
+        torch.cuda.synchronize()
+        ref = ws.to_host(n)
+        for k, t in out.items():
+            got = t.cpu().numpy()
+            assert np.array_equal(got[shift:shift + 8 * count[k]].view(np.uint64), ref[k]), k
+            assert (got[:shift] == 255).all() and (got[shift + 8 * count[k]:] == 255).all(), k
+    ws.close()
+    if n < 1000:
+        want = O.fnds(objs)
+        for k in KEYS:
+            assert np.array_equal(ref[k], want[k]), k
