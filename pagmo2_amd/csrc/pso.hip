@@ -1704,6 +1704,19 @@ pgh_status launch_step(const pgh_archi *a, uint32_t cls, const step_args &args, 
     return PGH_OK;
 }
 
+// Islands [i0, i1) are one island of one tile in a one-shot call: k_gens_one_tile
+// evolves it (the default variant and topology).
+bool one_tile_call(const pgh_archi *a, uint32_t i0, uint32_t i1)
+{
+    return a->one_shot && i1 == i0 + 1u && a->tile_begin[i1] - a->tile_begin[i0] == 1u &&
+           a->h_desc[i0].variant == 5u && a->h_desc[i0].topo == 2u;
+}
+
+// Bytes up to which arrays side by side are copied at once, through a host buffer:
+// a copy from or to pageable memory takes 25 us however small, as long as the
+// host's own copy of about this many.
+constexpr uint64_t kOneCopy = uint64_t(1) << 17;
+
 // k_gens_one_tile over the batch from generation g on of island i0 (tile t0).
 template <uint32_t CLASS>
 void launch_one_tile(pgh_archi *a, uint32_t grid, uint64_t stage_off, uint64_t stage_bytes, hipStream_t s, uint32_t i0,
@@ -1737,7 +1750,7 @@ pgh_status launch_range(pgh_archi *a, uint32_t i0, uint32_t i1, bool v_valid, bo
     const uint64_t e0 = a->h_desc[i0].eoff;
     const uint64_t e1 = i1 < a->h_desc.size() ? a->h_desc[i1].eoff : a->total_elems;
     const uint64_t total = e1 - e0;
-    const uint32_t t0 = a->tile_begin[i0], nt = a->tile_begin[i1] - t0;
+    const uint32_t t0 = a->tile_begin[i0];
     uint32_t gens = 0;
     for (uint32_t k = i0; k < i1; ++k) gens = std::max(gens, a->h_desc[k].gens);
     const uint32_t sg0 = a->h_desc[i0].seg0;
@@ -1759,8 +1772,7 @@ pgh_status launch_range(pgh_archi *a, uint32_t i0, uint32_t i1, bool v_valid, bo
     PGH_HIP(hipGetLastError());
     // a single island of one tile, evolved by the one-shot entry point: a
     // batch of generations per launch (k_gens_one_tile)
-    const bool fused = a->one_shot && i1 == i0 + 1u && nt == 1u && a->h_desc[i0].variant == 5u &&
-                       a->h_desc[i0].topo == 2u;
+    const bool fused = one_tile_call(a, i0, i1);
     // the gbest islands of the range: the swarm's best at the call's start
     const auto gb_lo = std::lower_bound(a->h_gb.begin(), a->h_gb.end(), i0);
     const auto gb_hi = std::lower_bound(a->h_gb.begin(), a->h_gb.end(), i1);
@@ -1919,7 +1931,7 @@ uint32_t von_cols(uint32_t pop)
 // Initial populations from host arrays (X0, F0) or, with `seeds`, drawn and
 // evaluated on the device.
 pgh_status archi_create(pgh_archi **out, const pgh_island_spec *islands, uint64_t n_islands,
-                        const double *const *X0, const double *const *F0, const uint32_t *seeds)
+                        const double *const *X0, const double *const *F0, const uint32_t *seeds, bool one_shot)
 {
     if (!out || !islands || (!seeds && (!X0 || !F0))) return fail(PGH_INVALID_ARGUMENT, "null argument");
     if (n_islands == 0u) return fail(PGH_INVALID_ARGUMENT, "an archipelago needs at least one island");
@@ -2155,11 +2167,12 @@ pgh_status archi_create(pgh_archi **out, const pgh_island_spec *islands, uint64_
     place(a->states, n_islands * sizeof(mt_state));
     place(a->gblist, a->h_gb.size() * sizeof(uint32_t));
     const uint64_t head_bytes = arena_bytes;
-    place(a->X, xoff * 8u);
-    place(a->V, xoff * 8u);
-    place(a->lbX, xoff * 8u);
+    place(a->X, xoff * 8u); // X beside fit and lbX beside lbfit: small ones go up and down in one copy
     place(a->fit, foff * 8u);
+    const uint64_t up_bytes = arena_bytes;
+    place(a->lbX, xoff * 8u);
     place(a->lbfit, foff * 8u);
+    place(a->V, xoff * 8u);
     place(a->gbest, gboff * 8u);
     place(a->words, std::max<uint64_t>(woff, 1u) * 4u);
     place(a->seg_states, seg_list.size() * sizeof(mt_state));
@@ -2175,9 +2188,14 @@ pgh_status archi_create(pgh_archi **out, const pgh_island_spec *islands, uint64_
                           &a->selA, &a->selB, &a->vsegs, &a->states_q}) {
         v->ptr = base + v->off;
     }
-    PGH_TRY(build_items(a.get()));
+    a->one_shot = one_shot;
+    if (!one_tile_call(a.get(), 0u, static_cast<uint32_t>(n_islands))) PGH_TRY(build_items(a.get()));
+    // a small population goes up with the tables (a copy of its own takes 25 us
+    // whatever its size; 10 KB with the tables: one copy for four)
+    bool together = !seeds && up_bytes <= kOneCopy;
+    for (uint64_t k = 0; together && k < n_islands; ++k) together = X0[k] && F0[k];
     {
-        std::vector<uint8_t> head(head_bytes, 0u);
+        std::vector<uint8_t> head(together ? up_bytes : head_bytes, 0u);
         auto put = [&](const arena_view &v, const void *src, uint64_t bytes) {
             if (bytes) std::memcpy(head.data() + v.off, src, bytes);
         };
@@ -2188,9 +2206,14 @@ pgh_status archi_create(pgh_archi **out, const pgh_island_spec *islands, uint64_
         put(a->jump_table, tab.data(), tab.size());
         put(a->states, states.data(), n_islands * sizeof(mt_state));
         put(a->gblist, a->h_gb.data(), a->h_gb.size() * sizeof(uint32_t));
-        PGH_HIP(hipMemcpy(base, head.data(), head_bytes, hipMemcpyHostToDevice));
+        for (uint64_t k = 0; together && k < n_islands; ++k) {
+            const island_desc &di = a->h_desc[k];
+            std::memcpy(head.data() + a->X.off + di.xoff * 8u, X0[k], static_cast<uint64_t>(di.pop) * di.nx * 8u);
+            std::memcpy(head.data() + a->fit.off + di.foff * 8u, F0[k], static_cast<uint64_t>(di.pop) * 8u);
+        }
+        PGH_HIP(hipMemcpy(base, head.data(), head.size(), hipMemcpyHostToDevice));
     }
-    for (uint64_t k = 0; k < n_islands; ++k) {
+    for (uint64_t k = 0; !together && k < n_islands; ++k) {
         const island_desc &di = a->h_desc[k];
         double *Xk = static_cast<double *>(a->X.ptr) + di.xoff;
         double *Fk = static_cast<double *>(a->fit.ptr) + di.foff;
@@ -2216,7 +2239,7 @@ extern "C" {
 pgh_status pgh_archi_create(pgh_archi **out, const pgh_island_spec *islands, uint64_t n_islands,
                             const double *const *X0, const double *const *F0)
 try {
-    return archi_create(out, islands, n_islands, X0, F0, nullptr);
+    return archi_create(out, islands, n_islands, X0, F0, nullptr, false);
 } catch (...) {
     return api_exception();
 }
@@ -2225,7 +2248,7 @@ pgh_status pgh_archi_create_seeded(pgh_archi **out, const pgh_island_spec *islan
                                    const uint32_t *pop_seeds)
 try {
     if (!pop_seeds) return fail(PGH_INVALID_ARGUMENT, "null argument");
-    return archi_create(out, islands, n_islands, nullptr, nullptr, pop_seeds);
+    return archi_create(out, islands, n_islands, nullptr, nullptr, pop_seeds, false);
 } catch (...) {
     return api_exception();
 }
@@ -2502,6 +2525,14 @@ try {
     // pop.set_xf(i, lbX[i], lbfit[i]), pso_gen.cpp:526-528
     const double *xs = static_cast<const double *>(a->evolved ? a->lbX.ptr : a->X.ptr);
     const double *fs = static_cast<const double *>(a->evolved ? a->lbfit.ptr : a->fit.ptr);
+    const uint64_t span = static_cast<uint64_t>(fs + di.foff + di.pop - (xs + di.xoff)) * 8u; // fs lies after xs
+    if (X && F && span <= kOneCopy) {
+        std::vector<uint8_t> both(span);
+        PGH_HIP(hipMemcpy(both.data(), xs + di.xoff, span, hipMemcpyDeviceToHost));
+        std::memcpy(X, both.data(), static_cast<uint64_t>(di.pop) * di.nx * 8u);
+        std::memcpy(F, both.data() + span - static_cast<uint64_t>(di.pop) * 8u, static_cast<uint64_t>(di.pop) * 8u);
+        return PGH_OK;
+    }
     if (X) {
         PGH_HIP(hipMemcpy(X, xs + di.xoff, static_cast<uint64_t>(di.pop) * di.nx * 8u, hipMemcpyDeviceToHost));
     }
@@ -2540,12 +2571,11 @@ try {
     pgh_archi *a = nullptr;
     const double *xs[1] = {X};
     const double *fs[1] = {F};
-    PGH_TRY(pgh_archi_create(&a, &sp, 1u, xs, fs));
+    PGH_TRY(archi_create(&a, &sp, 1u, xs, fs, nullptr, true));
     std::unique_ptr<pgh_archi> guard(a);
     // one island, evolved once: direct launches (capturing and instantiating
     // a graph that runs once costs more than it saves), a batch of
     // generations per launch when the island is one evaluation tile
-    a->one_shot = true;
     PGH_TRY(pgh_archi_evolve(a, PGH_ARCHI_PER_ISLAND, nullptr));
     return pgh_archi_get(a, 0u, X, F);
 } catch (...) {

@@ -89,3 +89,24 @@ def test_one_shot_tiles(kind, dim, pop, param):
     if kind == P.ROSENBROCK:
         Xo, Fo = O.pso_gen_evolve(kind, dim, X0, F0, 35, 21, neighb_param=param)
         assert np.array_equal(Xh, Xo) and np.array_equal(Fh, Fo)
+
+
+@pytest.mark.parametrize("pop", [5, 1800, 1819, 1820, 1821, 2048, 2100])
+@pytest.mark.parametrize("islands", [1, 2])
+def test_populations_in_and_out(pop, islands):
+    """Populations on both sides of 128 KiB (8 elements and a fitness a row) arrive
+    and come back unchanged before an evolve call and as the oracle's after one."""
+    isl = []
+    for k in range(islands):
+        X0, F0 = O.population_init(P.ROSENBROCK, 8, pop, 3 + k)
+        isl.append(dict(kind=P.ROSENBROCK, dim=8, X0=X0, F0=F0, algo=P.pso_params(gen=2, seed=9)))
+    a = P.Archipelago(isl)
+    for k, d in enumerate(isl):
+        X, F = a.get(k)
+        assert np.array_equal(X, d["X0"]) and np.array_equal(F, np.ravel(d["F0"]))
+    a.evolve()
+    for k, d in enumerate(isl):
+        X, F = a.get(k)
+        Xo, Fo = O.pso_gen_evolve(P.ROSENBROCK, 8, d["X0"], d["F0"], 2, 9)
+        assert np.array_equal(X, Xo) and np.array_equal(F, np.ravel(Fo))
+    a.close()
