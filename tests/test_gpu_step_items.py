@@ -77,6 +77,7 @@ def test_fitness_of_the_final_positions(variant, topo, mapping):
     (P.ROSENBROCK, 17, 256, 4),   # not held
     (P.RASTRIGIN, 1, 16, 2), (P.GRIEWANK, 65, 4, 2), (P.SCHWEFEL, 33, 16, 4), (P.ACKLEY, 300, 5, 4),
     (P.LENNARD_JONES, 3, 9, 4), (P.LENNARD_JONES, 75, 4, 2),
+    (P.ACKLEY, 1200, 4, 2), (P.RASTRIGIN, 5001, 3, 2), (P.LENNARD_JONES, 300, 4, 2),  # not held
 ])
 def test_one_shot_tiles(kind, dim, pop, param):
     """pgh_pso_gen_evolve_host of a single tile equals the archipelago's launches bit
