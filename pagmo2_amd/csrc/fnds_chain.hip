@@ -770,7 +770,10 @@ __global__ __launch_bounds__(kWide) void k_chain(const uint32_t *__restrict__ fo
     // a run's words, or a large front's slots by bin (max(2 P, 8 kStage) bytes)
     uint64_t *stage = reinterpret_cast<uint64_t *>(F + P + 64u);
     uint16_t *list = reinterpret_cast<uint16_t *>(stage);
-    __shared__ uint32_t fs[kWide + 2u], s_run, s_scan[kWide / 64u];
+    // s_words, a run's words, is stored by wavefront 0 alone, before the barrier that
+    // ends a run; its next store lies behind the barriers of the next run, so every
+    // wavefront has read it.  (s_run, which a next front stores at once, would not do.)
+    __shared__ uint32_t fs[kWide + 2u], s_run, s_words, s_scan[kWide / 64u];
     __shared__ __align__(16) uint64_t vplanes[kWaves * kPlanes];
     __shared__ uint32_t s_v[kWide], s_pos[kWide]; // zero between fronts
     const uint32_t t = threadIdx.x, lane = t & 63u, wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -914,13 +917,13 @@ __global__ __launch_bounds__(kWide) void k_chain(const uint32_t *__restrict__ fo
                         planes[b] = b < 7u ? p0[b] : 0u;
                         if (prev > 64u) planes[kPlanes + b] = b < 7u ? p1[b] : 0u;
                     }
-                    s_run = off;
+                    s_words = off;
                 }
             }
             L += run;
             load = L >= L0 + kWide;
             __syncthreads();
-            wb += s_run; // the run's words
+            wb += s_words;
             continue;
         }
         if (fl[2] - fl[1] <= kWide) {
