@@ -83,8 +83,10 @@ __device__ __forceinline__ double mt_canonical(uint32_t u0, uint32_t u1)
 
 // uniform_real_distribution<double>(a, b): canonical * (b - a) + a
 // (bits/random.h, operator()), multiply and add rounded separately.  w is
-// mt_width(a, b): the scaling by 2^-64 is exact on either factor (a sum is 0 or
-// at least 1, and |b - a| is far above 2^-958), so the product rounds alike.
+// mt_width(a, b): for |b - a| above 2^-958 the scaling by 2^-64 is exact on
+// either factor (a sum is 0 or at least 1), so the product rounds alike.  For a
+// problem's bounds, which are units apart or more; an island's velocity limits
+// can lie at any value and scale the sum (pso.hip, velocity_sink).
 __host__ __device__ __forceinline__ double mt_width(double a, double b)
 {
     return (b - a) * 0x1p-64;

@@ -162,7 +162,9 @@ __device__ __forceinline__ uint64_t velocity_words(const island_desc &di, uint32
     return (di.memory && v_valid) ? 0u : 2ull * di.pop * di.nx;
 }
 
-// Words handed out become velocities, U(minv, maxv) (pso_gen.cpp:177-200).
+// Words handed out become velocities, U(minv, maxv) (pso_gen.cpp:177-200).  max_vel
+// may be any value in (0, 1]: the width stays unscaled (mt_width would round it
+// below 2^-958).
 struct velocity_sink {
     double *V;   // the island's
     uint64_t m0; // element of the hand-out's first word
@@ -175,7 +177,7 @@ struct velocity_sink {
         bounds_of(kind, j, lb, ub);
         const double vwidth = (ub - lb) * max_vel;
         lo = -1. * vwidth;
-        width = mt_width(lo, vwidth);
+        width = vwidth - lo;
     }
     __device__ __forceinline__ velocity_sink(double *V_, uint64_t m0_, const island_desc &di)
         : V(V_), m0(m0_), nx(di.nx), kind(di.kind), max_vel(di.max_vel)
@@ -193,7 +195,7 @@ struct velocity_sink {
             const uint2 v = reinterpret_cast<const uint2 *>(words)[i];
             double a = minv, wi = w;
             if (cols) range((c0 + i) % nx, a, wi);
-            V[m + i] = mt_uniform(mt_temper(v.x), mt_temper(v.y), a, wi);
+            V[m + i] = mt_canonical(mt_temper(v.x), mt_temper(v.y)) * wi + a;
         }
     }
 };
