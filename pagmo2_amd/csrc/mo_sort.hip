@@ -135,6 +135,11 @@ __global__ __launch_bounds__(kBlock) void k_widen(const uint32_t *__restrict__ v
 // What one workgroup holds: 64-bit keys, 32-bit positions, two orders of
 // 16-bit slots and the distances, 24 bytes a member.
 constexpr uint32_t kFrontMax = 4096, kFrontBlock = 512;
+// crowding_distance of one front alone: the workgroup's sort doubles its cost with
+// every power of two, the radix sorts cost much the same up to there.  Two and ten
+// objectives: 1024 points 52 and 185 us against 64 and 222, 2048 points 82 and 335
+// against 84 and 312, 4096 points 147 and 658 against 83 and 322.
+constexpr uint32_t kCrowdMax = 1024;
 enum front_out : int {
     kFrontsSorted,  // out: every front's elements, (crowding descending, index)
     kFrontPart,     // out: whole fronts while they fit N, then the next by (crowding descending, position)
@@ -459,7 +464,7 @@ try {
     if (!points || !out) return fail(PGH_INVALID_ARGUMENT, "null buffer");
     if (n >= (uint64_t(1) << 31) || m > 512u) return fail(PGH_UNSUPPORTED, "crowding_distance: front too large");
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (n <= kFrontMax) {
+    if (n <= kCrowdMax) {
         PGH_TRY(launch_front_order<kFrontDistances>(ws, points, n, m, 0u, out, 1u, s));
         PGH_HIP(hipStreamSynchronize(s));
         return PGH_OK;
