@@ -23,8 +23,9 @@
 // final order, in one launch for all fronts (sort_population_mo), for the one
 // front that is taken in part (select_best_N_mo) or for the points given
 // (crowding_distance).  At 200 x 2 the 20 launches of the radix sorts took 0.1 ms
-// of a call, at 16384 x 3 28 launches 0.2 ms.  A larger front sets a flag that
-// the call reads with its other results, and takes the radix sorts.
+// of a call, at 16384 x 3 28 launches 0.2 ms.  Where a front to be sorted is larger
+// the kernel does nothing but set a flag, which the call reads with its other
+// results, and the radix sorts do all.
 #include <hip/hip_runtime.h>
 #include <rocprim/device/device_radix_sort.hpp>
 
@@ -238,6 +239,24 @@ __global__ __launch_bounds__(kFrontBlock) void k_front_order(const double *__res
         if (scalars[2]) return; // the peel gave up: no fronts
         const uint32_t fronts = static_cast<uint32_t>(min(scalars[0], static_cast<uint64_t>(n)));
         uint32_t f = blockIdx.x;
+        if (f >= fronts) return;
+        if constexpr (OUT == kFrontsSorted) {
+            // with a front beyond cap the call sorts all of them another way, and
+            // every workgroup's share here would be for nothing
+            if (n > cap) {
+                __shared__ uint32_t s_large;
+                if (threadIdx.x == 0) s_large = 0u;
+                __syncthreads();
+                bool large = false;
+                for (uint32_t q = threadIdx.x; q < fronts; q += kFrontBlock) large |= offsets[q + 1u] - offsets[q] > cap;
+                if (large) s_large = 1u;
+                __syncthreads();
+                if (s_large) { // uniform
+                    if (f == 0u && threadIdx.x == 0) scalars[3] = 1u;
+                    return;
+                }
+            }
+        }
         if constexpr (OUT == kFrontPart) {
             // the first front that does not fit whole: offsets[f] <= N < offsets[f + 1]
             uint32_t hi = fronts;
@@ -247,15 +266,15 @@ __global__ __launch_bounds__(kFrontBlock) void k_front_order(const double *__res
                 if (offsets[mid] <= N) f = mid;
                 else hi = mid;
             }
+            if (offsets[f] < N && offsets[f + 1u] - offsets[f] > cap) { // uniform: sorted another way
+                if (threadIdx.x == 0) scalars[3] = 1u;
+                return;
+            }
             for (uint64_t x = threadIdx.x; x < offsets[f]; x += kFrontBlock) o[x] = items[x];
             if (offsets[f] == N) return;
         }
         for (; f < fronts; f += gridDim.x) {
-            const uint32_t a = static_cast<uint32_t>(offsets[f]), c = static_cast<uint32_t>(offsets[f + 1u]) - a;
-            if (c > cap) { // uniform
-                if (threadIdx.x == 0) scalars[3] = 1u;
-                return;
-            }
+            const uint32_t a = static_cast<uint32_t>(offsets[f]), c = static_cast<uint32_t>(offsets[f + 1u]) - a; // <= cap
             const uint32_t P = pow2(c);
             const uint64_t *e = items + a;
             front_crowding(objs, m, c, P, K, V, ord, C, [e](uint32_t x) { return static_cast<uint32_t>(e[x]); });
