@@ -1,5 +1,5 @@
 """sort_population_mo and select_best_N_mo where one front is larger than a workgroup
-sorts (4096 members) beside others that are not, in every position, and where none
+sorts (4096 members, 2048 of at most 4096 points) beside others that are not, in every position, and where none
 is although the points are many.  Bit for bit with the oracle."""
 import numpy as np
 import pytest
@@ -30,14 +30,15 @@ def check(objs, Ns):
     out = torch.empty(n, dtype=torch.int64, device="cuda:0")
     ws.sort_population_mo(d, out)
     assert np.array_equal(out.cpu().numpy().astype(np.uint64), O.sort_population_mo(objs, stable=True))
-    for N in Ns:
+    for N in (N for N in Ns if N < n):
         got = torch.empty(N, dtype=torch.int64, device="cuda:0")
         assert ws.select_best_N_mo(d, N, got) == N
         assert np.array_equal(got.cpu().numpy().astype(np.uint64), O.select_best_N_mo(objs, N, stable=True)), N
     ws.close()
 
 
-@pytest.mark.parametrize("sizes", [(4097, 20), (20, 4097), (300, 4200, 700), (4096, 4096), (700, 700, 4096), (1, 4097)])
+@pytest.mark.parametrize("sizes", [(4097, 20), (20, 4097), (300, 4200, 700), (4096, 4096), (700, 700, 4096), (1, 4097),
+                                   (2048, 2048), (2049, 2047), (30, 2049), (2048, 2049), (1, 4095), (2049,)])
 def test_layers(sizes):
     ends = np.cumsum(sizes)
     check(layers(sizes, len(sizes)), sorted({1, *(int(e) for e in ends[:-1]), *(int(e) - 1 for e in ends),
