@@ -266,6 +266,7 @@ inline const field &the_field()
 struct poly_cache {
     std::mutex mu;
     std::map<uint64_t, poly> map; // references stay valid as entries are added
+    std::map<uint64_t, uint64_t> runs; // S -> c: z^S, z^(2 S), ..., z^(c S) are all in map
 };
 
 inline poly_cache &the_cache()
@@ -326,18 +327,20 @@ inline void prefetch_multiples(uint64_t S, uint64_t count)
 {
     if (count == 0u || S == 0u) return;
     poly_cache &c = the_cache();
-    const auto known = [&](uint64_t k) {
-        std::lock_guard<std::mutex> lk(c.mu);
-        return c.map.count(k * S) != 0u;
-    };
-    // made by an earlier call (the multiples come in order, the last one is
-    // entered with the rest)
-    if (known(count)) return;
     const field &f = the_field();
     std::vector<poly> res(count + 1u); // res[k]: z^(k S)
-    res[1] = jump_poly(S);
+    uint64_t have = 0u;
+    {
+        // (count S alone says nothing: it may be there as a multiple of another distance)
+        std::lock_guard<std::mutex> lk(c.mu);
+        const auto run = c.runs.find(S);
+        if (run != c.runs.end()) have = run->second;
+        if (have >= count) return;
+        for (uint64_t k = 1; k <= have; ++k) res[k] = c.map.at(k * S);
+    }
+    if (have == 0u) res[1] = jump_poly(S);
     const unsigned threads = std::min(8u, std::max(1u, std::thread::hardware_concurrency()));
-    for (uint64_t m = 1; m < count;) {
+    for (uint64_t m = std::max<uint64_t>(have, 1u); m < count;) {
         const uint64_t n = std::min(m, count - m);
         std::atomic<uint64_t> next{1};
         const auto work = [&] {
@@ -358,7 +361,9 @@ inline void prefetch_multiples(uint64_t S, uint64_t count)
         m += n;
     }
     std::lock_guard<std::mutex> lk(c.mu);
-    for (uint64_t k = 2; k <= count; ++k) c.map.emplace(k * S, std::move(res[k]));
+    for (uint64_t k = have + 1u; k <= count; ++k) c.map.emplace(k * S, std::move(res[k]));
+    uint64_t &run = c.runs[S];
+    run = std::max(run, count);
 }
 
 } // namespace mtj
