@@ -40,19 +40,20 @@ pgh_status jump_polys_multiples(uint64_t S, uint64_t count)
 
 namespace
 {
-// A device copy of the bytes, on a stream of its own: callers may be capturing
-// another stream, on this thread or on others.
-pgh_status upload_table(const std::vector<uint8_t> &h, void **out)
+// A device copy of the bytes, by the stream or, without one, by a stream of its own
+// (a process's first stream takes 3 ms).
+pgh_status upload_table(const std::vector<uint8_t> &h, const hipStream_t *on, void **out)
 {
     void *ptr = nullptr;
-    hipStream_t s = nullptr;
+    hipStream_t s = on ? *on : nullptr;
     PGH_HIP(hipMalloc(&ptr, h.size()));
-    pgh_status st = hip_status(hipStreamCreateWithFlags(&s, hipStreamNonBlocking), "hipStreamCreateWithFlags");
+    pgh_status st = PGH_OK;
+    if (!on) st = hip_status(hipStreamCreateWithFlags(&s, hipStreamNonBlocking), "hipStreamCreateWithFlags");
     if (st == PGH_OK) {
         st = hip_status(hipMemcpyAsync(ptr, h.data(), h.size(), hipMemcpyHostToDevice, s), "hipMemcpyAsync");
         const pgh_status w = hip_status(hipStreamSynchronize(s), "hipStreamSynchronize");
         if (st == PGH_OK) st = w;
-        (void)hipStreamDestroy(s);
+        if (!on) (void)hipStreamDestroy(s);
     }
     if (st != PGH_OK) {
         (void)hipFree(ptr);
@@ -61,20 +62,35 @@ pgh_status upload_table(const std::vector<uint8_t> &h, void **out)
     *out = ptr;
     return PGH_OK;
 }
+
+// The tables of the process, kept for its life.
+struct table_entry {
+    void *table = nullptr;
+    uint64_t spent = 0u; // words of the calls that did without
+};
+std::mutex tables_mu;
+std::map<std::tuple<int, uint64_t, uint32_t>, table_entry> tables; // by device, S, count
 } // namespace
 
-pgh_status jump_table_device(uint64_t S, uint32_t count, bool make, const uint32_t **out)
+pgh_status jump_table_find(uint64_t S, uint32_t count, const uint32_t **out)
 {
-    static std::mutex mu;
-    static std::map<std::tuple<int, uint64_t, uint32_t>, void *> cache;
+    int dev = 0;
+    PGH_HIP(hipGetDevice(&dev));
+    std::lock_guard<std::mutex> lk(tables_mu);
+    const auto it = tables.find(std::make_tuple(dev, S, count));
+    *out = it == tables.end() ? nullptr : static_cast<const uint32_t *>(it->second.table);
+    return PGH_OK;
+}
+
+pgh_status jump_table_make(uint64_t S, uint32_t count, uint64_t words, const hipStream_t *on, const uint32_t **out)
+{
     *out = nullptr;
     int dev = 0;
     PGH_HIP(hipGetDevice(&dev));
-    std::lock_guard<std::mutex> lk(mu);
-    const auto key = std::make_tuple(dev, S, count);
-    auto it = cache.find(key);
-    if (it == cache.end()) {
-        if (!make) return PGH_OK;
+    std::lock_guard<std::mutex> lk(tables_mu);
+    table_entry &e = tables[std::make_tuple(dev, S, count)];
+    if (!e.table) {
+        if (mtj::without_table(e.spent, words)) return PGH_OK;
         PGH_TRY(jump_polys_multiples(S, count));
         std::vector<uint64_t> dists;
         for (uint64_t k = 1; k <= count; ++k) dists.push_back(k * S);
@@ -82,13 +98,11 @@ pgh_status jump_table_device(uint64_t S, uint32_t count, bool make, const uint32
         PGH_TRY(jump_table_bytes(dists, h));
         hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
         PGH_HIP(hipThreadExchangeStreamCaptureMode(&mode));
-        void *ptr = nullptr;
-        const pgh_status st = upload_table(h, &ptr);
+        const pgh_status st = upload_table(h, on, &e.table);
         (void)hipThreadExchangeStreamCaptureMode(&mode);
         PGH_TRY(st);
-        it = cache.emplace(key, ptr).first;
     }
-    *out = static_cast<const uint32_t *>(it->second);
+    *out = static_cast<const uint32_t *>(e.table);
     return PGH_OK;
 }
 

@@ -16,10 +16,11 @@
 // Polynomials over GF(2) are bit vectors (bit i = coefficient of z^i), 312
 // 64-bit words below degree 19937.  Products use carry-less multiplication
 // (PCLMULQDQ when the CPU has it, a shift-and-add loop otherwise).  A product
-// of degree < 2 x 19968 is reduced through a table of z^(64 w) mod phi for the
-// words w >= 312 it has: each such word c contributes c * (z^(64 w) mod phi),
-// so the reduction is 312 x 312 independent word products; the bits 19937 ..
-// 19967 left over are reduced one by one.
+// is reduced from its highest words down by phi itself, which has 134 terms
+// below z^19937, the highest of them 623 below: nine words at a time, XORed in
+// at 134 places.  (Through a table of z^(64 w) mod phi, a carry-less product per
+// word of the table's 312 x 312, a multiplication took 155 us; so it takes 100,
+// and one by a power of z below the degree 20.)
 #pragma once
 
 #include <algorithm>
@@ -151,14 +152,10 @@ class field
         for (uint32_t i = 0; i < 31u; ++i) times(623u, 396u, (a >> i) & 1u);
         times(624u, 397u, (a >> 31) & 1u);
         if (!bit(phi, kDeg) || bits64(phi, kDeg + 1u)) return;
-        // tab[w - kWords] = z^(64 w) mod phi, w = kWords .. 2 kWords - 1
-        poly t = shift_reduce_bits(unit_at(64u * kWords));
-        tab.push_back(t);
-        for (uint32_t w = kWords + 1u; w < 2u * kWords; ++w) {
-            t = times_z64(t);
-            tab.push_back(t);
+        for (uint32_t e = 0; e < kDeg; ++e) {
+            if (bit(phi, e)) low.push_back(e);
         }
-        ok = true;
+        ok = low.back() + 64u * kRun <= kDeg; // reduce() folds onto lower words only
     }
 
     // a * b mod phi (a, b reduced)
@@ -168,7 +165,7 @@ class field
         for (uint32_t j = 0; j < kWords; ++j) {
             if (b[j]) mul_word_acc(a.data(), kWords, b[j], prod.data() + j);
         }
-        return reduce(prod);
+        return reduce(std::move(prod));
     }
 
     poly sqr(const poly &a) const
@@ -193,42 +190,23 @@ class field
     }
 
   private:
-    std::vector<poly> tab;
+    static constexpr uint32_t kRun = 9u; // words folded at a time
+    std::vector<uint32_t> low;           // phi's exponents below kDeg, ascending
 
-    static poly unit_at(uint64_t i)
+    // r ^= v z^at (z^kDeg mod phi), v of N words
+    template <uint32_t N>
+    void fold(uint64_t *__restrict__ r, const uint64_t *__restrict__ v, uint64_t at) const
     {
-        poly r(i / 64u + 1u, 0u);
-        r[i / 64u] = uint64_t(1) << (i & 63u);
-        return r;
-    }
-
-    // XOR of phi << s into r at bit position `at` (phi's leading bit lands on at + kDeg)
-    void add_phi_at(poly &r, uint64_t at) const
-    {
-        const uint64_t ws = at >> 6, bs = at & 63u;
-        for (uint64_t w = 0; w <= kWords; ++w) {
-            const uint64_t lo = phi[w] << bs;
-            const uint64_t hi = bs ? (phi[w] >> (64u - bs)) : 0u;
-            if (ws + w < r.size()) r[ws + w] ^= lo;
-            if (bs && ws + w + 1u < r.size()) r[ws + w + 1u] ^= hi;
+        for (const uint32_t e : low) {
+            uint64_t *__restrict__ o = r + ((at + e) >> 6);
+            const uint32_t b = (at + e) & 63u;
+            uint64_t t[N + 1u];
+            t[0] = v[0] << b;
+            // (two shifts: by 64 - b, also for b = 0)
+            for (uint32_t i = 1; i < N; ++i) t[i] = (v[i] << b) | ((v[i - 1u] >> 1) >> (63u - b));
+            t[N] = (v[N - 1u] >> 1) >> (63u - b);
+            for (uint32_t i = 0; i <= N; ++i) o[i] ^= t[i]; // (at + e lies over 600 below the words taken)
         }
-    }
-
-    // bit-by-bit reduction (used for the table and the last 31 bits)
-    poly shift_reduce_bits(poly r) const
-    {
-        for (uint64_t k = static_cast<uint64_t>(r.size()) * 64u; k-- > kDeg;) {
-            if (bit(r, k)) add_phi_at(r, k - kDeg);
-        }
-        r.resize(kWords);
-        return r;
-    }
-
-    poly times_z64(const poly &a) const
-    {
-        poly r(kWords + 1u, 0u);
-        for (uint32_t w = 0; w < kWords; ++w) r[w + 1u] = a[w];
-        return shift_reduce_bits(r);
     }
 
     poly times_z(const poly &a) const
@@ -240,20 +218,32 @@ class field
             carry = a[w] >> 63;
         }
         r[kWords] = carry;
-        return shift_reduce_bits(r);
+        return reduce(std::move(r));
     }
 
-    // prod has up to 2 kWords + 1 words: words w >= kWords fold through the
-    // table (word 2 kWords is zero for products of reduced operands: their
-    // degree is below 2 x 19937 - 1 < 64 x 2 kWords)
-    poly reduce(const poly &prod) const
+    // r mod phi, r of any length from kWords words on
+    poly reduce(poly r) const
     {
-        poly r(kWords + 1u, 0u);
-        for (uint32_t w = 0; w < kWords; ++w) r[w] = prod[w];
-        for (uint32_t w = kWords; w < 2u * kWords; ++w) {
-            if (prod[w]) mul_word_acc(tab[w - kWords].data(), kWords, prod[w], r.data());
+        uint64_t top = r.size();
+        for (; top >= kWords + kRun; top -= kRun) fold_top<kRun>(r, top);
+        for (; top > kWords; --top) fold_top<1u>(r, top);
+        // the last word's bits from kDeg on
+        const uint64_t v = r[kWords - 1u] >> (kDeg & 63u);
+        r[kWords - 1u] &= (uint64_t(1) << (kDeg & 63u)) - 1u;
+        fold<1u>(r.data(), &v, 0u);
+        r.resize(kWords);
+        return r;
+    }
+    template <uint32_t N>
+    void fold_top(poly &r, uint64_t top) const
+    {
+        uint64_t v[N], some = 0u;
+        for (uint32_t i = 0; i < N; ++i) {
+            v[i] = r[top - N + i];
+            r[top - N + i] = 0u;
+            some |= v[i];
         }
-        return shift_reduce_bits(r);
+        if (some) fold<N>(r.data(), v, 64u * (top - N) - kDeg);
     }
 };
 
@@ -339,8 +329,12 @@ inline void prefetch_multiples(uint64_t S, uint64_t count)
         for (uint64_t k = 1; k <= have; ++k) res[k] = c.map.at(k * S);
     }
     if (have == 0u) res[1] = jump_poly(S);
+    uint64_t known = std::max<uint64_t>(have, 1u);
+    // z^S is one term below the degree: its products are cheap, and the first few are
+    // sooner made one after another than by threads
+    for (; S < kDeg && known < std::min<uint64_t>(count, 32u); ++known) res[known + 1u] = f.mul(res[known], res[1]);
     const unsigned threads = std::min(8u, std::max(1u, std::thread::hardware_concurrency()));
-    for (uint64_t m = std::max<uint64_t>(have, 1u); m < count;) {
+    for (uint64_t m = known; m < count;) {
         const uint64_t n = std::min(m, count - m);
         std::atomic<uint64_t> next{1};
         const auto work = [&] {
@@ -364,6 +358,23 @@ inline void prefetch_multiples(uint64_t S, uint64_t count)
     for (uint64_t k = have + 1u; k <= count; ++k) c.map.emplace(k * S, std::move(res[k]));
     uint64_t &run = c.runs[S];
     run = std::max(run, count);
+}
+
+// ---- when a device table of multiples is worth making ----------------------------
+// Making one costs a process 1 to 3 ms once (31 to 127 multiples, an allocation and
+// an upload), as long as one workgroup takes for 2^21 to 2^23 words.  So calls of up
+// to kRentWords words do without, as one segment, until those of the table's size
+// class have come to that many words between them: a program that draws one
+// population never pays for the table, one that draws many soon has it.
+constexpr uint64_t kRentWords = uint64_t(1) << 21;
+
+// A call of `words` words finds no table, and those before it made `spent`: true if
+// it does without, which is entered.
+inline bool without_table(uint64_t &spent, uint64_t words)
+{
+    if (words > kRentWords || spent + words > kRentWords) return false;
+    spent += words;
+    return true;
 }
 
 } // namespace mtj

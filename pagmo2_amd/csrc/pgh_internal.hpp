@@ -83,10 +83,13 @@ pgh_status launch_batch_random_dv(const prob &p, uint64_t n, uint32_t seed, doub
 // ---- std::mt19937 jump-ahead (mt_jump.hip) ------------------------------------
 // Bytes of one polynomial of a table (layout: mt_dev.hpp, mt_jump).
 constexpr size_t kJumpPolyBytes = 624u * 4u;
-// Device table of z^(k S) mod phi for k = 1 .. count; made on first use per
-// device, S and count, and kept.  Synchronous the first time; with make false
-// a table that does not exist yet gives a null pointer instead.
-pgh_status jump_table_device(uint64_t S, uint32_t count, bool make, const uint32_t **out);
+// Device table of z^(k S) mod phi for k = 1 .. count, kept per device, S and count:
+// the one there is, or null.
+pgh_status jump_table_find(uint64_t S, uint32_t count, const uint32_t **out);
+// ... made if there is none, for a call of `words` words, unless that does without
+// (mt_jump_host.hpp, without_table; null).  Synchronous when it makes one; `on`: a
+// stream to copy on that is not being captured, or null.
+pgh_status jump_table_make(uint64_t S, uint32_t count, uint64_t words, const hipStream_t *on, const uint32_t **out);
 // The polynomials of the distances as bytes, for a caller that keeps its own
 // device copy.
 pgh_status jump_table_bytes(const std::vector<uint64_t> &dists, std::vector<uint8_t> &out);

@@ -2,6 +2,7 @@
 // batch_random_decision_vector (include/pagmo/utils/generic.hpp:326-388).
 #include "fitness_dev.hpp"
 #include "mt_dev.hpp"
+#include "mt_jump_host.hpp"
 #include "pgh_internal.hpp"
 
 #include <vector>
@@ -92,8 +93,12 @@ __global__ __launch_bounds__(kMtBlock) void k_mt19937(mt_state st, uint64_t skip
 constexpr uint64_t kMtSplitMin = uint64_t(1) << 17, kMtSegMin = uint64_t(1) << 14;
 constexpr uint32_t kMtMaxSegs = 512;
 // While the caller's stream is being captured no table is made for calls of up
-// to kMtCaptureSolo words: they run as one segment unless the table exists.
-constexpr uint64_t kMtCaptureSolo = uint64_t(1) << 21;
+// to kMtCaptureSolo words: they run as one segment unless the table exists.  Nor
+// is one made for a program's first such calls (mtj::without_table): 2^18 words
+// take 118 us in one segment and 93 in several, 2^21 words 0.87 ms and 98 us, and
+// the table for the first takes 1 ms, for the second 2 (and 6 more where its copy
+// is the process's first).
+constexpr uint64_t kMtCaptureSolo = mtj::kRentWords;
 
 template <int OUT>
 pgh_status launch_mt(uint32_t seed, uint64_t skip, uint64_t n, void *out, uint32_t nx, int kind, hipStream_t s)
@@ -108,15 +113,15 @@ pgh_status launch_mt(uint32_t seed, uint64_t skip, uint64_t n, void *out, uint32
         const uint32_t segs = static_cast<uint32_t>((n + B - 1u) / B);
         uint32_t count = 32u;
         while (count < segs) count <<= 1;
-        PGH_TRY(jump_table_device(B, count - 1u, false, &table));
+        PGH_TRY(jump_table_find(B, count - 1u, &table));
         if (!table) {
             hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-            if (n <= kMtCaptureSolo && hipStreamIsCapturing(s, &cs) != hipSuccess) (void)hipGetLastError();
-            if (cs == hipStreamCaptureStatusNone) {
-                PGH_TRY(jump_table_device(B, count - 1u, true, &table));
-            } else {
-                B = n;
+            if (hipStreamIsCapturing(s, &cs) != hipSuccess) (void)hipGetLastError();
+            const bool capturing = cs != hipStreamCaptureStatusNone;
+            if (!capturing || n > kMtCaptureSolo) {
+                PGH_TRY(jump_table_make(B, count - 1u, n, capturing ? nullptr : &s, &table));
             }
+            if (!table) B = n;
         }
     }
     const uint32_t segs = static_cast<uint32_t>((n + B - 1u) / B);

@@ -1,5 +1,6 @@
-"""The memoised multiples of a jump distance (pagmo2_amd/csrc/mt_jump_host.hpp), on the
-CPU (tests/cpp/test_mt_multiples.cpp)."""
+"""The memoised multiples of a jump distance and the first calls that go without a table
+of them (pagmo2_amd/csrc/mt_jump_host.hpp), on the CPU (tests/cpp/test_mt_multiples.cpp,
+test_mt_first_calls.cpp)."""
 import os
 import subprocess
 
@@ -7,11 +8,19 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 
 
-def test_every_multiple_is_memoised():
-    out = os.path.join(HERE, "cpp", "bin", "test_mt_multiples")
+def run(name):
+    out = os.path.join(HERE, "cpp", "bin", name)
     os.makedirs(os.path.dirname(out), exist_ok=True)
     subprocess.check_call(["g++", "-std=c++17", "-O2", "-Wall", "-I", os.path.join(ROOT, "pagmo2_amd", "csrc"),
-                           os.path.join(HERE, "cpp", "test_mt_multiples.cpp"), "-o", out + ".tmp", "-pthread"])
+                           os.path.join(HERE, "cpp", name + ".cpp"), "-o", out + ".tmp", "-pthread"])
     os.replace(out + ".tmp", out)
     r = subprocess.run([out], capture_output=True, text=True, timeout=300)
     assert r.returncode == 0 and r.stdout.strip() == "ok", r.stdout + r.stderr
+
+
+def test_every_multiple_is_memoised():
+    run("test_mt_multiples")
+
+
+def test_first_calls_make_no_table():
+    run("test_mt_first_calls")
