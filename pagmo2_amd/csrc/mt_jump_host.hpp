@@ -360,6 +360,19 @@ inline void prefetch_multiples(uint64_t S, uint64_t count)
     run = std::max(run, count);
 }
 
+// ---- shares of an archipelago's velocity draws -------------------------------------
+// Words per share, where all islands together draw `total` on a device of `cus` CUs:
+// 2^15, or the power of two that leaves two to four shares per CU.  A share costs a
+// jump, as much as making 1.5 10^5 words, and its polynomial's place in the
+// archipelago's table: 10^8 words in shares of 2^15 would be 3052 of them.
+inline uint64_t velocity_share(uint64_t total, uint32_t cus)
+{
+    const uint64_t want = total / (2u * std::max(cus, 1u));
+    uint64_t share = uint64_t(1) << 15;
+    while (share * 2u <= want) share *= 2u;
+    return share;
+}
+
 // ---- when a device table of multiples is worth making ----------------------------
 // Making one costs a process 1 to 3 ms once (31 to 127 multiples, an allocation and
 // an upload), as long as one workgroup takes for 2^21 to 2^23 words.  So calls of up

@@ -32,6 +32,7 @@
 
 #include "fitness_dev.hpp"
 #include "mt_dev.hpp"
+#include "mt_jump_host.hpp"
 #include "pgh_internal.hpp"
 
 namespace pgh
@@ -61,8 +62,10 @@ struct island_desc {
     uint64_t bwords, swords;
     uint32_t segs, seg0, gps;
     uint32_t j_n0, j_pos, j_main, j_last;
-    // the velocity draws (n0 words) split in vsegs shares of kVelShare words,
-    // share s reached by z^(s kVelShare) at j_vel + s - 1; 0: one share, made by
+    // the velocity draws (n0 words) split in vsegs shares of the archipelago's
+    // vel_share words (the draws of a large island, 4 M words at 4096 x 500, take
+    // one workgroup 1.4 ms), share s reached by z^(s vel_share) at j_vel + s - 1;
+    // 0: one share, made by
     // segment 0 on its way to the first batch
     uint32_t vsegs, j_vel;
     // pso_gen's variant (1..6) and topology (1 gbest, 2 lbest, 3 von Neumann),
@@ -94,10 +97,6 @@ constexpr uint32_t kBlock = 256;
 // the batch's words are made by many workgroups at once
 constexpr uint32_t kGenBatch = 32;
 constexpr uint64_t kSegMin = uint64_t(1) << 16, kSegMax = uint64_t(1) << 22, kSoloWords = uint64_t(1) << 20;
-// Words per share of the velocity draws: from two shares on, the draws of a
-// large island (4 M words at 4096 x 500, 1.4 ms in one workgroup) are made by
-// many workgroups before the call's first batch.
-constexpr uint64_t kVelShare = uint64_t(1) << 15;
 // seg_desc::s of the workgroup that copies an island's generator (k_rng_vel)
 constexpr uint32_t kSegCopy = 0xffffffffu;
 
@@ -204,7 +203,7 @@ __global__ __launch_bounds__(kMtBlock) void k_rng_vel(const island_desc *__restr
                                                       const seg_desc *__restrict__ vsd,
                                                       const mt_state *__restrict__ st, mt_state *__restrict__ stq,
                                                       const uint32_t *__restrict__ polys, double *__restrict__ V,
-                                                      uint32_t vs0, uint32_t v_valid)
+                                                      uint32_t vs0, uint64_t share, uint32_t v_valid)
 {
     __shared__ __align__(16) uint32_t buf[kMtBuf];
     const seg_desc sg = vsd[vs0 + blockIdx.x];
@@ -215,11 +214,11 @@ __global__ __launch_bounds__(kMtBlock) void k_rng_vel(const island_desc *__restr
         mt_store(stq[sg.island], buf, pos);
         return;
     }
-    const uint64_t n0 = velocity_words(di, v_valid), begin = sg.s * kVelShare;
+    const uint64_t n0 = velocity_words(di, v_valid), begin = sg.s * share;
     if (begin >= n0) return;
     mt_load(st[sg.island], buf, pos);
     if (sg.s > 0u) mt_jump(buf, polys + static_cast<uint64_t>(di.j_vel + sg.s - 1u) * kMtN);
-    mt_hand_out(buf, pos, min(kVelShare, n0 - begin),
+    mt_hand_out(buf, pos, min(share, n0 - begin),
                 velocity_sink(V + di.xoff, begin / 2u, di));
 }
 
@@ -1498,6 +1497,7 @@ struct pgh_archi {
     // contiguous from vseg_begin[k], and those copies
     arena_view vsegs, states_q;
     std::vector<uint32_t> vseg_begin;
+    uint64_t vel_share = 0; // words (mtj::velocity_share)
     // the gbest islands (their indices, in order) and their best positions
     arena_view gblist, gbest;
     std::vector<uint32_t> h_gb;
@@ -1764,7 +1764,7 @@ pgh_status launch_range(pgh_archi *a, uint32_t i0, uint32_t i1, bool v_valid, bo
     const uint32_t vv = v_valid ? 1u : 0u;
     const uint32_t vs0 = a->vseg_begin[i0];
     k_rng_vel<<<a->vseg_begin[i1] - vs0, kMtBlock, 0, s>>>(d, static_cast<const seg_desc *>(a->vsegs.ptr), st, stq, jt,
-                                                           V, vs0, vv);
+                                                           V, vs0, a->vel_share, vv);
     PGH_HIP(hipGetLastError());
     const auto make_words = [&](uint32_t b, hipStream_t on) {
         k_rng<<<ng, kMtBlock, 0, on>>>(d, sd, st, stq, segst, jt, w, V, sg0, b, vv);
@@ -1959,12 +1959,13 @@ pgh_status archi_create(pgh_archi **out, const pgh_island_spec *islands, uint64_
     uint64_t seg_words = kSegMin, max_segs = 1u, max_vsegs = 0u;
     // shares of an island's velocity draws: up to four (44 us in one workgroup,
     // about a jump) are left to segment 0
-    const auto vel_shares = [](uint64_t n0) {
-        return n0 > 4u * kVelShare ? static_cast<uint32_t>((n0 + kVelShare - 1u) / kVelShare) : 0u;
+    uint64_t vel_share = 0u;
+    const auto vel_shares = [&vel_share](uint64_t n0) {
+        return n0 > uint64_t(1) << 17 ? static_cast<uint32_t>((n0 + vel_share - 1u) / vel_share) : 0u;
     };
     {
-        uint64_t total = 0;
-        std::vector<uint64_t> bw(n_islands, 0u);
+        uint64_t total = 0, vel_total = 0;
+        std::vector<uint64_t> bw(n_islands, 0u), n0(n_islands, 0u);
         for (uint64_t k = 0; k < n_islands; ++k) {
             prob p;
             PGH_TRY(resolve(&islands[k].udp, p));
@@ -1974,8 +1975,11 @@ pgh_status archi_create(pgh_archi **out, const pgh_island_spec *islands, uint64_
             uint32_t wpu = 0u;
             bw[k] = gps * words_per_gen(q.variant, K, islands[k].pop, p.nx, wpu);
             total += bw[k];
-            max_vsegs = std::max<uint64_t>(max_vsegs, vel_shares(2u * islands[k].pop * p.nx));
+            n0[k] = 2u * islands[k].pop * p.nx;
+            vel_total += n0[k];
         }
+        vel_share = a->vel_share = mtj::velocity_share(vel_total, a->n_cus);
+        for (const uint64_t w : n0) max_vsegs = std::max<uint64_t>(max_vsegs, vel_shares(w));
         const uint64_t want = total / (2u * a->n_cus);
         while (seg_words * 2u <= want && seg_words < kSegMax) seg_words *= 2u;
         // a lone island of a small batch stays one generator (the one-shot
@@ -1988,8 +1992,8 @@ pgh_status archi_create(pgh_archi **out, const pgh_island_spec *islands, uint64_
     for (uint64_t k = 1; k < max_segs; ++k) dists.push_back(k * seg_words);
     PGH_TRY(jump_polys_multiples(seg_words, max_segs - 1u));
     const uint32_t j_vel = static_cast<uint32_t>(dists.size());
-    for (uint64_t k = 1; k < max_vsegs; ++k) dists.push_back(k * kVelShare);
-    if (max_vsegs > 1u) PGH_TRY(jump_polys_multiples(kVelShare, max_vsegs - 1u));
+    for (uint64_t k = 1; k < max_vsegs; ++k) dists.push_back(k * vel_share);
+    if (max_vsegs > 1u) PGH_TRY(jump_polys_multiples(vel_share, max_vsegs - 1u));
     std::vector<seg_desc> vseg_list;
     const auto dist_index = [&dists](uint64_t J) {
         for (size_t i = 0; i < dists.size(); ++i) {

@@ -1,6 +1,6 @@
-"""The memoised multiples of a jump distance and the first calls that go without a table
-of them (pagmo2_amd/csrc/mt_jump_host.hpp), on the CPU (tests/cpp/test_mt_multiples.cpp,
-test_mt_first_calls.cpp)."""
+"""The memoised multiples of a jump distance, the first calls that go without a table of
+them and the velocity shares that jumps reach (pagmo2_amd/csrc/mt_jump_host.hpp), on the
+CPU (tests/cpp/test_mt_multiples.cpp, test_mt_first_calls.cpp, test_velocity_shares.cpp)."""
 import os
 import subprocess
 
@@ -24,3 +24,7 @@ def test_every_multiple_is_memoised():
 
 def test_first_calls_make_no_table():
     run("test_mt_first_calls")
+
+
+def test_velocity_shares_are_bounded():
+    run("test_velocity_shares")
