@@ -327,8 +327,8 @@ pgh_status pgh_archi_get_trace(pgh_archi *a, uint64_t k, double *trace_F);
  *                  48 KiB, at most 64 KiB)
  *   blocks_per_cu: resident workgroups per CU, at most (0 = as many as can
  *                  be)
- * pgh_archi_tune times candidate mappings (form x lj_lds in {64, 32, 16}
- * KiB x blocks_per_cu in {0, 2}) with one batched evolve call each, `reps`
+ * pgh_archi_tune times candidate mappings (form x lj_lds in {64, 48, 32,
+ * 16} KiB x blocks_per_cu in {0, 2}) with one batched evolve call each, `reps`
  * times, from the archipelago's current state, which it restores afterwards;
  * every candidate must leave a population bit-identical to the first's
  * (else DEVICE_ERROR).  It keeps the fastest and returns it in *chosen.

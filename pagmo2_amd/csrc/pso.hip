@@ -30,6 +30,7 @@
 #include <string>
 #include <vector>
 
+#include "archi_map.hpp"
 #include "fitness_dev.hpp"
 #include "mt_dev.hpp"
 #include "mt_jump_host.hpp"
@@ -681,12 +682,6 @@ __host__ __device__ constexpr uint32_t step_class(int kind)
 constexpr uint32_t kStepRosenRows = (kBlock / 64u) * kRosenWaveRows;
 constexpr uint32_t kStepRosenTerms = (kBlock / 64u) * kRosenWaveRows * kRosenWaveStride, kStepRosenElems = 4096;
 constexpr size_t kStepRosenLds = (kStepRosenTerms + kStepRosenElems) * sizeof(double);
-// Default LDS for the individuals of a Lennard-Jones item: with it (and a
-// rosenbrock item's) three workgroups fit a CU (two: 101 against 88 us a
-// generation of the 32-island workload, 133 against 114 us of the 64-island one;
-// four, with 36 KiB: 90 and 111; 16 KiB cuts the items of 12 islands too small,
-// 56 against 51 us).
-constexpr uint32_t kStepLjLds = 49152;
 constexpr size_t kCuLds = 163840; // LDS of a CU
 
 struct step_args {
@@ -1514,7 +1509,7 @@ struct pgh_archi {
     uint32_t class_begin[4] = {0, 0, 0, 0}; // per step class, into the class order (+ end)
     size_t lj_lds = 0;                      // LDS of the Lennard-Jones items
     uint32_t n_cus = 0;
-    pgh_archi_mapping map{PGH_ARCHI_STEP_ONE, 0u, 0u, 0u}; // the 64-island workload's fastest form
+    pgh_archi_mapping map = kArchiDefault;
     size_t step_bytes[4] = {0, 0, 0, 0}; // k_step's dynamic LDS, per class
     uint32_t n_segs = 0;
     hipStream_t own = nullptr;
@@ -2411,12 +2406,7 @@ try {
         return PGH_OK;
     };
     a->trace = false;
-    std::vector<pgh_archi_mapping> cand;
-    for (uint32_t form : {static_cast<uint32_t>(PGH_ARCHI_STEP_SPLIT), static_cast<uint32_t>(PGH_ARCHI_STEP_ONE)}) {
-        for (uint32_t lds : {65536u, 32768u, 16384u}) {
-            for (uint32_t bpc : {0u, 2u}) cand.push_back(pgh_archi_mapping{form, lds, bpc, 0u});
-        }
-    }
+    const std::vector<pgh_archi_mapping> cand = archi_candidates();
     pgh_status st = PGH_OK;
     float best_ms = 0.f;
     pgh_archi_mapping best = cand[0];
