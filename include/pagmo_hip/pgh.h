@@ -202,12 +202,14 @@ pgh_status pgh_fnds_copy(pgh_fnds_ws *ws, uint64_t *dom_count, uint64_t *rank, u
  *
  *      Peel workgroups of a workspace: 0 = the default (up to 16384 points of
  *      one to three objectives: no peel, the fronts come from ranks; otherwise
- *      one workgroup per 256 points); at most 4096 may be set, and a run clamps
- *      the count to the peel's range: at least one per 1024 points, at most one
- *      per 64 points, the CU count and 256.  pgh_fnds_tune tries one per 64, 128,
- *      256, 512 and 1024 points within that range; *chosen is the fastest (0
- *      when n > 32768: nothing to tune), which is set on the workspace unless
- *      the default without a peel was faster still. */
+ *      one workgroup per 256 points); at most 4096 may be set, which peels
+ *      every later run, and a run clamps the count to the peel's range: at
+ *      least one per 1024 points, at most one per 64 points, the CU count and
+ *      256.  pgh_fnds_tune tries one per 64, 128, 256, 512 and 1024 points
+ *      within that range, and the default without a peel; *chosen is the fastest
+ *      peel (0 when n > 32768: nothing to tune).  Later runs of the workspace that
+ *      are peeled take that count; those that could do without a peel do, unless
+ *      the input timed was such a one and the peel was faster. */
 pgh_status pgh_fnds_set_peel_blocks(pgh_fnds_ws *ws, uint32_t blocks);
 pgh_status pgh_fnds_tune(pgh_fnds_ws *ws, const double *objs, uint64_t n, uint64_t m, uint32_t reps, void *stream,
                          uint32_t *chosen);

@@ -607,7 +607,7 @@ pgh_status launch_grid_peel(pgh_fnds_ws *ws, hipStream_t s, uint32_t n32, uint32
     uint32_t gmin = 0, gmax = 0;
     peel_range(w32, cus, gmin, gmax);
     if (gmin > gmax) return fail(PGH_UNSUPPORTED, "fast_non_dominated_sorting: too few CUs for the grid peel");
-    const uint32_t want = ws->peel_blocks ? ws->peel_blocks : default_peel_blocks(w32);
+    const uint32_t want = ws->peel.blocks ? ws->peel.blocks : default_peel_blocks(w32);
     const uint32_t g = std::min(std::max(want, gmin), gmax);
     const uint32_t wpw = (w32 + g - 1u) / g; // <= kColWords, since g >= gmin
     const uint32_t G = (w32 + wpw - 1u) / wpw; // <= g, and no workgroup without a word
@@ -745,7 +745,7 @@ pgh_status fnds_run(pgh_fnds_ws *ws, const double *objs, uint64_t n, uint64_t m,
     if (n >= (uint64_t(1) << 31)) return fail(PGH_OVERFLOW, "too many points for fast_non_dominated_sorting");
     if (m && !objs) return fail(PGH_INVALID_ARGUMENT, "null objective matrix");
     if (m > 512u) return fail(PGH_UNSUPPORTED, "at most 512 objectives are supported");
-    const bool chain = n <= kChainMaxN && m >= 1u && m <= kChainMaxM && ws->peel_blocks == 0u;
+    const bool chain = ws->peel.ranks(n, m);
     ws->stream = s;
     ws->n = 0u; // (no result while the buffers may be replaced)
     ws->m = m;
@@ -857,7 +857,7 @@ try {
         return fail(PGH_INVALID_ARGUMENT, "at most " + std::to_string(kMaxPeelBlocks) + " peel workgroups, got "
                                               + std::to_string(blocks));
     }
-    ws->peel_blocks = blocks;
+    ws->peel.set(blocks);
     return PGH_OK;
 } catch (...) {
     return api_exception();
@@ -870,7 +870,7 @@ try {
     if (reps == 0u) return fail(PGH_INVALID_ARGUMENT, "the tuner needs at least one timed repetition");
     if (chosen) *chosen = 0u;
     if (n > kGridMaxN) { // the single-workgroup peel: nothing to tune
-        ws->peel_blocks = 0u;
+        ws->peel.set(0u);
         return pgh_fnds_run(ws, objs, n, m, stream);
     }
     const uint32_t n32 = static_cast<uint32_t>(n);
@@ -880,7 +880,7 @@ try {
     // the peel's counts, and 0: the way taken without one (fnds_chain.hip up to
     // kChainMaxN points)
     std::vector<uint32_t> cands;
-    if (n <= kChainMaxN && m >= 1u && m <= kChainMaxM) cands.push_back(0u);
+    if (peel_choice::by_ranks(n, m)) cands.push_back(0u);
     for (uint32_t per : {64u, 128u, 256u, 512u, 1024u}) {
         const uint32_t b = std::min(gmax, std::max(gmin, (n32 + per - 1u) / per));
         if (std::find(cands.begin(), cands.end(), b) == cands.end()) cands.push_back(b);
@@ -897,7 +897,7 @@ try {
     uint32_t best_b = 0u;
     pgh_status st = PGH_OK;
     for (uint32_t b : cands) {
-        ws->peel_blocks = b;
+        ws->peel.set(b);
         st = pgh_fnds_run(ws, objs, n, m, stream); // warm-up (and argument checks)
         if (st != PGH_OK) break;
         if ((st = hip_status(hipEventRecord(e0, s), "hipEventRecord")) != PGH_OK) break;
@@ -926,10 +926,10 @@ try {
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     if (st != PGH_OK) {
-        ws->peel_blocks = 0u;
+        ws->peel.set(0u);
         return st;
     }
-    ws->peel_blocks = chain > 0.f && chain <= best ? 0u : best_b;
+    ws->peel.tuned(n, m, best_b, best < chain);
     if (chosen) *chosen = best_b;
     // leave the workspace holding a result computed with the chosen grid
     return pgh_fnds_run(ws, objs, n, m, stream);

@@ -8,6 +8,7 @@
 #include <cstdint>
 #include <vector>
 
+#include "fnds_route.hpp"
 #include "pgh_internal.hpp"
 
 namespace pgh
@@ -31,14 +32,6 @@ __device__ __forceinline__ void wave_lds_fence()
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
-
-// fnds_chain.hip takes up to kChainMaxN points (its sort keys, positions and bit
-// planes fit one workgroup's LDS) of one to kChainMaxM objectives.  With more
-// objectives the fronts are few and large, and the grid-wide peel, whose cost is
-// an exchange per front, is faster: 16384 x 3 (54 fronts) 0.70 against 0.90 ms
-// for the peel, 16384 x 5 (15 fronts) 1.30 against 0.67 ms; with two objectives
-// (8192: 176-213 fronts) 0.40 against 1.2-1.4 ms.
-constexpr uint32_t kChainMaxN = 16384, kChainMaxM = 3;
 
 // A buffer inside one of the workspace's allocations.
 struct ws_view {
@@ -86,9 +79,9 @@ struct pgh_fnds_ws {
     bool emitted = false; // dom_items holds the result's lists
     bool lists = false; // D, dom_offsets and dom_count hold this result's
     bool items = false; // front_items holds every front's
-    // workgroups of the grid-wide front peel: 0 = the default rule, else the
-    // value set or found by pgh_fnds_tune (any count gives the same result)
-    uint32_t peel_blocks = 0;
+    // workgroups of the grid-wide front peel, set or found by pgh_fnds_tune (any
+    // count gives the same result, and so do ranks)
+    pgh::peel_choice peel;
     // mo_sort.hip: sort keys and values (two of each), crowding, radix-sort
     // scratch, and a staged output
     pgh::dev_buf sk0, sk1, sv0, sv1, crowd, sort_tmp, out_staged;
