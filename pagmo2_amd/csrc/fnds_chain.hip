@@ -48,7 +48,7 @@ constexpr uint32_t kBlock = 256, kWide = 1024;
 constexpr uint32_t kRankBits = 14; // ranks and positions below kChainMaxN = 2^14
 constexpr uint32_t kPlanes = 16;   // bit planes' stride: kRankBits, padded
 
-// Exclusive scan over one workgroup of kWide threads; sh holds kWide / 64 + 1.
+// Exclusive scan over one workgroup of kWide threads; sh holds kWide / 64.
 __device__ __forceinline__ uint32_t wide_exclusive_scan(uint32_t v, uint32_t *sh, uint32_t &total)
 {
     const uint32_t lane = threadIdx.x & 63u, wid = threadIdx.x >> 6;

@@ -125,19 +125,17 @@ __device__ __forceinline__ void mt_block(const uint32_t *__restrict__ A, uint32_
     }
 }
 
-template <uint32_t NT = kMtBlock>
 __device__ __forceinline__ void mt_load(const mt_state &st, uint32_t *__restrict__ buf, uint32_t &pos)
 {
-    for (uint32_t i = threadIdx.x; i < kMtN; i += NT) buf[kMtCur + i] = st.x[i];
+    for (uint32_t i = threadIdx.x; i < kMtN; i += kMtBlock) buf[kMtCur + i] = st.x[i];
     pos = st.pos;
     __syncthreads();
 }
 
 // The state after the last call, whose barrier orders buf's words.
-template <uint32_t NT = kMtBlock>
 __device__ __forceinline__ void mt_store(mt_state &st, const uint32_t *__restrict__ buf, uint32_t pos)
 {
-    for (uint32_t i = threadIdx.x; i < kMtN; i += NT) st.x[i] = buf[kMtCur + i];
+    for (uint32_t i = threadIdx.x; i < kMtN; i += kMtBlock) st.x[i] = buf[kMtCur + i];
     if (threadIdx.x == 0) st.pos = pos;
 }
 
@@ -145,25 +143,22 @@ __device__ __forceinline__ void mt_store(mt_state &st, const uint32_t *__restric
 // LDS, untempered, from position `at` of the hand-out on (an even one after
 // the first run), by threads tid of nthr, which must not synchronise.  The
 // first four wavefronts make a phase of four blocks while the others hand out
-// the phase before it (a workgroup of 256 threads does both in turn), with a
-// barrier per block: making a block is a chain of LDS reads, about 30
-// instructions for a thread's three words and LDS writes, which the hand-out's
-// tempering and mapping (about 28 instructions per two words) overlaps.
+// the phase before it, with a barrier per block: making a block is a chain of LDS
+// reads, about 30 instructions for a thread's three words and LDS writes, which the
+// hand-out's tempering and mapping (about 28 instructions per two words) overlaps.
 // Measured: one workgroup alone makes 2.6 words/ns with the mapping to doubles
 // (1.3 with a barrier per 227 words and the hand-out in the same threads, and
 // the mapping in a pass of its own), two on a CU 3.4 together, which keeps its
 // SIMDs about 60% busy; four on a CU make 4.0 but need twice the jumps.
-template <uint32_t NT = kMtBlock, class Sink>
+template <class Sink>
 __device__ __forceinline__ void mt_hand_out(uint32_t *__restrict__ buf, uint32_t &pos, uint64_t count, Sink sink)
 {
-    static_assert(NT == 256u || NT == 512u, "four wavefronts make blocks, the rest hand out");
+    static_assert(kMtBlock == 512u, "four wavefronts make blocks, four hand out");
     const uint32_t t = threadIdx.x;
-    const bool emits = NT == 256u || t >= 256u;
-    const uint32_t et = NT == 256u ? t : t - 256u;
     uint64_t done = 0u, prev_at = 0u;
     const uint32_t have = static_cast<uint32_t>(min(static_cast<uint64_t>(kMtN - pos), count));
     if (have) {
-        sink(static_cast<uint64_t>(0), buf + kMtCur + pos, have, t, NT);
+        sink(static_cast<uint64_t>(0), buf + kMtCur + pos, have, t, kMtBlock);
         pos += have;
         done = have;
     }
@@ -180,9 +175,9 @@ __device__ __forceinline__ void mt_hand_out(uint32_t *__restrict__ buf, uint32_t
             }
             // the phase before, 256 pairs of words at a time: two, one, one and
             // the last 224
-            if (emits) {
+            if (t >= 256u) {
                 const uint32_t lo = b ? 512u * (b + 1u) : 0u, hi = min(prev_n, b < 3u ? 512u * (b + 2u) : kMtPhase);
-                if (lo < hi) sink(prev_at + lo, buf + prev + lo, hi - lo, et, 256u);
+                if (lo < hi) sink(prev_at + lo, buf + prev + lo, hi - lo, t - 256u, 256u);
             }
             __syncthreads();
         }
@@ -193,11 +188,11 @@ __device__ __forceinline__ void mt_hand_out(uint32_t *__restrict__ buf, uint32_t
         done += n;
         pos = n - (blocks - 1u) * kMtN;
     }
-    if (prev_n) sink(prev_at, buf + prev, prev_n, t, NT);
+    if (prev_n) sink(prev_at, buf + prev, prev_n, t, kMtBlock);
     // (the phase at kMtCur, unless it is the one just handed out and then cur
     // is kMtCur, was handed out before the last barrier)
     if (cur != kMtCur) {
-        for (uint32_t i = t; i < kMtN; i += NT) buf[kMtCur + i] = buf[cur + i];
+        for (uint32_t i = t; i < kMtN; i += kMtBlock) buf[kMtCur + i] = buf[cur + i];
     }
     __syncthreads();
 }

@@ -66,8 +66,7 @@ struct island_desc {
     // the velocity draws (n0 words) split in vsegs shares of the archipelago's
     // vel_share words (the draws of a large island, 4 M words at 4096 x 500, take
     // one workgroup 1.4 ms), share s reached by z^(s vel_share) at j_vel + s - 1;
-    // 0: one share, made by
-    // segment 0 on its way to the first batch
+    // 0: one share, made by segment 0 on its way to the first batch
     uint32_t vsegs, j_vel;
     // pso_gen's variant (1..6) and topology (1 gbest, 2 lbest, 3 von Neumann),
     // the neighbours per particle (lbest 2 radius, von Neumann 4) and the von
@@ -223,9 +222,7 @@ __global__ __launch_bounds__(kMtBlock) void k_rng_vel(const island_desc *__restr
                 velocity_sink(V + di.xoff, begin / 2u, di));
 }
 
-// Batch b's words of one segment (see above) from the generator in buf, by a
-// workgroup of NT threads.
-template <uint32_t NT>
+// Batch b's words of one segment (see above) from the generator in buf.
 __device__ __forceinline__ void rng_gen_segment(const island_desc &di, uint32_t s, uint32_t b, uint64_t n0,
                                                 mt_state *__restrict__ st, mt_state *__restrict__ mine,
                                                 uint32_t *__restrict__ batch_words, uint32_t *__restrict__ buf,
@@ -234,8 +231,8 @@ __device__ __forceinline__ void rng_gen_segment(const island_desc &di, uint32_t 
     uint64_t start, count, end;
     seg_span(di, s, b, n0, start, count, end);
     if (count == 0u) return;
-    mt_hand_out<NT>(buf, pos, count, mt_word_sink{batch_words + static_cast<uint64_t>(s) * di.swords});
-    mt_store<NT>(start + count == end ? *st : *mine, buf, pos);
+    mt_hand_out(buf, pos, count, mt_word_sink{batch_words + static_cast<uint64_t>(s) * di.swords});
+    mt_store(start + count == end ? *st : *mine, buf, pos);
 }
 
 __global__ __launch_bounds__(kMtBlock) void k_rng(const island_desc *__restrict__ d, const seg_desc *__restrict__ sd,
@@ -279,7 +276,7 @@ __global__ __launch_bounds__(kMtBlock) void k_rng(const island_desc *__restrict_
         mt_store(st[sg.island], buf, pos);
         return;
     }
-    rng_gen_segment<kMtBlock>(di, sg.s, b, n0, &st[sg.island], mine, words + di.woff + ((b & 1u) ? di.whalf : 0u), buf, pos);
+    rng_gen_segment(di, sg.s, b, n0, &st[sg.island], mine, words + di.woff + ((b & 1u) ? di.whalf : 0u), buf, pos);
 }
 
 // Start of an evolve call (pso_gen.cpp:183-200): X = lbX = the population.  The population is X/fit before the
@@ -1099,6 +1096,14 @@ __device__ __forceinline__ void step_item(const island_desc &di, const tile &tl,
     }
 }
 
+// Wavefronts per SIMD each class's kernel is built for (its register budget, so
+// that none spills in its loops): rosenbrock's move streams from memory and wants
+// occupancy, the separable and Lennard-Jones evaluations want registers.
+constexpr int step_min_waves(uint32_t cls)
+{
+    return cls == kStepRosen ? 8 : 4;
+}
+
 // One generation of item order[blockIdx.x] (or base + blockIdx.x): a workgroup
 // per item, so that nothing is kept over items.  (A persistent grid that took
 // items from a queue kept the constants of every class's evaluation over that
@@ -1107,17 +1112,6 @@ __device__ __forceinline__ void step_item(const island_desc &di, const tile &tl,
 // the evaluations.)  32 uneven islands, 4.1M elements: 70 us a generation against
 // 122; alone, the move takes 47 (memory) and the evaluation with the stores 50
 // (vector units, 29 us of issue).
-// Wavefronts per SIMD each class's kernel is built for (its register budget, so
-// that none spills in its loops): rosenbrock's move streams from memory and wants
-// occupancy, the separable and Lennard-Jones evaluations want registers.
-#ifndef PGH_STEP_BOUNDED
-#define PGH_STEP_BOUNDED 1
-#endif
-constexpr int step_min_waves(uint32_t cls)
-{
-    return !PGH_STEP_BOUNDED ? 1 : (cls == kStepRosen ? 8 : 4);
-}
-
 template <uint32_t CLASS, bool GEN>
 __global__ __launch_bounds__(kBlock, step_min_waves(CLASS)) void k_step(step_args a)
 {
@@ -1312,7 +1306,7 @@ __global__ __launch_bounds__(kMtBlock) void k_gens_one_tile(const island_desc *_
         __shared__ __align__(16) uint32_t buf[kMtBuf];
         uint32_t pos;
         mt_load(segst[di.seg0], buf, pos);
-        rng_gen_segment<kMtBlock>(di, 0u, g1 / di.gps, 0u, &st[island], &segst[di.seg0], words_next + di.woff, buf, pos);
+        rng_gen_segment(di, 0u, g1 / di.gps, 0u, &st[island], &segst[di.seg0], words_next + di.woff, buf, pos);
         return;
     }
     const uint32_t end = min(g1, di.gens);
