@@ -671,20 +671,52 @@ __global__ __launch_bounds__(kWide) void k_fronts(const uint32_t *__restrict__ s
 }
 
 // members: every front's elements by index.  A wavefront per element counts the
-// smaller ones.
+// smaller ones, in a front of up to kBigFront.  In a larger one (at most three) a
+// wavefront per 64 indices counts them in the ranks of all smaller indices, once for
+// all its elements of that front: one front of 16384 took 126 us element by element.
+constexpr uint32_t kBigFront = 4096;
 __global__ __launch_bounds__(kBlock) void k_slots(const uint32_t *__restrict__ any, const uint32_t *__restrict__ rank,
-                                                  const uint32_t *__restrict__ fo, uint32_t n,
+                                                  const uint32_t *__restrict__ fo, uint32_t n, uint32_t big_groups,
                                                   uint32_t *__restrict__ members)
 {
-    const uint32_t x = blockIdx.x * (kBlock / 64u) + (threadIdx.x >> 6), lane = threadIdx.x & 63u;
-    if (x >= n) return;
-    const uint32_t i = any[x], f = rank[i], a = fo[f], b = fo[f + 1u];
-    uint32_t slot = 0u;
-    for (uint32_t q = a; q < b; q += 64u) {
-        const uint32_t o = q + lane;
-        slot += static_cast<uint32_t>(__popcll(__ballot(o < b && any[min(o, b - 1u)] < i)));
+    const uint32_t lane = threadIdx.x & 63u;
+    if (blockIdx.x >= big_groups) {
+        const uint32_t x = (blockIdx.x - big_groups) * (kBlock / 64u) + (threadIdx.x >> 6);
+        if (x >= n) return;
+        const uint32_t i = any[x], f = rank[i], a = fo[f], b = fo[f + 1u];
+        if (b - a > kBigFront) return;
+        uint32_t slot = 0u;
+        for (uint32_t q = a; q < b; q += 64u) {
+            const uint32_t o = q + lane;
+            slot += static_cast<uint32_t>(__popcll(__ballot(o < b && any[min(o, b - 1u)] < i)));
+        }
+        if (lane == 0u) members[a + slot] = i;
+        return;
     }
-    if (lane == 0u) members[a + slot] = i;
+    // (these workgroups first: theirs is the longer chain)
+    const uint32_t x = blockIdx.x * (kBlock / 64u) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (64u * x >= n) return;
+    const uint32_t i = 64u * x + lane, r = rank[min(i, n - 1u)];
+    uint64_t todo = __ballot(i < n && fo[r + 1u] - fo[r] > kBigFront);
+    while (todo) { // uniform
+        const uint32_t f = __builtin_amdgcn_readlane(r, static_cast<uint32_t>(__builtin_ctzll(todo)));
+        const uint64_t mine = __ballot(i < n && r == f);
+        uint32_t before = 0u;
+        constexpr uint32_t kAtOnce = 16;
+        for (uint32_t q0 = 0; q0 < x; q0 += kAtOnce) {
+            uint32_t v[kAtOnce];
+#pragma unroll
+            for (uint32_t u = 0; u < kAtOnce; ++u) v[u] = rank[64u * min(q0 + u, x - 1u) + lane];
+#pragma unroll
+            for (uint32_t u = 0; u < kAtOnce; ++u) {
+                before += static_cast<uint32_t>(__popcll(__ballot(q0 + u < x && v[u] == f)));
+            }
+        }
+        if (i < n && r == f) {
+            members[fo[f] + before + static_cast<uint32_t>(__popcll(mine & ((uint64_t(1) << lane) - 1u)))] = i;
+        }
+        todo &= ~mine;
+    }
 }
 
 // For every element of a front but the first: the bits of its dominators among
@@ -1273,7 +1305,8 @@ pgh_status launch_chain_fronts(pgh_fnds_ws *ws, hipStream_t s, uint32_t n, uint3
     k_fronts<<<1, kWide, fronts_lds, s>>>(srank, perm, n, fo, static_cast<uint64_t *>(ws->front_offsets.ptr), wbase,
                                           rank, any, sc);
     PGH_HIP(hipGetLastError());
-    k_slots<<<waves, kBlock, 0, s>>>(any, rank, fo, n, members);
+    const uint32_t big_groups = n > kBigFront ? (nb + kBlock / 64u - 1u) / (kBlock / 64u) : 0u;
+    k_slots<<<waves + big_groups, kBlock, 0, s>>>(any, rank, fo, n, big_groups, members);
     PGH_HIP(hipGetLastError());
     by_m(k_masks<1>, k_masks<2>, k_masks<3>)<<<waves, kBlock, 0, s>>>(keys, cnt, members, rank, fo, wbase, n, masks);
     PGH_HIP(hipGetLastError());

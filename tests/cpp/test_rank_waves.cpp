@@ -1,4 +1,4 @@
-// test_rank_waves.cpp -- k_order, k_rank, k_far and k_fronts of
+// test_rank_waves.cpp -- k_order, k_rank, k_far, k_fronts and k_slots of
 // pagmo2_amd/csrc/fnds_chain.hip on the CPU under several orders of their wavefronts
 // (wave_emu.hpp): the ranks must be those of the definition, whatever share of the
 // points has no dominator.  Tiles that the kernels may not read hold garbage.
@@ -102,6 +102,19 @@ static int check(uint32_t n, int which, int how)
         if (any[e] < n) ++seen[any[e]];
     }
     for (uint32_t i = 0; i < n; ++i) ok = ok && seen[i] == 1u;
+    // every front's members by index
+    std::vector<uint32_t> members(n, 0xffffffffu);
+    const uint32_t per = kBlock / 64u, groups = (n + per - 1u) / per, extra = n > kBigFront ? (nb + per - 1u) / per : 0u;
+    for (uint32_t b = 0; ok && b < groups + extra; ++b) {
+        wave_emu::block_idx.x = b;
+        wave_emu::run(kBlock, how, 5u, [&] { k_slots(any.data(), rank.data(), fo.data(), n, extra, members.data()); });
+    }
+    wave_emu::block_idx.x = 0u;
+    for (uint32_t f = 0; ok && f < fronts; ++f) {
+        for (uint32_t q = fo[f]; q < fo[f + 1u]; ++q) {
+            ok = ok && members[q] < n && rank[members[q]] == f && (q == fo[f] || members[q - 1u] < members[q]);
+        }
+    }
     if (!ok) std::printf("%u points of kind %d, order %d\n", n, which, how);
     return ok ? 0 : 1;
 }
@@ -118,6 +131,9 @@ int main()
     bad += check(2300u, kOneFront, wave_emu::kFirstAhead);
     bad += check(2300u, kOneDominated, wave_emu::kShuffled);
     bad += check(2300u, kThreeFronts, wave_emu::kFirstAhead);
+    // a front beyond kBigFront, alone and beside another
+    bad += check(4161u, kOneFront, wave_emu::kShuffled);
+    bad += check(4900u, kSeventh, wave_emu::kFirstAhead);
     if (bad) return 1;
     std::puts("ok");
     return 0;

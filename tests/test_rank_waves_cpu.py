@@ -1,5 +1,5 @@
-"""k_order, k_rank, k_far and k_fronts (pagmo2_amd/csrc/fnds_chain.hip) give the ranks and
-fronts under any order of their wavefronts, also where most points have no dominator:
+"""k_order, k_rank, k_far, k_fronts and k_slots (pagmo2_amd/csrc/fnds_chain.hip) give the
+ranks and fronts under any order of their wavefronts, also where most points have no dominator:
 the kernels' own text on the CPU (tests/cpp/test_rank_waves.cpp)."""
 import os
 import subprocess
