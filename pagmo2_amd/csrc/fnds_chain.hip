@@ -92,21 +92,39 @@ __device__ __forceinline__ void scan_bins(uint32_t *bins, uint32_t n, uint32_t *
     __syncthreads();
 }
 
-// use(i, load(i)) for the workgroup's elements, kAtOnce loads in flight (one
-// after another their latency is most of these kernels).
+// use(i, load(i), true) for the workgroup's elements, kAtOnce loads in flight (one
+// after another their latency is most of these kernels); every lane calls use, those
+// past the end with false.
 template <class Load, class Use>
 __device__ __forceinline__ void in_batches(uint32_t n, Load load, Use use)
 {
     constexpr uint32_t kAtOnce = 8;
-    for (uint32_t i0 = threadIdx.x; i0 < n; i0 += kAtOnce * kWide) {
+    for (uint32_t b = 0; b < n; b += kAtOnce * kWide) {
+        const uint32_t i0 = b + threadIdx.x;
         decltype(load(i0)) v[kAtOnce];
 #pragma unroll
         for (uint32_t u = 0; u < kAtOnce; ++u) v[u] = load(min(i0 + u * kWide, n - 1u));
 #pragma unroll
         for (uint32_t u = 0; u < kAtOnce; ++u) {
-            if (i0 + u * kWide < n) use(i0 + u * kWide, v[u]);
+            if (b + u * kWide >= n) break; // uniform
+            use(i0 + u * kWide, v[u], i0 + u * kWide < n);
         }
     }
+}
+
+// bins[k] += 1 for every lane that is `in`, and what was there.  One addition for the
+// wavefront where all lanes have the same bin: 64 to one address take 64 turns (one
+// front of 16384, whose counts are all zero: k_order 41 us).
+__device__ __forceinline__ uint32_t bin_add(uint32_t *bins, uint32_t k, bool in)
+{
+    const uint64_t who = __ballot(in);
+    if (who == 0u) return 0u; // uniform
+    const uint32_t lead = static_cast<uint32_t>(__builtin_ctzll(who)), same = __builtin_amdgcn_readlane(k, lead);
+    if (__ballot(in && k != same) != 0u) return in ? atomicAdd(&bins[k], 1u) : 0u;
+    const uint32_t lane = threadIdx.x & 63u;
+    uint32_t old = 0u;
+    if (lane == lead) old = atomicAdd(&bins[same], static_cast<uint32_t>(__popcll(who)));
+    return __builtin_amdgcn_readlane(old, lead) + static_cast<uint32_t>(__popcll(who & ((uint64_t(1) << lane) - 1u)));
 }
 
 // Every element's place in the order by dominator count (equal counts in any
@@ -119,11 +137,14 @@ __global__ __launch_bounds__(kWide) void k_order(const uint32_t *__restrict__ cn
     for (uint32_t i = threadIdx.x; i < n; i += kWide) bins[i] = 0u;
     __syncthreads();
     in_batches(n, [&](uint32_t i) { return cnt[i]; },
-               [&](uint32_t, uint32_t c) { atomicAdd(&bins[min(c, n - 1u)], 1u); });
+               [&](uint32_t, uint32_t c, bool in) { bin_add(bins, min(c, n - 1u), in); });
     __syncthreads();
     scan_bins(bins, n, sh);
     in_batches(n, [&](uint32_t i) { return cnt[i]; },
-               [&](uint32_t i, uint32_t c) { place[i] = min(atomicAdd(&bins[min(c, n - 1u)], 1u), n - 1u); });
+               [&](uint32_t i, uint32_t c, bool in) {
+                   const uint32_t at = bin_add(bins, min(c, n - 1u), in);
+                   if (in) place[i] = min(at, n - 1u);
+               });
 }
 
 // The elements, their counts and their keys in that order (scattered here: one
@@ -634,9 +655,9 @@ __global__ __launch_bounds__(kWide) void k_fronts(const uint32_t *__restrict__ s
     __syncthreads();
     uint32_t big = 0u;
     in_batches(n, [&](uint32_t e) { return min(srank[e], n - 1u); },
-               [&](uint32_t, uint32_t r) {
-                   big = max(big, r + 1u);
-                   atomicAdd(&bins[r], 1u);
+               [&](uint32_t, uint32_t r, bool in) {
+                   big = in ? max(big, r + 1u) : big;
+                   bin_add(bins, r, in);
                });
     atomicMax(&s_fronts, big);
     __syncthreads();
@@ -664,9 +685,12 @@ __global__ __launch_bounds__(kWide) void k_fronts(const uint32_t *__restrict__ s
     if (t == 0) scalars[0] = F;
     __syncthreads();
     in_batches(n, [&](uint32_t e) { return make_uint2(min(srank[e], n - 1u), perm[e]); },
-               [&](uint32_t, uint2 v) {
-                   rank[v.y] = v.x;
-                   any[min(atomicAdd(&bins[v.x], 1u), n - 1u)] = v.y;
+               [&](uint32_t, uint2 v, bool in) {
+                   const uint32_t at = bin_add(bins, v.x, in);
+                   if (in) {
+                       rank[v.y] = v.x;
+                       any[min(at, n - 1u)] = v.y;
+                   }
                });
 }
 
