@@ -852,8 +852,14 @@ __device__ __forceinline__ uint32_t held_max(uint64_t word, const uint64_t (&p)[
 //    while the front before is ordered.
 //  - Beyond, where comparing all with all would cost more than its barriers, the
 //    members are put in bins by the position of their last dominator and only
-//    compared there.
+//    compared there.  Words of at most kFewBits bits in every member, as in fronts of
+//    which each member has few dominators, are read bit by bit instead of plane by
+//    plane (about 10 instructions a bit, 90 for 14 planes), and others only where the
+//    largest position of their 64 is above a member's so far: with many dominators a
+//    member that leaves a handful (from the last word on, since the first front's
+//    positions ascend).
 constexpr uint32_t kStage = 2048, kAhead = 8, kWaves = kWide / 64u, kBin = 64;
+constexpr int kFewBits = 5;
 __global__ __launch_bounds__(kWide) void k_chain(const uint32_t *__restrict__ fo, const uint64_t *__restrict__ masks,
                                                  uint64_t mask_words, uint32_t upto,
                                                  const uint64_t *__restrict__ scalars, uint32_t n, uint32_t P,
@@ -872,6 +878,7 @@ __global__ __launch_bounds__(kWide) void k_chain(const uint32_t *__restrict__ fo
     __shared__ uint32_t fs[kWide + 2u], s_run, s_words, s_scan[kWide / 64u];
     __shared__ __align__(16) uint64_t vplanes[kWaves * kPlanes];
     __shared__ uint32_t s_v[kWide], s_pos[kWide]; // zero between fronts
+    __shared__ uint16_t s_top[kChainMaxN / 64u];
     const uint32_t t = threadIdx.x, lane = t & 63u, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     // the fronts that start at or before `upto`
     uint32_t fronts = min(static_cast<uint32_t>(scalars[0]), n);
@@ -1102,19 +1109,42 @@ __global__ __launch_bounds__(kWide) void k_chain(const uint32_t *__restrict__ fo
         const uint64_t *src = masks + wb;
         wb += static_cast<uint64_t>(c) * sw;
         uint32_t *bins = F + 64u * cw; // s of them; s + c <= n <= P
-        for (uint32_t x = t; x < s; x += kWide) bins[x] = 0u;
+        // the positions of the front before by slot, for words of few bits, and the
+        // largest of every 64
+        for (uint32_t x = t; x < 64u * sw; x += kWide) {
+            const uint32_t p = x < s ? pos_out[fl[0] + x] : 0u, most = wave_max(p);
+            if (lane == 0u) s_top[x >> 6] = static_cast<uint16_t>(most);
+            if (x < s) {
+                bins[x] = 0u;
+                list[x] = static_cast<uint16_t>(p);
+            }
+        }
         if (t == 0) s_run = 0u;
+        __syncthreads();
         for (uint32_t x = t; x < 64u * cw; x += kWide) {
             uint32_t v = 0u;
-            for (uint32_t w0 = 0; w0 < sw; w0 += kAhead) {
+            for (uint32_t left = sw; left > 0u; left -= min(left, kAhead)) { // from the last: see above
                 uint64_t word[kAhead];
 #pragma unroll
                 for (uint32_t k = 0; k < kAhead; ++k) {
-                    word[k] = x < c && w0 + k < sw ? src[static_cast<uint64_t>(w0 + k) * c + x] : 0u;
+                    word[k] = x < c && k < left ? src[static_cast<uint64_t>(left - 1u - k) * c + x] : 0u;
                 }
 #pragma unroll
                 for (uint32_t k = 0; k < kAhead; ++k) {
-                    if (__ballot(word[k] != 0u)) v = max(v, plane_max(word[k], planes + (w0 + k) * kPlanes, sb));
+                    if (k >= left) break; // uniform
+                    const uint32_t w = left - 1u - k;
+                    if (__ballot(__popcll(word[k]) > kFewBits)) {
+                        if (__ballot(word[k] != 0u && s_top[w] > v)) {
+                            v = max(v, plane_max(word[k], planes + w * kPlanes, sb));
+                        }
+                        continue;
+                    }
+                    while (__ballot(word[k] != 0u)) {
+                        if (word[k]) {
+                            v = max(v, static_cast<uint32_t>(list[64u * w + __builtin_ctzll(word[k])]));
+                            word[k] &= word[k] - 1u;
+                        }
+                    }
                 }
             }
             F[x] = v;
