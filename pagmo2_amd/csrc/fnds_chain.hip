@@ -638,8 +638,8 @@ __global__ __launch_bounds__(kFarBlock) void k_far(const uint64_t *__restrict__ 
     if (threadIdx.x < 64u && e < n) base[e] = first ? rr[lane] : max(base[e], rr[lane]);
 }
 
-// Front offsets (32 and 64 bits), the offset of each front's words of k_masks,
-// the number of fronts, the elements' ranks by index and the members of every
+// Front offsets (32 and 64 bits), the offset of each front's words of k_masks (and at n
+// whether a front but the first has more than kWide members), the number of fronts, the elements' ranks by index and the members of every
 // front in any order.
 __global__ __launch_bounds__(kWide) void k_fronts(const uint32_t *__restrict__ srank,
                                                   const uint32_t *__restrict__ perm, uint32_t n,
@@ -648,10 +648,10 @@ __global__ __launch_bounds__(kWide) void k_fronts(const uint32_t *__restrict__ s
                                                   uint32_t *__restrict__ any, uint64_t *__restrict__ scalars)
 {
     extern __shared__ uint32_t bins[]; // n + 1
-    __shared__ uint32_t sh[kWide / 64u], s_fronts;
+    __shared__ uint32_t sh[kWide / 64u], s_fronts, s_large;
     const uint32_t t = threadIdx.x;
     for (uint32_t i = t; i <= n; i += kWide) bins[i] = 0u;
-    if (t == 0) s_fronts = 0u;
+    if (t == 0) s_fronts = s_large = 0u;
     __syncthreads();
     uint32_t big = 0u;
     in_batches(n, [&](uint32_t e) { return min(srank[e], n - 1u); },
@@ -680,10 +680,12 @@ __global__ __launch_bounds__(kWide) void k_fronts(const uint32_t *__restrict__ s
         for (uint32_t f = b; f < e; ++f) {
             wbase[f] = o;
             o += words(f);
+            if (f && bins[f + 1u] - bins[f] > kWide) s_large = 1u;
         }
     }
     if (t == 0) scalars[0] = F;
     __syncthreads();
+    if (t == 0) wbase[n] = s_large; // (a place of no front's)
     in_batches(n, [&](uint32_t e) { return make_uint2(min(srank[e], n - 1u), perm[e]); },
                [&](uint32_t, uint2 v, bool in) {
                    const uint32_t at = bin_add(bins, v.x, in);
@@ -743,21 +745,82 @@ __global__ __launch_bounds__(kBlock) void k_slots(const uint32_t *__restrict__ a
     }
 }
 
+// k_masks for a front of more than kWide members: a wavefront takes 64 of them, one per
+// lane, and kTileWords words of the front before, whose members it loads 64 at a time
+// and broadcasts.
+constexpr uint32_t kTileWords = 2;
+template <int MT>
+__device__ __forceinline__ void masks_of_large(const int64_t *__restrict__ keys, const uint32_t *__restrict__ cnt,
+                                               const uint32_t *__restrict__ members,
+                                               const uint32_t *__restrict__ rank, const uint32_t *__restrict__ fo,
+                                               const uint64_t *__restrict__ wbase, uint32_t n, uint32_t b, uint32_t w0,
+                                               uint64_t *__restrict__ masks)
+{
+    const uint32_t lane = threadIdx.x & 63u, x = 64u * b + lane;
+    if (64u * b >= n) return;
+    const uint32_t i = members[min(x, n - 1u)], f = rank[i], a = fo[f], size = fo[f + 1u] - a;
+    const uint32_t pa = f ? fo[f - 1u] : a; // the front before: pa .. a - 1
+    uint64_t todo = __ballot(x < n && f > 0u && size > kWide && 64u * w0 < a - pa);
+    if (todo == 0u) return;
+    point<MT> mine;
+    mine.load(keys, cnt, i);
+    const uint64_t base = wbase[f];
+    while (todo) { // the 64 members' fronts in turn, uniform
+        const uint32_t lead = static_cast<uint32_t>(__builtin_ctzll(todo));
+        const uint32_t ff = __builtin_amdgcn_readlane(f, lead), fa = __builtin_amdgcn_readlane(a, lead);
+        const uint32_t fp = __builtin_amdgcn_readlane(pa, lead);
+        const bool on = ((todo >> lane) & 1u) && f == ff;
+        todo &= ~__ballot(on);
+        const uint32_t words = min((fa - fp + 63u) / 64u, w0 + kTileWords);
+        for (uint32_t w = w0; w < words; ++w) {
+            const uint32_t q = fp + 64u * w, there = min(64u, fa - q);
+            point<MT> other;
+            other.load(keys, cnt, members[min(q + lane, fa - 1u)]);
+            uint32_t half[2] = {0u, 0u}; // bit u from the top down
+#pragma unroll
+            for (uint32_t h = 0; h < 2u; ++h) {
+#pragma unroll 4
+                for (uint32_t u = 32u * h; u < 32u * h + 32u; ++u) {
+                    point<MT> one;
+                    one.cnt = __builtin_amdgcn_readlane(other.cnt, u);
+#pragma unroll
+                    for (int k = 0; k < MT; ++k) one.k[k] = lane_i64(other.k[k], u);
+                    half[h] = 2u * half[h] + (u < there && dominates<MT>(one, mine) ? 1u : 0u);
+                }
+            }
+            const uint64_t bits = __brev(half[0]) | (static_cast<uint64_t>(__brev(half[1])) << 32);
+            if (on) masks[base + static_cast<uint64_t>(w) * size + (x - a)] = bits;
+        }
+    }
+}
+
 // For every element of a front but the first: the bits of its dominators among
 // the members of the front before, word w of member c of front f at
-// wbase[f] + w * size + c.
+// wbase[f] + w * size + c.  A wavefront per element, which reads the front before;
+// for fronts of more than kWide members (n > 2 kWide) the first large_x * large_y
+// workgroups, which read it once per 64 elements (fronts of 5701, 3636, 2603, ...
+// element by element: 124 us).
 template <int MT>
 __global__ __launch_bounds__(kBlock) void k_masks(const int64_t *__restrict__ keys, const uint32_t *__restrict__ cnt,
                                                   const uint32_t *__restrict__ members,
                                                   const uint32_t *__restrict__ rank, const uint32_t *__restrict__ fo,
-                                                  const uint64_t *__restrict__ wbase, uint32_t n,
-                                                  uint64_t *__restrict__ masks)
+                                                  const uint64_t *__restrict__ wbase, uint32_t n, uint32_t large_x,
+                                                  uint32_t large_y, uint64_t *__restrict__ masks)
 {
-    const uint32_t x = blockIdx.x * (kBlock / 64u) + (threadIdx.x >> 6), lane = threadIdx.x & 63u;
+    const uint32_t lane = threadIdx.x & 63u;
+    if (blockIdx.x < large_x * large_y) {
+        if (wbase[n] == 0u) return; // no such front
+        const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        masks_of_large<MT>(keys, cnt, members, rank, fo, wbase, n, blockIdx.x % large_x * (kBlock / 64u) + wave,
+                           blockIdx.x / large_x * kTileWords, masks);
+        return;
+    }
+    const uint32_t x = (blockIdx.x - large_x * large_y) * (kBlock / 64u) + (threadIdx.x >> 6);
     if (x >= n) return;
     const uint32_t i = members[x], f = rank[i];
     if (f == 0u) return;
     const uint32_t a = fo[f], size = fo[f + 1u] - a, pa = fo[f - 1u];
+    if (large_y && size > kWide) return;
     point<MT> mine, other;
     mine.load(keys, cnt, i);
     for (uint32_t q = pa, w = 0u; q < a; q += 64u, ++w) {
@@ -1362,7 +1425,10 @@ pgh_status launch_chain_fronts(pgh_fnds_ws *ws, hipStream_t s, uint32_t n, uint3
     const uint32_t big_groups = n > kBigFront ? (nb + kBlock / 64u - 1u) / (kBlock / 64u) : 0u;
     k_slots<<<waves + big_groups, kBlock, 0, s>>>(any, rank, fo, n, big_groups, members);
     PGH_HIP(hipGetLastError());
-    by_m(k_masks<1>, k_masks<2>, k_masks<3>)<<<waves, kBlock, 0, s>>>(keys, cnt, members, rank, fo, wbase, n, masks);
+    const uint32_t large_x = (nb + kBlock / 64u - 1u) / (kBlock / 64u);
+    const uint32_t large_y = n > 2u * kWide ? (nb + kTileWords - 1u) / kTileWords : 0u;
+    by_m(k_masks<1>, k_masks<2>, k_masks<3>)<<<large_x * large_y + waves, kBlock, 0, s>>>(
+        keys, cnt, members, rank, fo, wbase, n, large_x, large_y, masks);
     PGH_HIP(hipGetLastError());
     return launch_chain_items(ws, s, n, upto);
 }

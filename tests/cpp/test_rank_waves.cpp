@@ -1,8 +1,9 @@
-// test_rank_waves.cpp -- k_order, k_rank, k_far, k_fronts and k_slots of
+// test_rank_waves.cpp -- k_order, k_rank, k_far, k_fronts, k_slots and k_masks of
 // pagmo2_amd/csrc/fnds_chain.hip on the CPU under several orders of their wavefronts
 // (wave_emu.hpp): the ranks must be those of the definition, whatever share of the
 // points has no dominator.  Tiles that the kernels may not read hold garbage.
 #include <cstdio>
+#include <cstring>
 #include <string>
 #include <vector>
 
@@ -34,7 +35,7 @@ static int check(uint32_t n, int which, int how)
             case kLong: y[i] = x[i] + 0.05 * u(rng); break;
             case kChainOnly: y[i] = x[i]; break;
             case kOneFront: y[i] = -x[i]; break;
-            case kThreeFronts: y[i] = -x[i] + (i % 3u) * 0.01; break;
+            case kThreeFronts: y[i] = -x[i] + (i % 3u) * 3.; break;
             case kOneDominated: y[i] = -x[i] + (i == n / 2u ? 3. : 0.); break;
             default: y[i] = -x[i] + (i % 7u == 0u ? 3. : 0.); break;
         }
@@ -115,6 +116,44 @@ static int check(uint32_t n, int which, int how)
             ok = ok && members[q] < n && rank[members[q]] == f && (q == fo[f] || members[q - 1u] < members[q]);
         }
     }
+    // the dominators' bits in the front before
+    std::vector<int64_t> keys(2u * n);
+    for (uint32_t i = 0; i < n; ++i) {
+        // (positive once shifted: a double's bits then order as the double does)
+        const double v[2] = {x[i] + 8., y[i] + 8.};
+        std::memcpy(&keys[2u * i], v, sizeof v);
+    }
+    uint64_t words = 0u;
+    for (uint32_t f = 1; ok && f < fronts; ++f) {
+        ok = wbase[f] == words;
+        words += static_cast<uint64_t>(fo[f + 1u] - fo[f]) * ((fo[f] - fo[f - 1u] + 63u) / 64u);
+    }
+    std::vector<uint64_t> masks(words + 1u, 0xcdcdcdcdcdcdcdcd);
+    const uint32_t large_x = (nb + per - 1u) / per, large_y = n > 2u * kWide ? (nb + kTileWords - 1u) / kTileWords : 0u;
+    for (uint32_t b = 0; ok && b < large_x * large_y + groups; ++b) {
+        wave_emu::block_idx.x = b;
+        wave_emu::run(kBlock, how, 6u, [&] {
+            k_masks<2>(keys.data(), cnt.data(), members.data(), rank.data(), fo.data(), wbase.data(), n, large_x, large_y,
+                       masks.data());
+        });
+    }
+    wave_emu::block_idx.x = 0u;
+    const auto shifted_dom = [&](uint32_t a, uint32_t b) {
+        return keys[2u * a] <= keys[2u * b] && keys[2u * a + 1u] <= keys[2u * b + 1u] && cnt[a] < cnt[b];
+    };
+    for (uint32_t f = 1; ok && f < fronts; ++f) {
+        const uint32_t a = fo[f], size = fo[f + 1u] - a, pa = fo[f - 1u], sw = (a - pa + 63u) / 64u;
+        for (uint32_t c = 0; ok && c < size; ++c) {
+            for (uint32_t w = 0; ok && w < sw; ++w) {
+                uint64_t bits = 0u;
+                for (uint32_t q = 64u * w; q < std::min(64u * w + 64u, a - pa); ++q) {
+                    if (shifted_dom(members[pa + q], members[a + c])) bits |= uint64_t(1) << (q - 64u * w);
+                }
+                ok = masks[wbase[f] + static_cast<uint64_t>(w) * size + c] == bits;
+            }
+        }
+    }
+    ok = ok && masks[words] == 0xcdcdcdcdcdcdcdcd;
     if (!ok) std::printf("%u points of kind %d, order %d\n", n, which, how);
     return ok ? 0 : 1;
 }
@@ -134,6 +173,8 @@ int main()
     // a front beyond kBigFront, alone and beside another
     bad += check(4161u, kOneFront, wave_emu::kShuffled);
     bad += check(4900u, kSeventh, wave_emu::kFirstAhead);
+    // a second front beyond kWide behind one and before another
+    bad += check(3300u, kThreeFronts, wave_emu::kLastAhead);
     if (bad) return 1;
     std::puts("ok");
     return 0;

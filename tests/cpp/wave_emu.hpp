@@ -11,6 +11,7 @@
 // static and `extern __shared__ T x[]` turned into pointers to dynamic_lds.
 #pragma once
 
+#include <setjmp.h>
 #include <ucontext.h>
 
 #include <algorithm>
@@ -36,8 +37,11 @@ struct dim3_ {
 
 enum state : int { kReady, kAtWave, kAtBlock, kDone };
 
+// (ucontext starts a fiber; the switches after that are jumps, without system calls)
 struct fiber {
     ucontext_t ctx;
+    jmp_buf at;
+    bool started = false;
     state st = kReady;
     uint32_t tid = 0, ops = 0;
     std::vector<char> stack;
@@ -47,7 +51,7 @@ struct block {
     uint32_t threads = 0;
     std::vector<fiber> f;
     std::vector<uint64_t> val[2]; // a lane's operand, by the parity of its operation
-    ucontext_t main;
+    jmp_buf main;
     uint32_t cur = 0;
     std::function<void()> body;
 };
@@ -70,14 +74,24 @@ inline void entry()
 {
     g->body();
     g->f[g->cur].st = kDone;
-    swapcontext(&g->f[g->cur].ctx, &g->main);
+    _longjmp(g->main, 1);
 }
 
 inline void wait(state s)
 {
     fiber &me = g->f[g->cur];
     me.st = s;
-    swapcontext(&me.ctx, &g->main);
+    if (_setjmp(me.at) == 0) _longjmp(g->main, 1);
+}
+
+__attribute__((noinline)) inline void resume(uint32_t tid)
+{
+    fiber &x = g->f[tid];
+    g->cur = tid;
+    if (_setjmp(g->main) != 0) return;
+    if (x.started) _longjmp(x.at, 1);
+    x.started = true;
+    setcontext(&x.ctx);
 }
 
 // Deposits v and waits for the wavefront's 64 lanes; afterwards operand(lane).
@@ -117,6 +131,7 @@ inline void run(uint32_t threads, int how, uint32_t seed, std::function<void()> 
         fiber &x = b.f[t];
         if (x.stack.empty()) x.stack.resize(65536u);
         x.st = kReady;
+        x.started = false;
         x.tid = t;
         x.ops = 0u;
         getcontext(&x.ctx);
@@ -138,10 +153,7 @@ inline void run(uint32_t threads, int how, uint32_t seed, std::function<void()> 
                 uint32_t here[4] = {0u, 0u, 0u, 0u};
                 for (uint32_t l = 64u; l-- > 0u;) {
                     fiber &x = b.f[64u * w + l];
-                    if (x.st == kReady) {
-                        b.cur = 64u * w + l;
-                        swapcontext(&b.main, &x.ctx);
-                    }
+                    if (x.st == kReady) resume(64u * w + l);
                     ++here[x.st];
                 }
                 if (here[kAtWave] == 0u) {

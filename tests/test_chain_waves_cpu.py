@@ -25,7 +25,7 @@ def test_positions_under_any_order_of_the_wavefronts():
     with open(os.path.join(BIN, "fnds_chain_kernels.inc"), "w") as f:
         f.write(kernels())
     out = os.path.join(BIN, "test_chain_waves")
-    subprocess.check_call(["g++", "-std=c++20", "-O1", "-w", os.path.join(HERE, "cpp", "test_chain_waves.cpp"),
+    subprocess.check_call(["g++", "-std=c++20", "-O1", "-U_FORTIFY_SOURCE", "-w", os.path.join(HERE, "cpp", "test_chain_waves.cpp"),
                            "-o", out + ".tmp"])
     os.replace(out + ".tmp", out)
     r = subprocess.run([out], capture_output=True, text=True, timeout=300)

@@ -1,5 +1,5 @@
-"""k_order, k_rank, k_far, k_fronts and k_slots (pagmo2_amd/csrc/fnds_chain.hip) give the
-ranks and fronts under any order of their wavefronts, also where most points have no dominator:
+"""k_order, k_rank, k_far, k_fronts, k_slots and k_masks (pagmo2_amd/csrc/fnds_chain.hip)
+give the ranks, fronts and dominators under any order of their wavefronts, also where most points have no dominator:
 the kernels' own text on the CPU (tests/cpp/test_rank_waves.cpp)."""
 import os
 import subprocess
@@ -12,7 +12,7 @@ def test_ranks_under_any_order_of_the_wavefronts():
     with open(os.path.join(BIN, "fnds_chain_kernels.inc"), "w") as f:
         f.write(kernels())
     out = os.path.join(BIN, "test_rank_waves")
-    subprocess.check_call(["g++", "-std=c++20", "-O1", "-w", os.path.join(HERE, "cpp", "test_rank_waves.cpp"),
+    subprocess.check_call(["g++", "-std=c++20", "-O1", "-U_FORTIFY_SOURCE", "-w", os.path.join(HERE, "cpp", "test_rank_waves.cpp"),
                            "-o", out + ".tmp"])
     os.replace(out + ".tmp", out)
     r = subprocess.run([out], capture_output=True, text=True, timeout=300)
