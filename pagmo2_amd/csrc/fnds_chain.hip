@@ -148,16 +148,17 @@ __global__ __launch_bounds__(kWide) void k_order(const uint32_t *__restrict__ cn
 }
 
 // The elements, their counts and their keys in that order (scattered here: one
-// workgroup stores 64 scattered words no faster than one a cycle).
+// workgroup stores 64 scattered words no faster than one a cycle), and `first` cleared.
 __global__ __launch_bounds__(kBlock) void k_scatter(const int64_t *__restrict__ keys,
                                                     const uint32_t *__restrict__ cnt,
                                                     const uint32_t *__restrict__ place, uint32_t n, uint32_t m,
                                                     uint32_t *__restrict__ perm, uint32_t *__restrict__ scnt,
-                                                    int64_t *__restrict__ skeys)
+                                                    int64_t *__restrict__ skeys, uint32_t *__restrict__ first)
 {
     const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= n) return;
     const uint32_t e = place[i];
+    first[i] = 0u;
     perm[e] = i;
     scnt[e] = cnt[i];
     for (uint32_t q = 0; q < m; ++q) {
@@ -747,14 +748,16 @@ __global__ __launch_bounds__(kBlock) void k_slots(const uint32_t *__restrict__ a
 
 // k_masks for a front of more than kWide members: a wavefront takes 64 of them, one per
 // lane, and kTileWords words of the front before, whose members it loads 64 at a time
-// and broadcasts.
+// and broadcasts.  Of the second front the words are not kept: the first front's
+// positions are its members' places, so the position of a member's last dominator
+// there, all that k_chain wants of them, is its highest bit (`first`, by place).
 constexpr uint32_t kTileWords = 2;
 template <int MT>
 __device__ __forceinline__ void masks_of_large(const int64_t *__restrict__ keys, const uint32_t *__restrict__ cnt,
                                                const uint32_t *__restrict__ members,
                                                const uint32_t *__restrict__ rank, const uint32_t *__restrict__ fo,
                                                const uint64_t *__restrict__ wbase, uint32_t n, uint32_t b, uint32_t w0,
-                                               uint64_t *__restrict__ masks)
+                                               uint64_t *__restrict__ masks, uint32_t *__restrict__ first)
 {
     const uint32_t lane = threadIdx.x & 63u, x = 64u * b + lane;
     if (64u * b >= n) return;
@@ -772,6 +775,7 @@ __device__ __forceinline__ void masks_of_large(const int64_t *__restrict__ keys,
         const bool on = ((todo >> lane) & 1u) && f == ff;
         todo &= ~__ballot(on);
         const uint32_t words = min((fa - fp + 63u) / 64u, w0 + kTileWords);
+        uint32_t last = 0u;
         for (uint32_t w = w0; w < words; ++w) {
             const uint32_t q = fp + 64u * w, there = min(64u, fa - q);
             point<MT> other;
@@ -789,8 +793,13 @@ __device__ __forceinline__ void masks_of_large(const int64_t *__restrict__ keys,
                 }
             }
             const uint64_t bits = __brev(half[0]) | (static_cast<uint64_t>(__brev(half[1])) << 32);
-            if (on) masks[base + static_cast<uint64_t>(w) * size + (x - a)] = bits;
+            if (ff == 1u) {
+                last = bits ? 64u * w + 63u - static_cast<uint32_t>(__clzll(static_cast<long long>(bits))) : last;
+            } else if (on) {
+                masks[base + static_cast<uint64_t>(w) * size + (x - a)] = bits;
+            }
         }
+        if (on && last) atomicMax(&first[x], last);
     }
 }
 
@@ -805,14 +814,15 @@ __global__ __launch_bounds__(kBlock) void k_masks(const int64_t *__restrict__ ke
                                                   const uint32_t *__restrict__ members,
                                                   const uint32_t *__restrict__ rank, const uint32_t *__restrict__ fo,
                                                   const uint64_t *__restrict__ wbase, uint32_t n, uint32_t large_x,
-                                                  uint32_t large_y, uint64_t *__restrict__ masks)
+                                                  uint32_t large_y, uint64_t *__restrict__ masks,
+                                                  uint32_t *__restrict__ first)
 {
     const uint32_t lane = threadIdx.x & 63u;
     if (blockIdx.x < large_x * large_y) {
         if (wbase[n] == 0u) return; // no such front
         const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
         masks_of_large<MT>(keys, cnt, members, rank, fo, wbase, n, blockIdx.x % large_x * (kBlock / 64u) + wave,
-                           blockIdx.x / large_x * kTileWords, masks);
+                           blockIdx.x / large_x * kTileWords, masks, first);
         return;
     }
     const uint32_t x = (blockIdx.x - large_x * large_y) * (kBlock / 64u) + (threadIdx.x >> 6);
@@ -926,7 +936,7 @@ constexpr int kFewBits = 5;
 __global__ __launch_bounds__(kWide) void k_chain(const uint32_t *__restrict__ fo, const uint64_t *__restrict__ masks,
                                                  uint64_t mask_words, uint32_t upto,
                                                  const uint64_t *__restrict__ scalars, uint32_t n, uint32_t P,
-                                                 uint32_t *__restrict__ pos_out)
+                                                 const uint32_t *__restrict__ first, uint32_t *__restrict__ pos_out)
 {
     extern __shared__ __align__(16) uint64_t lds64[];
     const uint32_t W = (n + 63u) / 64u;
@@ -1184,9 +1194,11 @@ __global__ __launch_bounds__(kWide) void k_chain(const uint32_t *__restrict__ fo
         }
         if (t == 0) s_run = 0u;
         __syncthreads();
+        // (the second front's last dominators are known: see k_masks)
+        const bool known = L == 1u && n > 2u * kWide;
         for (uint32_t x = t; x < 64u * cw; x += kWide) {
-            uint32_t v = 0u;
-            for (uint32_t left = sw; left > 0u; left -= min(left, kAhead)) { // from the last: see above
+            uint32_t v = known && x < c ? first[at + x] : 0u;
+            for (uint32_t left = known ? 0u : sw; left > 0u; left -= min(left, kAhead)) { // from the last: see above
                 uint64_t word[kAhead];
 #pragma unroll
                 for (uint32_t k = 0; k < kAhead; ++k) {
@@ -1367,7 +1379,7 @@ void chain_parts(pgh_fnds_ws *ws, uint32_t n, uint32_t m, std::vector<ws_part> &
         {&ws->any, n * 4u},           {&ws->tiles, nb * (nb + 1u) / 2u * 64u * 8u},
         {&ws->rank32, n * 4u},        {&ws->fo32, (n + 1u) * 4u},
         {&ws->wbase, (n + 1u) * 8u},  {&ws->members, n * 4u},
-        {&ws->masks, mask_words_of(n) * 8u}, {&ws->pos32, n * 4u},
+        {&ws->masks, mask_words_of(n) * 8u}, {&ws->pos32, n * 4u}, {&ws->first, n * 4u},
     };
     parts.insert(parts.end(), std::begin(own), std::end(own));
 }
@@ -1405,7 +1417,8 @@ pgh_status launch_chain_fronts(pgh_fnds_ws *ws, hipStream_t s, uint32_t n, uint3
     auto *top = reinterpret_cast<uint32_t *>(planes + static_cast<uint64_t>(nb) * kPlanes);
     k_order<<<1, kWide, order_lds, s>>>(cnt, n, any); // (any: a place to keep the places)
     PGH_HIP(hipGetLastError());
-    k_scatter<<<(n + kBlock - 1u) / kBlock, kBlock, 0, s>>>(keys, cnt, any, n, m, perm, scnt, skeys);
+    k_scatter<<<(n + kBlock - 1u) / kBlock, kBlock, 0, s>>>(keys, cnt, any, n, m, perm, scnt, skeys,
+                                                            static_cast<uint32_t *>(ws->first.ptr));
     PGH_HIP(hipGetLastError());
     const uint32_t rows = wave_rows(nb);
     const dim3 tg(nb, (nb + rows * (kBlock / 64u) - 1u) / (rows * (kBlock / 64u)));
@@ -1428,7 +1441,7 @@ pgh_status launch_chain_fronts(pgh_fnds_ws *ws, hipStream_t s, uint32_t n, uint3
     const uint32_t large_x = (nb + kBlock / 64u - 1u) / (kBlock / 64u);
     const uint32_t large_y = n > 2u * kWide ? (nb + kTileWords - 1u) / kTileWords : 0u;
     by_m(k_masks<1>, k_masks<2>, k_masks<3>)<<<large_x * large_y + waves, kBlock, 0, s>>>(
-        keys, cnt, members, rank, fo, wbase, n, large_x, large_y, masks);
+        keys, cnt, members, rank, fo, wbase, n, large_x, large_y, masks, static_cast<uint32_t *>(ws->first.ptr));
     PGH_HIP(hipGetLastError());
     return launch_chain_items(ws, s, n, upto);
 }
@@ -1448,7 +1461,7 @@ pgh_status launch_chain_items(pgh_fnds_ws *ws, hipStream_t s, uint32_t n, uint32
     auto *pos = static_cast<uint32_t *>(ws->pos32.ptr);
     k_chain<<<1, kWide, chain_lds_bytes(n), s>>>(fo, static_cast<const uint64_t *>(ws->masks.ptr), mask_words_of(n),
                                                  upto, static_cast<const uint64_t *>(ws->scalars.ptr), n, pow2_of(n),
-                                                 pos);
+                                                 static_cast<const uint32_t *>(ws->first.ptr), pos);
     PGH_HIP(hipGetLastError());
     k_items<<<(n + kBlock - 1u) / kBlock, kBlock, 0, s>>>(static_cast<const uint32_t *>(ws->members.ptr), rank, fo, pos,
                                                           n, upto, static_cast<uint64_t *>(ws->front_items.ptr),

@@ -72,8 +72,9 @@ struct pgh_fnds_ws {
     // fnds_chain.hip: the order by dominator count with the keys, counts and
     // ranks in it, the dominance bits, what far blocks give a rank, the ranks'
     // bit planes; ranks by index, front offsets, offsets of the fronts' words
-    // of `masks`, the members in any order and by index, and their positions
-    pgh::ws_view perm, skeys, scnt, srank, tiles, base, planes, rank32, fo32, wbase, any, members, masks, pos32;
+    // of `masks`, the members in any order and by index, their positions, and the last
+    // dominators of a large second front
+    pgh::ws_view perm, skeys, scnt, srank, tiles, base, planes, rank32, fo32, wbase, any, members, masks, pos32, first;
     uint64_t h_sizes[3] = {0, 0, 0}; // n_fronts, n_dom_items, peel barrier timeout
     bool sized = false;
     bool emitted = false; // dom_items holds the result's lists

@@ -77,7 +77,7 @@ static int check(const problem &pr, int how, uint32_t seed)
     // the kernel's inputs: offsets, members by index, and their dominators' bits
     std::vector<uint32_t> fo(n + 1u, 0u), want(n);
     std::vector<uint64_t> masks;
-    std::vector<uint32_t> before;
+    std::vector<uint32_t> before, first(n, 0u); // first: the second front's last dominators' places
     for (size_t f = 0; f < fronts.size(); ++f) {
         std::vector<uint32_t> by = fronts[f];
         std::sort(by.begin(), by.end());
@@ -95,7 +95,9 @@ static int check(const problem &pr, int how, uint32_t seed)
                     for (uint32_t q = 64u * w; q < std::min<size_t>(64u * w + 64u, before.size()); ++q) {
                         if (dom(before[q], by[c])) bits |= uint64_t(1) << (q - 64u * w);
                     }
-                    masks.push_back(bits);
+                    if (f == 1u && bits) first[at + c] = 64u * w + 63u - static_cast<uint32_t>(__builtin_clzll(bits));
+                    // (a large second front's words are not there on the device)
+                    masks.push_back(f == 1u && size > kWide && n > 2u * kWide ? 0xababababababababull : bits);
                 }
             }
         }
@@ -109,7 +111,7 @@ static int check(const problem &pr, int how, uint32_t seed)
     std::vector<uint32_t> got(n, 0xffffffffu);
     std::memset(wave_emu::dynamic_lds, 0xcd, sizeof wave_emu::dynamic_lds);
     wave_emu::run(kWide, how, seed, [&] {
-        k_chain(fo.data(), masks.data(), mask_words, n, scalars, n, P, got.data());
+        k_chain(fo.data(), masks.data(), mask_words, n, scalars, n, P, first.data(), got.data());
     });
     for (uint32_t i = 0; i < n; ++i) {
         if (got[i] != want[i]) {
@@ -136,6 +138,9 @@ int main()
         ps.push_back(layers("a middle front between", s, 2.0, 4u));
     }
     ps.push_back(layers("one large front after a small one", {90u, 1200u, 100u, 100u}, 2.0, 5u));
+    // a large second front, and one behind it
+    ps.push_back(layers("two large fronts", {300u, 1500u, 1100u, 60u}, 2.0, 6u));
+    ps.push_back(layers("two large fronts of few dominators", {1500u, 1400u, 1200u}, 0.002, 7u));
     int bad = 0;
     for (const problem &p : ps) {
         bad += check(p, wave_emu::kFirstAhead, 0u);

@@ -129,12 +129,13 @@ static int check(uint32_t n, int which, int how)
         words += static_cast<uint64_t>(fo[f + 1u] - fo[f]) * ((fo[f] - fo[f - 1u] + 63u) / 64u);
     }
     std::vector<uint64_t> masks(words + 1u, 0xcdcdcdcdcdcdcdcd);
+    std::vector<uint32_t> first(n, 0u);
     const uint32_t large_x = (nb + per - 1u) / per, large_y = n > 2u * kWide ? (nb + kTileWords - 1u) / kTileWords : 0u;
     for (uint32_t b = 0; ok && b < large_x * large_y + groups; ++b) {
         wave_emu::block_idx.x = b;
         wave_emu::run(kBlock, how, 6u, [&] {
             k_masks<2>(keys.data(), cnt.data(), members.data(), rank.data(), fo.data(), wbase.data(), n, large_x, large_y,
-                       masks.data());
+                       masks.data(), first.data());
         });
     }
     wave_emu::block_idx.x = 0u;
@@ -144,6 +145,12 @@ static int check(uint32_t n, int which, int how)
     for (uint32_t f = 1; ok && f < fronts; ++f) {
         const uint32_t a = fo[f], size = fo[f + 1u] - a, pa = fo[f - 1u], sw = (a - pa + 63u) / 64u;
         for (uint32_t c = 0; ok && c < size; ++c) {
+            if (f == 1u && size > kWide && large_y) { // the last dominator's place instead
+                uint32_t last = 0u;
+                for (uint32_t q = 0; q < a - pa; ++q) last = shifted_dom(members[pa + q], members[a + c]) ? q : last;
+                ok = first[a + c] == last;
+                continue;
+            }
             for (uint32_t w = 0; ok && w < sw; ++w) {
                 uint64_t bits = 0u;
                 for (uint32_t q = 64u * w; q < std::min(64u * w + 64u, a - pa); ++q) {

@@ -245,6 +245,10 @@ inline int __clz(int v)
 {
     return v ? __builtin_clz(static_cast<unsigned>(v)) : 32;
 }
+inline int __clzll(long long v)
+{
+    return v ? __builtin_clzll(static_cast<unsigned long long>(v)) : 64;
+}
 inline uint32_t __brev(uint32_t v)
 {
     uint32_t r = 0u;
