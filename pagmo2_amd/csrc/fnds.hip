@@ -745,7 +745,7 @@ pgh_status fnds_run(pgh_fnds_ws *ws, const double *objs, uint64_t n, uint64_t m,
     if (n >= (uint64_t(1) << 31)) return fail(PGH_OVERFLOW, "too many points for fast_non_dominated_sorting");
     if (m && !objs) return fail(PGH_INVALID_ARGUMENT, "null objective matrix");
     if (m > 512u) return fail(PGH_UNSUPPORTED, "at most 512 objectives are supported");
-    const bool chain = ws->peel.ranks(n, m);
+    const bool chain = ws->by_ranks = ws->peel.ranks(n, m);
     ws->stream = s;
     ws->n = 0u; // (no result while the buffers may be replaced)
     ws->m = m;

@@ -113,36 +113,38 @@ __device__ __forceinline__ void in_batches(uint32_t n, Load load, Use use)
 }
 
 // bins[k] += 1 for every lane that is `in`, and what was there.  One addition for the
-// wavefront where all lanes have the same bin: 64 to one address take 64 turns (one
-// front of 16384, whose counts are all zero: k_order 41 us).
+// wavefront where all lanes have bin 0 (or, ANY, any one bin): 64 to one address take
+// 64 turns (one front of 16384, whose counts are all zero: k_order 41 us).
+template <bool ANY>
 __device__ __forceinline__ uint32_t bin_add(uint32_t *bins, uint32_t k, bool in)
 {
+    uint32_t same = 0u;
+    if constexpr (ANY) same = __builtin_amdgcn_readfirstlane(k); // (lanes past the end repeat the last element)
+    if (__ballot(k != same) != 0u) return in ? atomicAdd(&bins[k], 1u) : 0u;
     const uint64_t who = __ballot(in);
-    if (who == 0u) return 0u; // uniform
-    const uint32_t lead = static_cast<uint32_t>(__builtin_ctzll(who)), same = __builtin_amdgcn_readlane(k, lead);
-    if (__ballot(in && k != same) != 0u) return in ? atomicAdd(&bins[k], 1u) : 0u;
     const uint32_t lane = threadIdx.x & 63u;
     uint32_t old = 0u;
-    if (lane == lead) old = atomicAdd(&bins[same], static_cast<uint32_t>(__popcll(who)));
-    return __builtin_amdgcn_readlane(old, lead) + static_cast<uint32_t>(__popcll(who & ((uint64_t(1) << lane) - 1u)));
+    if (lane == 0u && who) old = atomicAdd(&bins[same], static_cast<uint32_t>(__popcll(who)));
+    return __builtin_amdgcn_readfirstlane(old) + static_cast<uint32_t>(__popcll(who & ((uint64_t(1) << lane) - 1u)));
 }
 
 // Every element's place in the order by dominator count (equal counts in any
-// order; no result depends on it).
+// order; no result depends on it), and the number of those without dominators.
 __global__ __launch_bounds__(kWide) void k_order(const uint32_t *__restrict__ cnt, uint32_t n,
-                                                 uint32_t *__restrict__ place)
+                                                 uint32_t *__restrict__ place, uint64_t *__restrict__ n_free)
 {
     extern __shared__ uint32_t bins[]; // n
     __shared__ uint32_t sh[kWide / 64u];
     for (uint32_t i = threadIdx.x; i < n; i += kWide) bins[i] = 0u;
     __syncthreads();
     in_batches(n, [&](uint32_t i) { return cnt[i]; },
-               [&](uint32_t, uint32_t c, bool in) { bin_add(bins, min(c, n - 1u), in); });
+               [&](uint32_t, uint32_t c, bool in) { bin_add<false>(bins, min(c, n - 1u), in); });
     __syncthreads();
+    if (threadIdx.x == 0) *n_free = bins[0]; // (its next store is this thread's)
     scan_bins(bins, n, sh);
     in_batches(n, [&](uint32_t i) { return cnt[i]; },
                [&](uint32_t i, uint32_t c, bool in) {
-                   const uint32_t at = bin_add(bins, min(c, n - 1u), in);
+                   const uint32_t at = bin_add<false>(bins, min(c, n - 1u), in);
                    if (in) place[i] = min(at, n - 1u);
                });
 }
@@ -342,12 +344,12 @@ __device__ __forceinline__ uint64_t tile_at(uint32_t J, uint32_t I)
     return (static_cast<uint64_t>(J) * (J + 1u) / 2u + I) * 64u;
 }
 
-// Block J has no element with a dominator (the counts ascend).  Such blocks, a front's
-// worth of them, are not worth a tile nor a step of k_rank: one front of 16384 points
-// took k_rank 235 us, and k_tiles 51.
-__device__ __forceinline__ bool block_is_free(const uint32_t *__restrict__ scnt, uint32_t n, uint32_t J)
+// Block J has no element with a dominator (the first n_free have none).  Such blocks, a
+// front's worth of them, are not worth a tile nor a step of k_rank: one front of 16384
+// points took k_rank 235 us, and k_tiles 51.
+__device__ __forceinline__ bool block_is_free(uint64_t n_free, uint32_t n, uint32_t J)
 {
-    return scnt[min(64u * J + 63u, n - 1u)] == 0u;
+    return min(64u * J + 63u, n - 1u) < n_free;
 }
 
 // Word c of tile (J, I), I <= J: the dominators of element 64 J + c (in perm's
@@ -357,13 +359,14 @@ __device__ __forceinline__ bool block_is_free(const uint32_t *__restrict__ scnt,
 template <int MT, uint32_t ROWS>
 __global__ __launch_bounds__(kBlock) void k_tiles(const int64_t *__restrict__ skeys,
                                                   const uint32_t *__restrict__ scnt, uint32_t n,
+                                                  const uint64_t *__restrict__ n_free,
                                                   uint64_t *__restrict__ tiles)
 {
     const uint32_t J = blockIdx.x, lane = threadIdx.x & 63u;
     const uint32_t I0 = (blockIdx.y * (kBlock / 64u) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * ROWS;
     if (I0 > J) return; // wavefront-uniform, no barrier below
     const uint32_t c0 = 64u * J, cols = min(64u, n - c0);
-    if (block_is_free(scnt, n, J)) return; // no word of it is read
+    if (block_is_free(*n_free, n, J)) return; // no word of it is read
     uint64_t out[ROWS];
     point<MT> row[ROWS];
 #pragma unroll
@@ -492,7 +495,7 @@ constexpr uint32_t kSpan = 32; // blocks per launch at most
 __global__ __launch_bounds__(kWide) void k_rank(const uint64_t *__restrict__ tiles, uint32_t n, uint32_t J0,
                                                 uint32_t J1, const uint32_t *__restrict__ base,
                                                 uint32_t *__restrict__ rank, uint64_t *__restrict__ planes_out,
-                                                uint32_t *__restrict__ top_out, const uint32_t *__restrict__ scnt)
+                                                uint32_t *__restrict__ top_out, const uint64_t *__restrict__ n_free)
 {
     __shared__ __align__(16) uint64_t planes[kSpan * kPlanes];
     __shared__ uint32_t top[kSpan];
@@ -582,9 +585,9 @@ __global__ __launch_bounds__(kWide) void k_rank(const uint64_t *__restrict__ til
     // wavefront 0 holds blocks J and J + 1, the others J + 1 and J + 2
     fetch(wave == 0u ? J0 : J0 + 1u, 0u);
     fetch(wave == 0u ? J0 + 1u : J0 + 2u, 1u);
-    // (in flight beside those; lane l: block J0 + l)
-    const bool is_free = lane < J1 - J0 && block_is_free(scnt, n, min(J0 + lane, J1 - 1u));
-    const uint32_t Js = J0 + static_cast<uint32_t>(__popcll(__ballot(is_free)));
+    // the first block with a dominator, or J1 (looked at while those are in flight)
+    const uint64_t free_now = *n_free;
+    const uint32_t Js = free_now >= n ? J1 : min(max(static_cast<uint32_t>(free_now) / 64u, J0), J1);
     if (Js > J0) { // uniform
         for (uint32_t x = threadIdx.x; x < (Js - J0) * kPlanes; x += kWide) {
             planes[x] = 0u;
@@ -617,12 +620,12 @@ constexpr uint32_t kFarBlock = 512;
 __global__ __launch_bounds__(kFarBlock) void k_far(const uint64_t *__restrict__ tiles, uint32_t n, uint32_t I0,
                                                    uint32_t I1, const uint64_t *__restrict__ planes,
                                                    const uint32_t *__restrict__ top, uint32_t *__restrict__ base,
-                                                   uint32_t first, const uint32_t *__restrict__ scnt)
+                                                   uint32_t first, const uint64_t *__restrict__ n_free)
 {
     __shared__ uint32_t rr[64];
     const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t J = I1 + blockIdx.x, e = 64u * J + lane;
-    if (block_is_free(scnt, n, J)) return; // uniform; its base is not read
+    if (block_is_free(*n_free, n, J)) return; // uniform; its base is not read
     if (threadIdx.x < 64u) rr[lane] = 0u;
     __syncthreads();
     uint32_t r = 0u;
@@ -640,7 +643,7 @@ __global__ __launch_bounds__(kFarBlock) void k_far(const uint64_t *__restrict__ 
 }
 
 // Front offsets (32 and 64 bits), the offset of each front's words of k_masks (and at n
-// whether a front but the first has more than kWide members), the number of fronts, the elements' ranks by index and the members of every
+// the most members of a front but the first), the number of fronts, the elements' ranks by index and the members of every
 // front in any order.
 __global__ __launch_bounds__(kWide) void k_fronts(const uint32_t *__restrict__ srank,
                                                   const uint32_t *__restrict__ perm, uint32_t n,
@@ -658,7 +661,7 @@ __global__ __launch_bounds__(kWide) void k_fronts(const uint32_t *__restrict__ s
     in_batches(n, [&](uint32_t e) { return min(srank[e], n - 1u); },
                [&](uint32_t, uint32_t r, bool in) {
                    big = in ? max(big, r + 1u) : big;
-                   bin_add(bins, r, in);
+                   bin_add<true>(bins, r, in);
                });
     atomicMax(&s_fronts, big);
     __syncthreads();
@@ -677,19 +680,21 @@ __global__ __launch_bounds__(kWide) void k_fronts(const uint32_t *__restrict__ s
         };
         uint32_t sum = 0u, total; // at most n + n^2 / 256
         for (uint32_t f = b; f < e; ++f) sum += words(f);
-        uint32_t o = wide_exclusive_scan(sum, sh, total);
+        uint32_t o = wide_exclusive_scan(sum, sh, total), most = 0u;
         for (uint32_t f = b; f < e; ++f) {
             wbase[f] = o;
             o += words(f);
-            if (f && bins[f + 1u] - bins[f] > kWide) s_large = 1u;
+            if (f) most = max(most, bins[f + 1u] - bins[f]);
         }
+        most = wave_max(most);
+        if ((t & 63u) == 0u && most) atomicMax(&s_large, most);
     }
     if (t == 0) scalars[0] = F;
     __syncthreads();
     if (t == 0) wbase[n] = s_large; // (a place of no front's)
     in_batches(n, [&](uint32_t e) { return make_uint2(min(srank[e], n - 1u), perm[e]); },
                [&](uint32_t, uint2 v, bool in) {
-                   const uint32_t at = bin_add(bins, v.x, in);
+                   const uint32_t at = bin_add<true>(bins, v.x, in);
                    if (in) {
                        rank[v.y] = v.x;
                        any[min(at, n - 1u)] = v.y;
@@ -819,10 +824,12 @@ __global__ __launch_bounds__(kBlock) void k_masks(const int64_t *__restrict__ ke
 {
     const uint32_t lane = threadIdx.x & 63u;
     if (blockIdx.x < large_x * large_y) {
-        if (wbase[n] == 0u) return; // no such front
+        if (wbase[n] <= kWide) return; // no such front
         const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-        masks_of_large<MT>(keys, cnt, members, rank, fo, wbase, n, blockIdx.x % large_x * (kBlock / 64u) + wave,
-                           blockIdx.x / large_x * kTileWords, masks, first);
+        for (uint32_t w0 = blockIdx.x / large_x * kTileWords; 64u * w0 < n; w0 += large_y * kTileWords) {
+            masks_of_large<MT>(keys, cnt, members, rank, fo, wbase, n, blockIdx.x % large_x * (kBlock / 64u) + wave, w0,
+                               masks, first);
+        }
         return;
     }
     const uint32_t x = (blockIdx.x - large_x * large_y) * (kBlock / 64u) + (threadIdx.x >> 6);
@@ -1415,7 +1422,8 @@ pgh_status launch_chain_fronts(pgh_fnds_ws *ws, hipStream_t s, uint32_t n, uint3
     auto *base = static_cast<uint32_t *>(ws->base.ptr), *any = static_cast<uint32_t *>(ws->any.ptr);
     auto *planes = static_cast<uint64_t *>(ws->planes.ptr);
     auto *top = reinterpret_cast<uint32_t *>(planes + static_cast<uint64_t>(nb) * kPlanes);
-    k_order<<<1, kWide, order_lds, s>>>(cnt, n, any); // (any: a place to keep the places)
+    // (any, wbase: places to keep the places and the number of points without dominators)
+    k_order<<<1, kWide, order_lds, s>>>(cnt, n, any, wbase);
     PGH_HIP(hipGetLastError());
     k_scatter<<<(n + kBlock - 1u) / kBlock, kBlock, 0, s>>>(keys, cnt, any, n, m, perm, scnt, skeys,
                                                             static_cast<uint32_t *>(ws->first.ptr));
@@ -1423,13 +1431,13 @@ pgh_status launch_chain_fronts(pgh_fnds_ws *ws, hipStream_t s, uint32_t n, uint3
     const uint32_t rows = wave_rows(nb);
     const dim3 tg(nb, (nb + rows * (kBlock / 64u) - 1u) / (rows * (kBlock / 64u)));
     const auto by_m = [m](auto f1, auto f2, auto f3) { return m == 1u ? f1 : (m == 2u ? f2 : f3); };
-    if (rows == 1u) by_m(k_tiles<1, 1>, k_tiles<2, 1>, k_tiles<3, 1>)<<<tg, kBlock, 0, s>>>(skeys, scnt, n, tiles);
-    else by_m(k_tiles<1, 4>, k_tiles<2, 4>, k_tiles<3, 4>)<<<tg, kBlock, 0, s>>>(skeys, scnt, n, tiles);
+    if (rows == 1u) by_m(k_tiles<1, 1>, k_tiles<2, 1>, k_tiles<3, 1>)<<<tg, kBlock, 0, s>>>(skeys, scnt, n, wbase, tiles);
+    else by_m(k_tiles<1, 4>, k_tiles<2, 4>, k_tiles<3, 4>)<<<tg, kBlock, 0, s>>>(skeys, scnt, n, wbase, tiles);
     PGH_HIP(hipGetLastError());
     for (uint32_t J0 = 0; J0 < nb; J0 += kSpan) {
         const uint32_t J1 = std::min(J0 + kSpan, nb);
-        k_rank<<<1, kWide, 0, s>>>(tiles, n, J0, J1, J0 ? base : nullptr, srank, planes, top, scnt);
-        if (J1 < nb) k_far<<<nb - J1, kFarBlock, 0, s>>>(tiles, n, J0, J1, planes, top, base, J0 == 0u ? 1u : 0u, scnt);
+        k_rank<<<1, kWide, 0, s>>>(tiles, n, J0, J1, J0 ? base : nullptr, srank, planes, top, wbase);
+        if (J1 < nb) k_far<<<nb - J1, kFarBlock, 0, s>>>(tiles, n, J0, J1, planes, top, base, J0 == 0u ? 1u : 0u, wbase);
         PGH_HIP(hipGetLastError());
     }
     k_fronts<<<1, kWide, fronts_lds, s>>>(srank, perm, n, fo, static_cast<uint64_t *>(ws->front_offsets.ptr), wbase,
@@ -1439,7 +1447,7 @@ pgh_status launch_chain_fronts(pgh_fnds_ws *ws, hipStream_t s, uint32_t n, uint3
     k_slots<<<waves + big_groups, kBlock, 0, s>>>(any, rank, fo, n, big_groups, members);
     PGH_HIP(hipGetLastError());
     const uint32_t large_x = (nb + kBlock / 64u - 1u) / (kBlock / 64u);
-    const uint32_t large_y = n > 2u * kWide ? (nb + kTileWords - 1u) / kTileWords : 0u;
+    const uint32_t large_y = n > 2u * kWide ? std::min((nb + kTileWords - 1u) / kTileWords, 32u) : 0u;
     by_m(k_masks<1>, k_masks<2>, k_masks<3>)<<<large_x * large_y + waves, kBlock, 0, s>>>(
         keys, cnt, members, rank, fo, wbase, n, large_x, large_y, masks, static_cast<uint32_t *>(ws->first.ptr));
     PGH_HIP(hipGetLastError());

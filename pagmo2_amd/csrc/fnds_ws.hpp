@@ -80,6 +80,7 @@ struct pgh_fnds_ws {
     bool emitted = false; // dom_items holds the result's lists
     bool lists = false; // D, dom_offsets and dom_count hold this result's
     bool items = false; // front_items holds every front's
+    bool by_ranks = false; // the result's fronts come from ranks (fnds_chain.hip)
     // workgroups of the grid-wide front peel, set or found by pgh_fnds_tune (any
     // count gives the same result, and so do ranks)
     pgh::peel_choice peel;

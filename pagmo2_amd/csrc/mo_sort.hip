@@ -219,6 +219,7 @@ __global__ __launch_bounds__(kFrontBlock) void k_front_order(const double *__res
                                                              const uint64_t *__restrict__ items,
                                                              const uint64_t *__restrict__ offsets, uint32_t cap,
                                                              uint64_t N, uint64_t *__restrict__ scalars,
+                                                             const uint64_t *__restrict__ largest,
                                                              void *__restrict__ out)
 {
     // K, V, two orders, distances: cap members each (a power of two)
@@ -245,13 +246,18 @@ __global__ __launch_bounds__(kFrontBlock) void k_front_order(const double *__res
             // every workgroup's share here would be for nothing
             if (n > cap) {
                 __shared__ uint32_t s_large;
-                if (threadIdx.x == 0) s_large = 0u;
-                __syncthreads();
-                bool large = false;
-                for (uint32_t q = threadIdx.x; q < fronts; q += kFrontBlock) large |= offsets[q + 1u] - offsets[q] > cap;
-                if (large) s_large = 1u;
-                __syncthreads();
-                if (s_large) { // uniform
+                bool large = offsets[1] > cap;
+                if (largest) {
+                    large |= *largest > cap;
+                } else { // (the peel does not say)
+                    if (threadIdx.x == 0) s_large = 0u;
+                    __syncthreads();
+                    for (uint32_t q = threadIdx.x; q < fronts; q += kFrontBlock) large |= offsets[q + 1u] - offsets[q] > cap;
+                    if (large) s_large = 1u;
+                    __syncthreads();
+                    large = s_large != 0u;
+                }
+                if (large) { // uniform
                     if (f == 0u && threadIdx.x == 0) scalars[3] = 1u;
                     return;
                 }
@@ -325,7 +331,8 @@ pgh_status launch_front_order(pgh_fnds_ws *ws, const double *objs, uint64_t n, u
     const uint32_t cap = front_cap(n); // (kFrontDistances: n <= kCrowdMax)
     k_front_order<OUT><<<grid, kFrontBlock, front_lds(cap), s>>>(
         objs, static_cast<uint32_t>(n), static_cast<uint32_t>(m), static_cast<const uint64_t *>(ws->front_items.ptr),
-        static_cast<const uint64_t *>(ws->front_offsets.ptr), cap, N, static_cast<uint64_t *>(ws->scalars.ptr), out);
+        static_cast<const uint64_t *>(ws->front_offsets.ptr), cap, N, static_cast<uint64_t *>(ws->scalars.ptr),
+        ws->by_ranks ? static_cast<const uint64_t *>(ws->wbase.ptr) + n : nullptr, out);
     PGH_HIP(hipGetLastError());
     return PGH_OK;
 }

@@ -43,19 +43,20 @@ static int check(uint32_t n, int which, int how)
     const auto dom = [&](uint32_t a, uint32_t b) {
         return x[a] <= x[b] && y[a] <= y[b] && (x[a] < x[b] || y[a] < y[b]);
     };
-    std::vector<uint32_t> cnt(n, 0u), place(n), perm(n), scnt(n);
+    std::vector<uint32_t> cnt(n, 0u), place(n), perm(n);
     for (uint32_t i = 0; i < n; ++i) {
         for (uint32_t j = 0; j < n; ++j) cnt[j] += dom(i, j) ? 1u : 0u;
     }
-    wave_emu::run(kWide, how, 1u, [&] { k_order(cnt.data(), n, place.data()); });
+    uint64_t n_free = ~uint64_t(0);
+    wave_emu::run(kWide, how, 1u, [&] { k_order(cnt.data(), n, place.data(), &n_free); });
+    bool ok = n_free == static_cast<uint64_t>(std::count(cnt.begin(), cnt.end(), 0u));
     for (uint32_t i = 0; i < n; ++i) {
         perm[place[i]] = i;
-        scnt[place[i]] = cnt[i];
     }
     const uint32_t nb = (n + 63u) / 64u;
     std::vector<uint64_t> tiles(static_cast<size_t>(nb) * (nb + 1u) / 2u * 64u, 0xabababababababab);
     for (uint32_t J = 0; J < nb; ++J) {
-        if (block_is_free(scnt.data(), n, J)) continue;
+        if (block_is_free(n_free, n, J)) continue;
         for (uint32_t I = 0; I <= J; ++I) {
             for (uint32_t c = 0; c < 64u; ++c) {
                 uint64_t w = 0u;
@@ -79,12 +80,12 @@ static int check(uint32_t n, int which, int how)
         const uint32_t J1 = std::min(J0 + kSpan, nb);
         wave_emu::run(kWide, how, 2u, [&] {
             k_rank(tiles.data(), n, J0, J1, J0 ? base.data() : nullptr, ranks.data(), planes.data(), top.data(),
-                   scnt.data());
+                   &n_free);
         });
         for (uint32_t b = 0; b < nb - J1; ++b) {
             wave_emu::block_idx.x = b;
             wave_emu::run(kFarBlock, how, 3u, [&] {
-                k_far(tiles.data(), n, J0, J1, planes.data(), top.data(), base.data(), J0 == 0u ? 1u : 0u, scnt.data());
+                k_far(tiles.data(), n, J0, J1, planes.data(), top.data(), base.data(), J0 == 0u ? 1u : 0u, &n_free);
             });
         }
         wave_emu::block_idx.x = 0u;
@@ -95,7 +96,7 @@ static int check(uint32_t n, int which, int how)
     wave_emu::run(kWide, how, 4u, [&] {
         k_fronts(ranks.data(), perm.data(), n, fo.data(), fo64.data(), wbase.data(), rank.data(), any.data(), scalars);
     });
-    bool ok = scalars[0] == fronts;
+    ok = ok && scalars[0] == fronts;
     std::vector<uint32_t> seen(n, 0u);
     for (uint32_t e = 0; e < n; ++e) {
         ok = ok && ranks[e] == want[e] && rank[perm[e]] == want[e] && any[e] < n && rank[any[e]] < fronts &&
@@ -130,7 +131,7 @@ static int check(uint32_t n, int which, int how)
     }
     std::vector<uint64_t> masks(words + 1u, 0xcdcdcdcdcdcdcdcd);
     std::vector<uint32_t> first(n, 0u);
-    const uint32_t large_x = (nb + per - 1u) / per, large_y = n > 2u * kWide ? (nb + kTileWords - 1u) / kTileWords : 0u;
+    const uint32_t large_x = (nb + per - 1u) / per, large_y = n > 2u * kWide ? std::min((nb + kTileWords - 1u) / kTileWords, 7u) : 0u;
     for (uint32_t b = 0; ok && b < large_x * large_y + groups; ++b) {
         wave_emu::block_idx.x = b;
         wave_emu::run(kBlock, how, 6u, [&] {
