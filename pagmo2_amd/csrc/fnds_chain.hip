@@ -1447,7 +1447,7 @@ pgh_status launch_chain_fronts(pgh_fnds_ws *ws, hipStream_t s, uint32_t n, uint3
     k_slots<<<waves + big_groups, kBlock, 0, s>>>(any, rank, fo, n, big_groups, members);
     PGH_HIP(hipGetLastError());
     const uint32_t large_x = (nb + kBlock / 64u - 1u) / (kBlock / 64u);
-    const uint32_t large_y = n > 2u * kWide ? std::min((nb + kTileWords - 1u) / kTileWords, 32u) : 0u;
+    const uint32_t large_y = n > 2u * kWide ? std::min((nb + kTileWords - 1u) / kTileWords, 64u) : 0u;
     by_m(k_masks<1>, k_masks<2>, k_masks<3>)<<<large_x * large_y + waves, kBlock, 0, s>>>(
         keys, cnt, members, rank, fo, wbase, n, large_x, large_y, masks, static_cast<uint32_t *>(ws->first.ptr));
     PGH_HIP(hipGetLastError());
