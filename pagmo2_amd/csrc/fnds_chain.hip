@@ -25,7 +25,7 @@
 // What stays serial is a few hundred instructions per 64 elements (k_rank) and
 // per front (k_chain), on bits: the largest of a set of small numbers is found
 // from their bit planes, a 64-bit AND per bit, with no loop over the set.
-// Measured (8192 x 2 with 213 fronts; 16384 x 3 with 54): the grid-wide peel took
+// Measured (8192 x 2 with 213 fronts; 16384 x 3 with 54): the peel's kernel took
 // 1.16 and 0.75 ms, here k_rank takes 0.18 and 0.26 ms, k_chain 0.12 and 0.27 and
 // the rest 0.08 and 0.15.  Both serial kernels are bound by the latency of one
 // wavefront's dependent instructions.

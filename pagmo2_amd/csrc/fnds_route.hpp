@@ -10,9 +10,11 @@ namespace pgh
 // fnds_chain.hip takes up to kChainMaxN points (its sort keys, positions and bit
 // planes fit one workgroup's LDS) of one to kChainMaxM objectives.  With more
 // objectives the fronts are few and large, and the grid-wide peel, whose cost is
-// an exchange per front, is faster: 16384 x 3 (54 fronts) 0.70 against 0.90 ms
-// for the peel, 16384 x 5 (15 fronts) 1.30 against 0.67 ms; with two objectives
-// (8192: 176-213 fronts) 0.40 against 1.2-1.4 ms.
+// an exchange per front, is faster: ranks and order inside the fronts of 16384 x 3
+// (54 fronts) took 0.70 ms against 0.90 for the peel with what leads up to it, of
+// 16384 x 5 (15 fronts) 1.30 against 0.67; with two objectives (8192: 176-213 fronts)
+// 0.40 against 1.2-1.4.  (Since then a large front costs the ranks a fraction of
+// that; a whole call of 16384 x 3 takes 1.03 against 1.3 ms.)
 constexpr uint32_t kChainMaxN = 16384, kChainMaxM = 3;
 
 // A workspace's choice of peel.
