@@ -20,10 +20,16 @@ def kernels():
     return re.sub(r"(?<!_)__shared__\b", "static", text)
 
 
+def write_kernels():
+    inc = os.path.join(BIN, "fnds_chain_kernels.inc")
+    with open(f"{inc}.{os.getpid()}", "w") as f:
+        f.write(kernels())
+    os.replace(f"{inc}.{os.getpid()}", inc)
+
+
 def test_positions_under_any_order_of_the_wavefronts():
     os.makedirs(BIN, exist_ok=True)
-    with open(os.path.join(BIN, "fnds_chain_kernels.inc"), "w") as f:
-        f.write(kernels())
+    write_kernels()
     out = os.path.join(BIN, "test_chain_waves")
     subprocess.check_call(["g++", "-std=c++20", "-O1", "-U_FORTIFY_SOURCE", "-w", os.path.join(HERE, "cpp", "test_chain_waves.cpp"),
                            "-o", out + ".tmp"])

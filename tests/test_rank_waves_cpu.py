@@ -4,13 +4,12 @@ the kernels' own text on the CPU (tests/cpp/test_rank_waves.cpp)."""
 import os
 import subprocess
 
-from test_chain_waves_cpu import BIN, HERE, kernels
+from test_chain_waves_cpu import BIN, HERE, write_kernels
 
 
 def test_ranks_under_any_order_of_the_wavefronts():
     os.makedirs(BIN, exist_ok=True)
-    with open(os.path.join(BIN, "fnds_chain_kernels.inc"), "w") as f:
-        f.write(kernels())
+    write_kernels()
     out = os.path.join(BIN, "test_rank_waves")
     subprocess.check_call(["g++", "-std=c++20", "-O1", "-U_FORTIFY_SOURCE", "-w", os.path.join(HERE, "cpp", "test_rank_waves.cpp"),
                            "-o", out + ".tmp"])
